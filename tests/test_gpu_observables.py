@@ -110,3 +110,55 @@ def test_frame_contact_map_two_copies():
     assert got.shape == (cms * (cms + 1) // 2,)
     assert np.array_equal(got, want)
     sim.close()
+
+
+@pytest.mark.parametrize("N", [8, 64, 65, 66, 127, 258, 1089, 4223])
+def test_distance_contact_tile_edges(N):
+    # separations and starting beads at the edges of the kernel's tiles (32 x
+    # 64): one separation, a tile and one more or less, many ragged tiles
+    step(f"d(s), P(s) N={N}")
+    R_n = radius_for(N, 0.2)
+    sim = sim_with(N, R_n, walk(N, R_n, seed=N), np.zeros(N, np.uint8))
+    sd, cp = sim.distance_contact(0)
+    wsd, wcp = po.sd_cp(sim.positions, 0)
+    assert np.array_equal(sd, wsd) and np.array_equal(cp, wcp)
+    sim.close()
+
+
+@pytest.mark.parametrize("N", [8, 60, 68, 1027, 1028, 4164])
+def test_frame_contact_map_tile_edges(N):
+    # map sides at the edges of the kernel's blocks (256 columns x 16 rows),
+    # with beads past the last whole pixel
+    step(f"frame contact map N={N}")
+    R_n = radius_for(N, 0.3)
+    sim = sim_with(N, R_n, walk(N, R_n, seed=N + 1), np.zeros(N, np.uint8))
+    assert np.array_equal(sim.frame_contact_map(), po.ccp_contact_map(sim.positions))
+    sim.close()
+
+
+def test_frame_contact_map_rounded_rows():
+    # rows long enough that ccp's FP32 root of the packed index leaves the
+    # row: every pixel of some rows against ccp's index arithmetic in numpy
+    N = 57400
+    step(f"frame contact map N={N}")
+    R_n = radius_for(N, 0.2)
+    sim = sim_with(N, R_n, walk(N, R_n, seed=5), np.zeros(N, np.uint8))
+    r = sim.positions
+    got = sim.frame_contact_map()
+    cms = N // 4
+    rows = np.array([cms - 1, cms - 2, cms - 700])
+    moved = 0
+    for row in rows:
+        ia = row * (row + 1) // 2 + np.arange(row + 1)
+        ix = np.minimum((np.sqrt((2.0 * ia + 0.25).astype(np.float32)).astype(np.float64) - 0.5).astype(np.int64),
+                        cms - 1)
+        iy = np.clip((ia - ix * (ix + 1.0) / 2.0).astype(np.int64), 0, cms - 1)
+        moved += int((ix != row).sum())
+        n = np.zeros(len(ia), np.int64)
+        for p in range(4):
+            for q in range(4):
+                d = r[4 * ix + p] - r[4 * iy + q]
+                n += ((d[:, 0] * d[:, 0] + d[:, 1] * d[:, 1]) + d[:, 2] * d[:, 2]) < np.float32(4.0)
+        assert np.array_equal(got[ia], (1000 * n / 16).astype(np.float32)), row
+    assert moved > 0
+    sim.close()

@@ -1402,7 +1402,8 @@ int ccp_distance_contact(ccp_sim *h, uint32_t chromosome, float *sd, float *cp, 
     need(n == lsdcp, "distance/contact size mismatch");
     DevBuf<float> out;
     out.alloc(2 * (size_t)lsdcp);
-    launch_sd_cp(h->stream, h->r.p, h->N, lsdcp, i_s, i_e, out.p, out.p + lsdcp, nullptr, nullptr);
+    const SdCpJob job{i_s, i_e, lsdcp, out.p, out.p + lsdcp, nullptr, nullptr};
+    launch_sd_cp(h->stream, h->r.p, h->N, &job, 1);
     hip_check(hipGetLastError());
     hip_check(hipMemcpyAsync(sd, out.p, lsdcp * sizeof(float), hipMemcpyDeviceToHost, h->stream));
     hip_check(hipMemcpyAsync(cp, out.p + lsdcp, lsdcp * sizeof(float), hipMemcpyDeviceToHost, h->stream));
@@ -1417,7 +1418,7 @@ int ccp_frame_contact_map(ccp_sim *h, float *cm, size_t lcm) {
     need(cm && lcm == (size_t)cms * (cms + 1) / 2, "contact map size mismatch");
     DevBuf<float> out;
     out.alloc(lcm);
-    launch_ccp_cm(h->stream, h->N, (uint32_t)lcm, h->r.p, out.p, nullptr);
+    launch_ccp_cm(h->stream, h->N, cms, (uint32_t)lcm, h->r.p, out.p, nullptr);
     hip_check(hipGetLastError());
     hip_check(hipMemcpyAsync(cm, out.p, lcm * sizeof(float), hipMemcpyDeviceToHost, h->stream));
     hip_check(hipStreamSynchronize(h->stream));
@@ -1532,13 +1533,13 @@ void add_frame(ccp_analysis *a) {
   hip_check(hipMemsetAsync(a->obs.p, 0, n_acc * sizeof(double), h->stream));
   launch_observables(h->stream, (int)h->N, (double)h->R_n, (double)h->nod, (double)RCO / 2.0, (int)nb, h->r.p,
                      a->obs.p);
+  SdCpJob jobs[6];
   for (uint32_t c = 0; c < 6; ++c) {
-    const uint32_t L = a->lsdcp[c];
-    if (!L) continue;
     double *b = a->sdcp[c].p;
-    launch_sd_cp(h->stream, h->r.p, h->N, L, a->i_s[c], a->i_e[c], nullptr, nullptr, b, b + L);
+    jobs[c] = SdCpJob{a->i_s[c], a->i_e[c], a->lsdcp[c], nullptr, nullptr, b, b + a->lsdcp[c]};
   }
-  launch_ccp_cm(h->stream, h->N, a->lcm, h->r.p, nullptr, a->cm.p);
+  launch_sd_cp(h->stream, h->r.p, h->N, jobs, 6);
+  launch_ccp_cm(h->stream, h->N, a->cms, a->lcm, h->r.p, nullptr, a->cm.p);
   hip_check(hipGetLastError());
   std::vector<double> acc(n_acc);
   hip_check(hipMemcpyAsync(acc.data(), a->obs.p, n_acc * sizeof(double), hipMemcpyDeviceToHost, h->stream));

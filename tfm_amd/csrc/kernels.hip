@@ -1789,20 +1789,20 @@ __global__ __launch_bounds__(BEAD_BLOCK) void k_noise(KParams p, uint64_t step, 
   out[i] = make_float4(z0, z1, z2, __uint_as_float(a));
 }
 
-// ccp's per-frame observables (chrana.cu:372-480) summed in FP64: out[0..2]
-// sum of r, [3] sum of |r|^2, [4] sum of the bond order P2(cos), [5] beads
-// with z < nod, then the radial density of A, B and all beads (3 x n_b,
-// lens volume of a bead of radius a inside the sphere of each bin edge,
-// differenced bin by bin).
 // Volume of a bead of radius a at distance d from the centre inside each of
-// n_b shells of equal volume (edges R_n cbrt((k + 1) / n_b)), as lens
-// volumes at the outer edge differenced bin by bin; add(k, net) receives the
-// nonzero differences.
-template <class F> __device__ __forceinline__ void lens_bins(double d, double a, double R_n, int n_b, F &&add) {
+// n_b shells of equal volume (edges R_n root(k), root(k) = cbrt((k + 1) / n_b)),
+// as lens volumes at the outer edge differenced bin by bin; add(k, net)
+// receives the nonzero differences. The bins inside the bead's near side are
+// all zero: the scan starts a few bins before the first edge beyond d - a
+// (the start from an FP32 cube, two bins early for its rounding).
+template <class E, class F>
+__device__ __forceinline__ void lens_bins(double d, double a, double R_n, int n_b, E &&root, F &&add) {
   const double vb = 4.0 / 3.0 * M_PI * a * a * a;
   double prev = 0.0;
-  for (int k = 0; k < n_b; ++k) {
-    const double rb = R_n * cbrt((k + 1.0) / n_b);
+  const float in = fmaxf((float)((d - a) / R_n), 0.0f);
+  const int k0 = (int)fminf((float)n_b * in * in * in * 0.9999f, (float)n_b) - 2;
+  for (int k = max(k0, 0); k < n_b; ++k) {
+    const double rb = R_n * root(k);
     double v;
     if (d - a > rb) v = 0.0;
     else if (d + a < rb) v = vb;
@@ -1818,89 +1818,226 @@ template <class F> __device__ __forceinline__ void lens_bins(double d, double a,
     if (v == vb) break; // the rest of the bins see no change
   }
 }
+// the bins' cube roots, once per workgroup where they fit its table (an FP64
+// cube root per bead and bin was most of the kernels' time)
+constexpr int LENS_TABLE = 1024;
+struct LensRoots {
+  const double *table; // n_b entries, or nullptr: more bins than the table holds
+  int n_b;
+  __device__ __forceinline__ double operator()(int k) const { return table ? table[k] : cbrt((k + 1.0) / n_b); }
+};
+__device__ __forceinline__ LensRoots lens_roots(double *table, int n_b) {
+  if (n_b > LENS_TABLE) return LensRoots{nullptr, n_b};
+  for (int k = threadIdx.x; k < n_b; k += blockDim.x) table[k] = cbrt((k + 1.0) / n_b);
+  return LensRoots{table, n_b}; // (the caller's barrier comes before its use)
+}
 
+// sum over the 64 lanes (all active), in lane 0
+__device__ __forceinline__ double wave_sum_d(double v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o);
+  return v;
+}
+
+// ccp's per-frame observables (chrana.cu:372-480) summed in FP64: out[0..2]
+// sum of r, [3] sum of |r|^2, [4] sum of the bond order P2(cos), [5] beads
+// with z < nod, then the radial density of A, B and all beads (3 x n_b,
+// lens volume of a bead of radius a inside the sphere of each bin edge,
+// differenced bin by bin). The six scalars are summed over each wavefront by
+// shuffles (all lanes adding to one LDS word queued up behind each other), which
+// with the table and the scan start takes 8.4 us at N = 30386 instead of 46.
 __global__ __launch_bounds__(BEAD_BLOCK) void k_observables(int N, double R_n, double nod, double a, int n_b,
                                                             const float4 *pos, double *out) {
   extern __shared__ double s_acc[];
+  __shared__ double s_root[LENS_TABLE];
   const int tid = threadIdx.x, n_acc = 6 + 3 * n_b;
   for (int k = tid; k < n_acc; k += BEAD_BLOCK) s_acc[k] = 0.0;
+  const LensRoots root = lens_roots(s_root, n_b);
   __syncthreads();
   const int i = blockIdx.x * BEAD_BLOCK + tid;
+  double v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   if (i < N) {
     const float4 q = pos[i];
     const double x = q.x, y = q.y, z = q.z;
-    atomicAdd(&s_acc[0], x);
-    atomicAdd(&s_acc[1], y);
-    atomicAdd(&s_acc[2], z);
     const double d2 = x * x + y * y + z * z;
-    atomicAdd(&s_acc[3], d2);
+    v[0] = x;
+    v[1] = y;
+    v[2] = z;
+    v[3] = d2;
     if (i + 1 < N) {
       const float4 n = pos[i + 1];
       const double vx = (double)n.x - x, vy = (double)n.y - y, vz = (double)n.z - z;
       const double c = (vx * x + vy * y + vz * z) / (sqrt(vx * vx + vy * vy + vz * vz) * sqrt(d2));
-      atomicAdd(&s_acc[4], 0.5 * (3.0 * c * c - 1.0));
+      v[4] = 0.5 * (3.0 * c * c - 1.0);
     }
-    if (z < nod) atomicAdd(&s_acc[5], 1.0);
+    if (z < nod) v[5] = 1.0;
     const int t = (wbits(q) & W_HET) ? 0 : 1;
-    lens_bins(sqrt(d2), a, R_n, n_b, [&](int k, double net) {
-      atomicAdd(&s_acc[6 + t * n_b + k], net);
-      atomicAdd(&s_acc[6 + 2 * n_b + k], net);
-    });
+    lens_bins(sqrt(d2), a, R_n, n_b, root, [&](int k, double net) { atomicAdd(&s_acc[6 + t * n_b + k], net); });
   }
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {
+    const double s = wave_sum_d(v[k]);
+    if ((tid & 63) == 0) atomicAdd(&s_acc[k], s);
+  }
+  __syncthreads();
+  // the row of all beads is the sum of the other two
+  for (int k = tid; k < n_b; k += BEAD_BLOCK) s_acc[6 + 2 * n_b + k] = s_acc[6 + k] + s_acc[6 + n_b + k];
   __syncthreads();
   for (int k = tid; k < n_acc; k += BEAD_BLOCK)
     if (s_acc[k] != 0.0) atomicAdd(&out[k], s_acc[k]);
 }
 
 // Radial density of every system of a batch (the all-bead row of
-// k_observables), one lane per bead, FP64 sums into out[s n_b + k].
+// k_observables), one lane per bead, FP64 sums into out[s n_b + k]. The
+// workgroup's beads mostly belong to one system: that of its first bead is
+// summed in LDS and added once per bin, the others' beads go out directly.
 __global__ __launch_bounds__(BEAD_BLOCK) void k_radial_batch(const SysParams *sys, const uint32_t *sys_slot,
                                                              int n_sys, int n, double a, int n_b, const float4 *pos,
                                                              double *out) {
+  __shared__ double s_root[LENS_TABLE], s_acc[LENS_TABLE];
   const int i = blockIdx.x * BEAD_BLOCK + threadIdx.x;
-  if (i >= n) return;
-  const int s = system_of(sys_slot, n_sys, (uint32_t)i);
-  const float4 q = pos[i];
-  const double x = q.x, y = q.y, z = q.z;
-  double *o = out + (size_t)s * n_b;
-  lens_bins(sqrt(x * x + y * y + z * z), a, (double)sys[s].R_n, n_b, [&](int k, double net) { atomicAdd(o + k, net); });
+  const int first = system_of(sys_slot, n_sys, (uint32_t)(blockIdx.x * BEAD_BLOCK));
+  const LensRoots root = lens_roots(s_root, n_b);
+  const bool local = n_b <= LENS_TABLE;
+  if (local)
+    for (int k = threadIdx.x; k < n_b; k += BEAD_BLOCK) s_acc[k] = 0.0;
+  __syncthreads();
+  if (i < n) {
+    const int s = system_of(sys_slot, n_sys, (uint32_t)i);
+    const float4 q = pos[i];
+    const double x = q.x, y = q.y, z = q.z;
+    const bool here = local && s == first;
+    lens_bins(sqrt(x * x + y * y + z * z), a, (double)sys[s].R_n, n_b, root, [&](int k, double net) {
+      if (here) atomicAdd(&s_acc[k], net);
+      else atomicAdd(out + (size_t)s * n_b + k, net);
+    });
+  }
+  __syncthreads();
+  if (local)
+    for (int k = threadIdx.x; k < n_b; k += BEAD_BLOCK)
+      if (s_acc[k] != 0.0) atomicAdd(out + (size_t)first * n_b + k, s_acc[k]);
 }
 
-// ccp's d(s) and 1000 P(s) of one chromosome (calc_sd_cp, chrana.cu:13-45):
-// one thread per separation s = ia + 1, FP32 sums over the pairs (p, p+s) of
-// beads [i_s, i_e) and, when N = 30386, of the homologue N/2 further on.
-// Writes the frame's values to sd/cp and, when given, adds them to the FP64
-// per-simulation sums as ccp's host loop does (chrana.cu:496-502).
-__global__ __launch_bounds__(BEAD_BLOCK) void k_sd_cp(const float4 *pos, uint32_t N, uint32_t lsdcp, uint32_t i_s,
-                                                      uint32_t i_e, float *sd, float *cp, double *sum_sd,
-                                                      double *sum_cp) {
+// ccp's d(s) and 1000 P(s) of one or several chromosomes (calc_sd_cp,
+// chrana.cu:13-45): FP32 sums over the pairs (p, p+s) of beads [i_s, i_e)
+// and, when N = 30386, of the homologue N/2 further on, for every separation
+// s = 1 .. lsdcp. Writes the frame's values to sd/cp and, when given, adds
+// them to the FP64 per-simulation sums as ccp's host loop does
+// (chrana.cu:496-502). blockIdx.y is the chromosome.
+//
+// ccp adds a separation's distances one after the other in FP32, so the sum
+// of one separation is a serial chain of up to 2 (i_e - i_s) additions and
+// only the distances can be computed in any order. One lane doing both waits
+// for its loads on every pair (180 ns a pair, with 18 to 25 wavefronts on the
+// whole chip). Here a workgroup takes 32 separations: seven wavefronts
+// compute the distances of 64 starting beads x 32 separations into LDS while
+// the first one adds the previous tile's in ccp's order, and the positions of
+// the tile after next are on their way. 32 separations, not 64: the distances of a tile (about 30 VALU
+// instructions each, on one CU) then take as long as its additions.
+// N = 30386, six chromosomes of 2284 to 3170 beads, a launch each: 897 -> 76 us
+// (124 us with 64 separations, the distances then the longer part).
+constexpr int SD_S = 32, SD_P = 64, SD_THREADS = 512;
+constexpr int SD_WAVES = SD_THREADS / 64 - 1; // wavefronts that compute distances
+__global__ __launch_bounds__(SD_THREADS) void k_sd_cp(const float4 *__restrict__ pos, uint32_t N, SdCpJobs jobs) {
 #pragma clang fp contract(off)
-  const uint32_t ia = blockIdx.x * BEAD_BLOCK + threadIdx.x;
-  if (ia >= lsdcp) return;
-  const uint32_t s = ia + 1, ncc = (N == 30386u) ? 2u : 1u;
-  float a = 0.0f, c = 0.0f;
-  for (uint32_t k = 0; k < ncc; ++k) {
-    for (uint32_t p = i_s; p < i_e - s; ++p) {
-      const float4 u = pos[p], v = pos[p + s];
-      const float dx = v.x - u.x, dy = v.y - u.y, dz = v.z - u.z;
+  const SdCpJob J = jobs.job[blockIdx.y];
+  const uint32_t s0 = 1u + blockIdx.x * SD_S;
+  if (s0 > J.lsdcp) return;
+  __shared__ float s_d[2][SD_P][SD_S];
+  // the tile's first beads p0 .. p0 + 63, then those s0 .. s0 + SD_P + SD_S - 1 further on
+  __shared__ float4 s_pos[2][SD_P + SD_P + SD_S];
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const uint32_t ncc = (N == 30386u) ? 2u : 1u;
+  const uint32_t n_p = J.i_e - J.i_s - s0; // starting beads of the shortest separation
+  const uint32_t per = (n_p + SD_P - 1u) / SD_P, tiles = ncc * per;
+  auto tile_start = [&](uint32_t t) { return J.i_s + (t / per) * (N / ncc) + (t % per) * SD_P; };
+  // positions of tile t, one per lane of the wavefronts 1 to 3 (clamped: a
+  // value past the chain belongs to pairs that are not added)
+  const bool loads = tid >= 64 && tid < 64 + SD_P + SD_P + SD_S;
+  const uint32_t slot = (uint32_t)tid - 64u;
+  auto load_pos = [&](uint32_t t) {
+    const uint32_t p0 = tile_start(t);
+    return pos[min(slot < (uint32_t)SD_P ? p0 + slot : p0 + s0 + (slot - SD_P), N - 1u)];
+  };
+  auto distances = [&](uint32_t t) {
+    const float4 *u = s_pos[t & 1u], *v = s_pos[t & 1u] + SD_P;
+    // a wavefront takes two starting beads at a time, half its lanes each
+    const int sep = lane % SD_S;
+#pragma unroll 5
+    for (int r = 2 * (wid - 1) + lane / SD_S; r < SD_P; r += 2 * SD_WAVES) {
+      const float4 a = u[r], b = v[r + sep];
+      const float dx = b.x - a.x, dy = b.y - a.y, dz = b.z - a.z;
       const float xx = dx * dx, yy = dy * dy, zz = dz * dz;
-      const float d = sqrtf((xx + yy) + zz);
-      a += d;
-      if (d < 2.0f) c += 1000.0f;
+      s_d[t & 1u][r][sep] = sqrtf((xx + yy) + zz);
     }
-    i_s += N / ncc;
-    i_e += N / ncc;
+  };
+  if (loads) {
+    s_pos[0][slot] = load_pos(0u);
+    if (tiles > 1u) s_pos[1][slot] = load_pos(1u);
   }
-  const float m = (float)(ncc * (i_e - i_s - s));
+  __syncthreads();
+  if (wid > 0) distances(0u);
+  __syncthreads();
+  const uint32_t s = s0 + (uint32_t)(lane % SD_S);
+  // ccp adds 1000 per contact in FP32: exact, whatever the order, while the
+  // sum is at most 2^24 times 8 (the largest power of two in 1000)
+  const bool counts = ncc * (J.i_e - J.i_s) <= (1u << 27) / 1000u;
+  float a = 0.0f, c = 0.0f;
+  uint32_t n = 0;
+  // the additions are the long chain: their wavefront goes first on its SIMD
+  if (wid == 0) __builtin_amdgcn_s_setprio(3);
+  for (uint32_t t = 0; t < tiles; ++t) {
+    if (wid == 0) {
+      const float(*d)[SD_S] = s_d[t & 1u];
+      const uint32_t q = (t % per) * SD_P; // first starting bead of the tile, from the chromosome's first
+      if (counts && q + SD_P + s0 + SD_S - 1u <= J.i_e - J.i_s) {
+        // every pair of the tile is inside the chromosome
+#pragma unroll
+        for (int r0 = 0; r0 < SD_P; r0 += 16) {
+          float x[16];
+#pragma unroll
+          for (int r = 0; r < 16; ++r) x[r] = d[r0 + r][lane % SD_S];
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            a += x[r];
+            n += x[r] < 2.0f ? 1u : 0u;
+          }
+        }
+      } else {
+        for (int r = 0; r < SD_P; ++r) {
+          const float x = d[r][lane % SD_S];
+          if (q + (uint32_t)r + s < J.i_e - J.i_s) {
+            a += x;
+            if (x < 2.0f) {
+              c += 1000.0f;
+              ++n;
+            }
+          }
+        }
+      }
+    } else {
+      float4 next = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      const bool more = loads && t + 2u < tiles;
+      if (more) next = load_pos(t + 2u);
+      if (t + 1u < tiles) distances(t + 1u);
+      // tile t's positions were read in the round before this one
+      if (more) s_pos[t & 1u][slot] = next;
+    }
+    __syncthreads();
+  }
+  if (tid >= SD_S || s > J.lsdcp) return;
+  const uint32_t ia = s - 1u;
+  if (counts) c = (float)(1000u * n);
+  const float m = (float)(ncc * (J.i_e - J.i_s - s));
   a /= m;
   c /= m;
-  if (sd) {
-    sd[ia] = a;
-    cp[ia] = c;
+  if (J.sd) {
+    J.sd[ia] = a;
+    J.cp[ia] = c;
   }
-  if (sum_sd) {
-    sum_sd[ia] += (double)a;
-    sum_cp[ia] += (double)c;
+  if (J.sum_sd) {
+    J.sum_sd[ia] += (double)a;
+    J.sum_cp[ia] += (double)c;
   }
 }
 
@@ -1909,32 +2046,101 @@ __global__ __launch_bounds__(BEAD_BLOCK) void k_sd_cp(const float4 *pos, uint32_
 // contact if |r_p - r_q| < 2, factor 1000, average over the two chromosome
 // copies when N = 30386. Writes the frame's map to cm and, when given, adds
 // it to the FP64 per-simulation sum (chrana.cu:505-511).
-__global__ __launch_bounds__(BEAD_BLOCK) void k_ccp_cm(uint32_t N, uint32_t lcm, const float4 *pos, float *cm,
-                                                       double *sum) {
+//
+// sqrtf(x) < 2 and x < 4 select the same FP32 values x (the root is rounded
+// correctly, and the root of the largest float below 4 rounds below 2).
+__device__ __forceinline__ float cm_pixel(const float4 *__restrict__ pos, uint32_t N, uint32_t ncc, uint32_t ix,
+                                          uint32_t iy) {
 #pragma clang fp contract(off)
-  const uint32_t ia = blockIdx.x * BEAD_BLOCK + threadIdx.x;
-  if (ia >= lcm) return;
-  const uint32_t px = 4, ncc = (N == 30386u) ? 2u : 1u, cms = (N / ncc) / px;
-  // ccp's pixel coordinates; the clamps keep the reads inside the chain
-  // where the FP32 root of a large index would round past the last row
-  const uint32_t ixp = min((uint32_t)((double)sqrtf((float)(2.0 * ia + 0.25)) - 0.5), cms - 1);
-  const uint32_t iyp = min((uint32_t)(ia - ixp * (ixp + 1.0) / 2.0), cms - 1);
-  uint32_t sx = ixp * px, ex = sx + px, sy = iyp * px, ey = sy + px;
-  float acc = 0.0f;
+  uint32_t n = 0;
   for (uint32_t c = 0; c < ncc; ++c) {
-    for (uint32_t p = sx; p < ex; ++p)
-      for (uint32_t q = sy; q < ey; ++q) {
-        const float4 u = pos[p], v = pos[q];
-        const float dx = u.x - v.x, dy = u.y - v.y, dz = u.z - v.z;
+    const float4 *u = pos + c * (N / ncc) + 4u * ix, *v = pos + c * (N / ncc) + 4u * iy;
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float dx = u[p].x - v[q].x, dy = u[p].y - v[q].y, dz = u[p].z - v[q].z;
         const float xx = dx * dx, yy = dy * dy, zz = dz * dz;
-        const float d = sqrtf((xx + yy) + zz);
-        if (d < 2.0f) acc += 1000.0f;
+        n += ((xx + yy) + zz) < 4.0f ? 1u : 0u;
       }
-    sx += N / ncc; ex += N / ncc; sy += N / ncc; ey += N / ncc;
   }
-  const float v = acc / (float)(ncc * px * px);
-  if (cm) cm[ia] = v;
-  if (sum) sum[ia] += (double)v;
+  // whole thousands of at most 32 contacts: exact in FP32, as ccp's sum of them
+  return (float)(1000u * n) / (float)(ncc * 16u);
+}
+
+// First bead and the distance of the farthest of a pixel's other three, with
+// which two pixels that hold no contact are told apart without their 16
+// pairs. The bound only has to hold up to the rounding of its own few
+// operations (1e-6 of each distance): CM_REACH is 0.5 % above 2, and the sum
+// is widened by 1e-4 of itself. A first bead at NaN fails the test and takes
+// the pairs.
+constexpr float CM_REACH = 2.01f, CM_WIDEN = 1.0001f;
+__device__ __forceinline__ float4 cm_bound(const float4 *__restrict__ p) {
+  const float4 a = p[0];
+  float r2 = 0.0f;
+#pragma unroll
+  for (int k = 1; k < 4; ++k) {
+    const float4 b = p[k];
+    const float d2 = dist2(b.x - a.x, b.y - a.y, b.z - a.z);
+    r2 = fmaxf(r2, d2); // (a bead at NaN is in no contact: its distance may drop out)
+  }
+  return make_float4(a.x, a.y, a.z, sqrtf(r2));
+}
+__device__ __forceinline__ bool cm_apart(float4 a, float4 b) {
+  const float t = (CM_REACH + a.w + b.w) * CM_WIDEN;
+  return dist2(a.x - b.x, a.y - b.y, a.z - b.z) > t * t;
+}
+
+// One lane per column pixel of a block of CM_COLS columns x CM_ROWS rows. A
+// packed row is contiguous, so the stores are coalesced, and a column's
+// bound is loaded once for CM_ROWS pixels. Nearly every pixel is empty (a
+// contact reaches 2 sigma in a nucleus of tens), so the test of the bounds
+// decides all but a few per cent of the wavefronts' pixels; one lane per
+// packed pixel evaluating its 32 pairs took 253 us at N = 30386 (7.2 M pixels);
+// this takes 68 us, 16 rows a block (111 us with 64: a block with contacts then
+// holds up the launch).
+constexpr int CM_COLS = 256, CM_ROWS = 16;
+__global__ __launch_bounds__(CM_COLS) void k_ccp_cm(uint32_t N, uint32_t cms, uint32_t lcm,
+                                                    const float4 *__restrict__ pos, float *cm, double *sum) {
+  const uint32_t col0 = blockIdx.x * CM_COLS, row0 = blockIdx.y * CM_ROWS;
+  if (col0 > row0 + CM_ROWS - 1u) return;
+  const uint32_t ncc = (N == 30386u) ? 2u : 1u;
+  __shared__ float4 s_row[2][CM_ROWS];
+  for (uint32_t k = threadIdx.x; k < ncc * CM_ROWS; k += CM_COLS) {
+    const uint32_t c = k / CM_ROWS, r = min(row0 + k % CM_ROWS, cms - 1u);
+    s_row[c][k % CM_ROWS] = cm_bound(pos + c * (N / ncc) + 4u * r);
+  }
+  const uint32_t col = col0 + threadIdx.x;
+  float4 mine[2];
+#pragma unroll
+  for (uint32_t c = 0; c < 2u; ++c)
+    mine[c] = cm_bound(pos + (c < ncc ? c : 0u) * (N / ncc) + 4u * min(col, cms - 1u));
+  __syncthreads();
+  for (uint32_t k = 0; k < (uint32_t)CM_ROWS; ++k) {
+    const uint32_t row = row0 + k;
+    if (row >= cms) break;
+    if (col > row) continue;
+    const uint32_t ia = (uint32_t)((uint64_t)row * (row + 1u) / 2u) + col;
+    uint32_t ix = row, iy = col;
+    // ccp finds the row as an FP32 root of the packed index, which near a
+    // row's ends may round to a neighbouring row (by less than 0.008 of the
+    // row's length up to 65535 rows). The pixels close to an end take ccp's
+    // row and column; the clamps keep the reads inside the chain where the
+    // root would round past the last row.
+    const float edge = 0.01f * (float)(row + 1u) + 1.0f;
+    if ((float)col < edge || (float)(row - col) < edge) {
+      ix = min((uint32_t)((double)sqrtf((float)(2.0 * ia + 0.25)) - 0.5), cms - 1u);
+      iy = min((uint32_t)(ia - ix * (ix + 1.0) / 2.0), cms - 1u);
+    }
+    const bool as_packed = ix == row && iy == col;
+    bool apart = cm_apart(mine[0], s_row[0][k]);
+    if (ncc == 2u) apart = apart && cm_apart(mine[1], s_row[1][k]);
+    float v = 0.0f;
+    if (!(as_packed && apart)) v = cm_pixel(pos, N, ncc, ix, iy);
+    if (cm) cm[ia] = v;
+    // (an empty pixel adds nothing)
+    if (sum && v != 0.0f) sum[ia] += (double)v;
+  }
 }
 
 // Closes one simulation of ccp's basic observables (simobs_b,
@@ -2137,15 +2343,22 @@ void launch_observables(hipStream_t s, int N, double R_n, double nod, double a, 
                                                                                                pos, out);
 }
 
-void launch_sd_cp(hipStream_t s, const float4 *pos, uint32_t N, uint32_t lsdcp, uint32_t i_s, uint32_t i_e,
-                  float *sd, float *cp, double *sum_sd, double *sum_cp) {
-  if (lsdcp == 0) return;
-  k_sd_cp<<<blocks_for((int)lsdcp, BEAD_BLOCK), BEAD_BLOCK, 0, s>>>(pos, N, lsdcp, i_s, i_e, sd, cp, sum_sd, sum_cp);
+void launch_sd_cp(hipStream_t s, const float4 *pos, uint32_t N, const SdCpJob *jobs, int n_jobs) {
+  SdCpJobs all{};
+  uint32_t n = 0, longest = 0;
+  for (int k = 0; k < n_jobs; ++k)
+    if (jobs[k].lsdcp) {
+      all.job[n++] = jobs[k];
+      longest = jobs[k].lsdcp > longest ? jobs[k].lsdcp : longest;
+    }
+  if (n == 0) return;
+  k_sd_cp<<<dim3((longest + SD_S - 1) / SD_S, n), SD_THREADS, 0, s>>>(pos, N, all);
 }
 
-void launch_ccp_cm(hipStream_t s, uint32_t N, uint32_t lcm, const float4 *pos, float *cm, double *sum) {
+void launch_ccp_cm(hipStream_t s, uint32_t N, uint32_t cms, uint32_t lcm, const float4 *pos, float *cm, double *sum) {
   if (lcm == 0) return;
-  k_ccp_cm<<<blocks_for((int)lcm, BEAD_BLOCK), BEAD_BLOCK, 0, s>>>(N, lcm, pos, cm, sum);
+  k_ccp_cm<<<dim3((cms + CM_COLS - 1) / CM_COLS, (cms + CM_ROWS - 1) / CM_ROWS), CM_COLS, 0, s>>>(N, cms, lcm, pos,
+                                                                                                cm, sum);
 }
 
 void launch_bin_batch(hipStream_t s, const SysParams *sys, const uint32_t *sys_slot, int n_sys, int n,

@@ -176,6 +176,18 @@ struct BondJob {
   int n_sys;
 };
 
+// d(s) and P(s) of one chromosome, beads [i_s, i_e): the frame's values (sd,
+// cp; may be null) and the FP64 per-simulation sums (may be null), lsdcp each.
+struct SdCpJob {
+  uint32_t i_s, i_e, lsdcp;
+  float *sd, *cp;
+  double *sum_sd, *sum_cp;
+};
+constexpr int SD_CP_JOBS = 6; // ccp's chromosomes
+struct SdCpJobs {
+  SdCpJob job[SD_CP_JOBS];
+};
+
 // Het beads per 128-lane workgroup of k_force_typed (eight lanes each).
 constexpr int TYPED_HET_BEADS_PER_BLOCK = 16;
 
@@ -216,9 +228,10 @@ void launch_overlaps(hipStream_t s, const KParams &p, const float4 *spos, const 
 void launch_noise(hipStream_t s, const KParams &p, uint64_t step, float4 *out);
 void launch_observables(hipStream_t s, int N, double R_n, double nod, double a, int n_b, const float4 *pos,
                         double *out);
-void launch_sd_cp(hipStream_t s, const float4 *pos, uint32_t N, uint32_t lsdcp, uint32_t i_s, uint32_t i_e,
-                  float *sd, float *cp, double *sum_sd, double *sum_cp);
-void launch_ccp_cm(hipStream_t s, uint32_t N, uint32_t lcm, const float4 *pos, float *cm, double *sum);
+// d(s) and P(s) of up to SD_CP_JOBS chromosomes in one launch
+void launch_sd_cp(hipStream_t s, const float4 *pos, uint32_t N, const SdCpJob *jobs, int n_jobs);
+// packed map of cms x cms pixels (lcm = cms (cms + 1) / 2 of them)
+void launch_ccp_cm(hipStream_t s, uint32_t N, uint32_t cms, uint32_t lcm, const float4 *pos, float *cm, double *sum);
 void launch_bin_batch(hipStream_t s, const SysParams *sys, const uint32_t *sys_slot, int n_sys, int n,
                       const float4 *pos, uint32_t *count, uint32_t *blocksum, float4 *bucket, uint32_t *flags,
                       uint32_t *hblocksum = nullptr);
