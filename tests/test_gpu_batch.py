@@ -231,3 +231,29 @@ def test_ensemble_full_size_half_cells():
     xyz, _ = b.state()
     assert np.isfinite(xyz).all()
     b.close()
+
+
+@pytest.mark.parametrize("size", [1.25, 1.49, 1.5])
+def test_batch_scan_blocks_at_system_edges(size):
+    # systems whose cells end inside a scan block (256 cells, 512 below 1.5
+    # sigma), from a handful of beads up: each system's positions and contact
+    # map equal the single run's
+    step(f"batch scan blocks, cells of {size}")
+    systems = [dict(n_beads=n, volume_fraction=v, eps_het=0.6, eps_lam=1.0, het_fraction=0.3, lad_fraction=0.1,
+                    seed=6000 + n) for n, v in ((5, 0.1), (40, 0.3), (33, 0.02), (700, 0.25), (12, 0.2))]
+    b = tfm_amd.Batch(systems, dict(timestep=0.001, contact_interval=20, graph_steps=10, lanes_per_bead=8,
+                                    cell_reach=2, cell_size=size))
+    b.generate_initial_conditions()
+    xyz0, fl0 = b.state()
+    b.run_steps(40)
+    xyz, _ = b.state()
+    maps, _ = b.contact_maps()
+    for s in range(len(systems)):
+        sim = single_from(b, s, xyz0, fl0)
+        sim.run_steps(40)
+        o0, o1 = b.offsets[s], b.offsets[s + 1]
+        assert np.array_equal(sim.positions, xyz[o0:o1]), s
+        m, _ = sim.contact_map()
+        assert np.array_equal(m, maps[s][:len(m), :len(m)]), s
+        sim.close()
+    b.close()

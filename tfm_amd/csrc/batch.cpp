@@ -30,6 +30,7 @@ struct BatchGrid {
   DevBuf<uint32_t> count, bs0, bs1, cstart;
   DevBuf<float4> bucket, spos; // bucket: members' positions, index in the w bits
   DevBuf<uint32_t> hbs0, hbs1, work; // type-ordered work list (k_force_typed)
+  DevBuf<OrderBlock> blocks;         // g.nblk scan blocks, each of one system
   int clean = 0;
   bool valid = false;
   uint32_t *bs(int k) { return k ? bs1.p : bs0.p; }
@@ -41,6 +42,7 @@ struct BatchGrid {
     bucket.alloc((size_t)g.n_c * g.cap);
     cstart.alloc((size_t)g.n_c + 1);
     spos.alloc(n_obj);
+    blocks.alloc(g.nblk);
     hip_check(hipMemset(count.p, 0, (size_t)g.n_c * 4));
     hip_check(hipMemset(bs0.p, 0, (size_t)g.nblk * 4));
     hip_check(hipMemset(bs1.p, 0, (size_t)g.nblk * 4));
@@ -61,7 +63,9 @@ struct BatchGrid {
     for (auto *b : u) b->free_();
     bucket.free_();
     spos.free_();
+    blocks.free_();
   }
+  OrderTable table() const { return {blocks.p, 1 << (g.bshift - SCAN_SHIFT)}; }
   OrderJob order_job(uint32_t n_het, uint32_t n_slots) {
     OrderJob j{g, count.p, bs(clean), bs(clean ^ 1), bucket.p, spos.p, nullptr, cstart.p};
     if (work.p) {
@@ -147,8 +151,24 @@ struct ccp_batch {
       h[i] = make_float4(hr[3 * i], hr[3 * i + 1], hr[3 * i + 2], wf);
     }
     hip_check(hipMemcpyAsync(r.p, h.data(), (size_t)N * sizeof(float4), hipMemcpyHostToDevice, stream));
+    const std::vector<OrderBlock> ob = order_blocks();
+    hip_check(hipMemcpyAsync(grid.blocks.p, ob.data(), ob.size() * sizeof(OrderBlock), hipMemcpyHostToDevice, stream));
     hip_check(hipStreamSynchronize(stream));
     grid.valid = false;
+  }
+  // the scan blocks of every system's cells, with the slots and the het beads
+  // of the systems before it
+  std::vector<OrderBlock> order_blocks() const {
+    std::vector<OrderBlock> ob;
+    ob.reserve(grid.g.nblk);
+    uint32_t het = 0;
+    for (const SysParams &S : sys) {
+      const int cells = 1 << S.g.bshift;
+      for (int c = 0; c < S.g.n_c; c += cells)
+        ob.push_back({S.g.coff + c, std::min(cells, S.g.n_c - c), (uint32_t)S.g.boff, S.slot, het});
+      for (uint32_t i = S.slot; i < S.slot + S.n; ++i) het += (hfl[i] & CCP_HET) ? 1u : 0u;
+    }
+    return ob;
   }
   void download() {
     std::vector<float4> h(N);
@@ -186,7 +206,7 @@ struct ccp_batch {
       launch_bin_batch(stream, dsys.p, dslot.p, (int)n_sys, (int)N, r.p, grid.count.p, grid.bs(grid.clean),
                        grid.bucket.p, flags.p, grid.work.p ? grid.hbs(grid.clean) : nullptr);
       const OrderJob j = grid.order_job((uint32_t)kp.n_het, N);
-      launch_order(stream, j, nullptr, flags.p, nullptr);
+      launch_order(stream, j, nullptr, flags.p, nullptr, nullptr, nullptr, nullptr, grid.table());
       hip_check(hipGetLastError());
       grid.clean ^= 1;
       if (!take_overflow()) break;
@@ -271,7 +291,7 @@ struct ccp_batch {
     const NoiseJob nj = noise_job(1);
     const BondJob bj = bond_job(q.out0, mode);
     launch_order(stream, j, nullptr, flags.p, stage == 2 ? dstep.p : nullptr, stage == 1 ? &nj : nullptr, &k,
-                 bond_pass() ? &bj : nullptr);
+                 bond_pass() ? &bj : nullptr, grid.table());
     grid.clean ^= 1;
   }
   void run_chunk(uint64_t n) {
@@ -462,7 +482,7 @@ void plan_batch(ccp_batch &bt, const char *common_params, const ccp_batch_system
   if (!(1 <= b->rd_bins && b->rd_bins <= 1024)) throw Error(CCP_ERR_PARAM, "radial_bins out of range");
   b->n_sys = n_sys;
   b->slot.push_back(0);
-  int coff = 0;
+  int coff = 0, boff = 0;
   uint64_t total = 0;
   for (uint32_t s = 0; s < n_sys; ++s) {
     const ccp_batch_system &in = systems[s];
@@ -486,6 +506,12 @@ void plan_batch(ccp_batch &bt, const char *common_params, const ccp_batch_system
     S.n = one.N;
     S.g = one.gf.g;
     S.g.coff = coff;
+    S.g.boff = boff;
+    // Two cells per lane of the order pass for cells of about a bead each, so
+    // that a block's members still fit its LDS (1024) with room to spare;
+    // larger cells (2.5 sigma: six beads) keep one.
+    S.g.bshift = S.g.csl < 1.5f ? SCAN_SHIFT + 1 : SCAN_SHIFT;
+    S.g.nblk = (S.g.n_c + (1 << S.g.bshift) - 1) >> S.g.bshift;
     if (s == 0) {
       b->kp = one.kp;
       b->contact_rc = one.contact_rc;
@@ -505,6 +531,7 @@ void plan_batch(ccp_batch &bt, const char *common_params, const ccp_batch_system
     // fit the 32-bit offsets of the force kernels' row loads
     if ((uint64_t)coff + (uint64_t)one.gf.g.n_c >= (1ull << 30)) throw Error(CCP_ERR_PARAM, "batch too large");
     coff += one.gf.g.n_c;
+    boff += S.g.nblk;
     total += one.N;
     if (total >= (1ull << ID_BITS)) throw Error(CCP_ERR_PARAM, "batch too large");
     b->slot.push_back((uint32_t)total);
@@ -521,7 +548,8 @@ void plan_batch(ccp_batch &bt, const char *common_params, const ccp_batch_system
   b->grid.g = b->kp.gf;
   b->grid.g.n_c = coff;
   b->grid.g.coff = 0;
-  b->grid.g.nblk = (coff + SCAN_BLOCK - 1) / SCAN_BLOCK;
+  b->grid.g.nblk = boff;
+  b->grid.g.bshift = b->sys[0].g.bshift;
   b->hr.assign(3 * (size_t)b->N, 0.0f);
   b->hfl.assign(b->N, 0);
   b->rd_sum.assign((size_t)n_sys * b->rd_bins, 0.0);

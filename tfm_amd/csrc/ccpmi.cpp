@@ -126,6 +126,7 @@ void ccp_sim::configure(const ParMap &par) {
     g.n_c = (int)(cps * cps * cps);
     g.cap = (int)capacity;
     g.nblk = (g.n_c + SCAN_BLOCK - 1) / SCAN_BLOCK;
+    g.bshift = SCAN_SHIFT;
     return g;
   };
   gh.g = geometry(csl, cap);

@@ -36,6 +36,8 @@
 
 #include "kernels.hpp"
 
+#include <type_traits>
+
 namespace ccpmi {
 namespace {
 
@@ -201,12 +203,13 @@ __device__ __forceinline__ void bin_into(const GridGeom &g, uint32_t *count, uin
                                          uint32_t *flags, float4 v, uint32_t *hblocksum = nullptr) {
   bool outside = false;
   const int gx = cell_coord(v.x, g, outside), gy = cell_coord(v.y, g, outside), gz = cell_coord(v.z, g, outside);
-  const uint32_t key = (uint32_t)(g.coff + (gz * g.cps + gy) * g.cps + gx);
+  const uint32_t cell = (uint32_t)((gz * g.cps + gy) * g.cps + gx), key = (uint32_t)g.coff + cell;
   // beads of one wavefront mostly sit in distinct cells: plain atomics
   const uint32_t slot = atomicAdd(count + key, 1u);
   // the block totals and the flag need no slot: done while it returns
-  agg_add_noret(blocksum, key / SCAN_BLOCK);
-  if (hblocksum && (wbits(v) & W_HET)) agg_add_noret(hblocksum, key / SCAN_BLOCK);
+  const uint32_t blk = (uint32_t)g.boff + (cell >> g.bshift);
+  agg_add_noret(blocksum, blk);
+  if (hblocksum && (wbits(v) & W_HET)) agg_add_noret(hblocksum, blk);
   if (outside) atomicAdd(flags + FLAG_OUTSIDE, 1u);
   if (slot < (uint32_t)g.cap) bucket[(size_t)key * g.cap + slot] = v;
 }
@@ -1485,37 +1488,66 @@ __global__ __launch_bounds__(BEAD_BLOCK) void k_bin_batch(const SysParams *sys, 
 // in the w bits. The block's entries are staged in LDS; each entry's rank
 // within its cell (number of smaller indices) is then found in parallel and
 // the entry written to its sorted slot.
+//
+// BATCH: the scan blocks come from a table, each holding cells of one system
+// (CPT per lane). That system's first slot is known, so a block's prefix
+// starts at the system's first block, and a block with no members (nearly
+// half lie outside the nucleus) only writes its starts. With one run of
+// 256-cell blocks over all systems every block read the totals of all blocks
+// before it; 256 systems of 2048 beads over 1.375 sigma cells (3.3 M cells)
+// took 46.6 us a launch, 30 us with the table, 27.4 us with two cells per lane
+// (cells below 1.5 sigma, about one bead each: half as many workgroups, each
+// waiting out the same chain of loads) and the early end of empty blocks.
 constexpr int ORDER_LDS = 1024;
 
-__global__ __launch_bounds__(SCAN_BLOCK) void k_order(OrderJob ja, OrderJob jb, uint32_t *flags,
-                                                      uint64_t *step_inc, NoiseJob nj, KParams bp, BondJob bj) {
+//
+// TWO: a second grid's blocks follow the first's (the het grid of the split
+// pair sum). Without it the job's fields are plain kernel arguments, not
+// loads through a selected address.
+template <int N_JOBS> struct OrderJobs {
+  OrderJob j[N_JOBS];
+};
+template <bool BATCH, int CPT, bool TWO>
+__global__ __launch_bounds__(SCAN_BLOCK) void k_order(OrderJobs<TWO ? 2 : 1> jobs, const OrderBlock *blocks,
+                                                      uint32_t *flags, uint64_t *step_inc, NoiseJob nj, KParams bp,
+                                                      BondJob bj) {
+  static_assert(BATCH || CPT == 1, "a single system's blocks hold one cell per lane");
+  static_assert(!(BATCH && TWO), "a batch has one grid");
+  constexpr int CELLS = SCAN_BLOCK * CPT; // cells of a full block
   __shared__ uint32_t red[SCAN_BLOCK / 64], wsum[SCAN_BLOCK / 64], msum[SCAN_BLOCK / 64];
   __shared__ uint32_t hred[SCAN_BLOCK / 64], hsum[SCAN_BLOCK / 64];
   __shared__ uint32_t s_id[ORDER_LDS];
   __shared__ float4 s_pos[ORDER_LDS];
-  __shared__ uint8_t s_cell[ORDER_LDS];
-  __shared__ uint32_t s_loff[SCAN_BLOCK + 1];
-  __shared__ uint32_t s_start[SCAN_BLOCK];
-  __shared__ uint32_t s_hoff[SCAN_BLOCK];
+  __shared__ std::conditional_t<(CPT > 1), uint16_t, uint8_t> s_cell[ORDER_LDS];
+  __shared__ uint32_t s_loff[CELLS + 1];
+  __shared__ uint32_t s_start[CELLS];
+  __shared__ uint32_t s_hoff[CELLS];
   const int bx = xcd_block();
-  const bool second = bx >= ja.g.nblk;
-  const OrderJob &J = second ? jb : ja;
-  const int b = second ? bx - ja.g.nblk : bx;
+  const bool second = TWO && bx >= jobs.j[0].g.nblk;
+  const OrderJob &J = jobs.j[second ? 1 : 0];
+  const int b = second ? bx - jobs.j[0].g.nblk : bx;
   const int tid = threadIdx.x, lane = __lane_id(), wid = tid >> 6;
-  const int c = b * SCAN_BLOCK + tid;
+  OrderBlock ob{b * CELLS, CELLS, 0u, 0u, 0u};
+  if constexpr (BATCH) ob = blocks[b];
   const int cap = J.g.cap, n_c = J.g.n_c;
+  // this lane's cells c0 .. c0 + CPT - 1, those below c_end
+  const int c0 = ob.cell0 + tid * CPT, c_end = BATCH ? ob.cell0 + ob.n_cells : n_c;
   // type-ordered work list of this grid (workgroup-uniform)
   const bool typed = J.work != nullptr;
   // The ordering's first loads go out before the per-bead terms below, so
-  // that their latency overlaps that work: this cell's count and the totals
+  // that their latency overlaps that work: this lane's counts and the totals
   // of the workgroups before this one (four per lane at once; with the work
   // list also their het totals).
   constexpr int PRE = 4;
-  const uint32_t cnt = (c < n_c) ? J.count[c] : 0u;
+  uint32_t cnt[CPT];
+#pragma unroll
+  for (int u = 0; u < CPT; ++u) cnt[u] = c0 + u < c_end ? J.count[c0 + u] : 0u;
+  bool empty = false;
+  if constexpr (BATCH) empty = J.bs_read[b] == 0u;
   uint32_t pv[PRE], hv[PRE];
 #pragma unroll
   for (int u = 0; u < PRE; ++u) {
-    const int k = tid + u * SCAN_BLOCK;
+    const int k = (int)ob.blk0 + tid + u * SCAN_BLOCK;
     pv[u] = k < b ? J.bs_read[k] : 0u;
     hv[u] = typed && k < b ? J.hbs_read[k] : 0u;
   }
@@ -1539,7 +1571,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_order(OrderJob ja, OrderJob jb, 
   }
   uint32_t part = (pv[0] + pv[1]) + (pv[2] + pv[3]);
   uint32_t hpart = (hv[0] + hv[1]) + (hv[2] + hv[3]);
-  for (int k0 = tid + PRE * SCAN_BLOCK; k0 < b; k0 += PRE * SCAN_BLOCK) {
+  for (int k0 = (int)ob.blk0 + tid + PRE * SCAN_BLOCK; k0 < b; k0 += PRE * SCAN_BLOCK) {
 #pragma unroll
     for (int u = 0; u < PRE; ++u) {
       const int k = k0 + u * SCAN_BLOCK;
@@ -1555,69 +1587,106 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_order(OrderJob ja, OrderJob jb, 
     hpart = wave_sum(hpart);
     if (lane == 0) hred[wid] = hpart;
   }
-  uint32_t m = cnt;
-  if (m > (uint32_t)cap) {
-    atomicAdd(flags + FLAG_OVERFLOW, 1u);
-    m = (uint32_t)cap;
-  }
-  // the cell's first entries, loaded together now so that their latency
-  // overlaps the scans and the barrier below
-  const float4 *bk = J.bucket + (size_t)c * cap;
-  constexpr uint32_t EARLY = 4;
-  float4 ev[EARLY];
-#pragma unroll
-  for (uint32_t k = 0; k < EARLY; ++k)
-    if (k < m) ev[k] = bk[k];
-  const uint32_t incl = wave_incl_scan(cnt);
-  const uint32_t mincl = wave_incl_scan(m);
-  if (lane == 63) {
-    wsum[wid] = incl;
-    msum[wid] = mincl;
-  }
-  // het members of this cell (the work list places them before the others)
-  uint32_t hc = 0, hincl = 0;
-  if (typed) {
-#pragma unroll
-    for (uint32_t k = 0; k < EARLY; ++k)
-      if (k < m) hc += (wbits(ev[k]) & W_HET) ? 1u : 0u;
-    for (uint32_t k = EARLY; k < m; ++k) hc += (wbits(bk[k]) & W_HET) ? 1u : 0u;
-    hincl = wave_incl_scan(hc);
-    if (lane == 63) hsum[wid] = hincl;
-  }
-  __syncthreads();
-  uint32_t prefix = 0, woff = 0, moff = 0, mtotal = 0, hprefix = 0, hoff = 0;
-#pragma unroll
-  for (int k = 0; k < SCAN_BLOCK / 64; ++k) {
-    prefix += red[k];
-    mtotal += msum[k];
-    if (k < wid) {
-      woff += wsum[k];
-      moff += msum[k];
-    }
-  }
-  if (typed) {
-#pragma unroll
-    for (int k = 0; k < SCAN_BLOCK / 64; ++k) {
-      hprefix += hred[k];
-      if (k < wid) hoff += hsum[k];
-    }
-    // het slots before this cell's: those of the blocks before and of the
-    // cells before it in this block
-    hoff += hprefix + hincl - hc;
-  }
-  const uint32_t start = prefix + woff + incl - cnt;
-  moff += mincl - m;
-  if (c < n_c) {
-    J.cstart[c] = start;
-    J.count[c] = 0u;
-  }
-  if (c == n_c - 1) J.cstart[n_c] = start + cnt;
   if (tid == 0) {
     J.bs_clear[b] = 0u;
     // the grid's het totals are cleared by every ordering of its buffers
     // (those with no work list too), so that the next binning finds them zero
     if (J.hbs_clear) J.hbs_clear[b] = 0u;
     if (b == 0 && !second && step_inc) *step_inc += 1ull;
+  }
+  if constexpr (BATCH) {
+    if (empty) { // (workgroup-uniform; the counts are zero already)
+      __syncthreads();
+      uint32_t prefix = ob.slot0;
+#pragma unroll
+      for (int k = 0; k < SCAN_BLOCK / 64; ++k) prefix += red[k];
+#pragma unroll
+      for (int u = 0; u < CPT; ++u) {
+        if (c0 + u < c_end) J.cstart[c0 + u] = prefix;
+        if (c0 + u == n_c - 1) J.cstart[n_c] = prefix;
+      }
+      return;
+    }
+  }
+  uint32_t m[CPT], cnt_all = 0, m_all = 0;
+#pragma unroll
+  for (int u = 0; u < CPT; ++u) {
+    m[u] = cnt[u];
+    if (m[u] > (uint32_t)cap) {
+      atomicAdd(flags + FLAG_OVERFLOW, 1u);
+      m[u] = (uint32_t)cap;
+    }
+    cnt_all += cnt[u];
+    m_all += m[u];
+  }
+  // the cells' first entries, loaded together now so that their latency
+  // overlaps the scans and the barrier below
+  const float4 *bk = J.bucket + (size_t)c0 * cap;
+  constexpr uint32_t EARLY = CPT == 1 ? 4 : 2;
+  float4 ev[CPT][EARLY];
+#pragma unroll
+  for (int u = 0; u < CPT; ++u)
+#pragma unroll
+    for (uint32_t k = 0; k < EARLY; ++k)
+      if (k < m[u]) ev[u][k] = bk[u * cap + k];
+  const uint32_t incl = wave_incl_scan(cnt_all);
+  const uint32_t mincl = wave_incl_scan(m_all);
+  if (lane == 63) {
+    wsum[wid] = incl;
+    msum[wid] = mincl;
+  }
+  // het members of these cells (the work list places them before the others)
+  uint32_t hc[CPT] = {}, hincl = 0, hc_all = 0;
+  if (typed) {
+#pragma unroll
+    for (int u = 0; u < CPT; ++u) {
+#pragma unroll
+      for (uint32_t k = 0; k < EARLY; ++k)
+        if (k < m[u]) hc[u] += (wbits(ev[u][k]) & W_HET) ? 1u : 0u;
+      for (uint32_t k = EARLY; k < m[u]; ++k) hc[u] += (wbits(bk[u * cap + k]) & W_HET) ? 1u : 0u;
+      hc_all += hc[u];
+    }
+    hincl = wave_incl_scan(hc_all);
+    if (lane == 63) hsum[wid] = hincl;
+  }
+  __syncthreads();
+  uint32_t prefix = ob.slot0, woff = 0, mbase = 0, mtotal = 0, hprefix = ob.het0, hbase = 0;
+#pragma unroll
+  for (int k = 0; k < SCAN_BLOCK / 64; ++k) {
+    prefix += red[k];
+    mtotal += msum[k];
+    if (k < wid) {
+      woff += wsum[k];
+      mbase += msum[k];
+    }
+  }
+  if (typed) {
+#pragma unroll
+    for (int k = 0; k < SCAN_BLOCK / 64; ++k) {
+      hprefix += hred[k];
+      if (k < wid) hbase += hsum[k];
+    }
+    // het slots before this lane's cells: those of the blocks before and of
+    // the cells before them in this block
+    hbase += hprefix + hincl - hc_all;
+  }
+  uint32_t start[CPT], moff[CPT], hoff[CPT];
+  start[0] = prefix + woff + incl - cnt_all;
+  moff[0] = mbase + mincl - m_all;
+  hoff[0] = hbase;
+#pragma unroll
+  for (int u = 1; u < CPT; ++u) {
+    start[u] = start[u - 1] + cnt[u - 1];
+    moff[u] = moff[u - 1] + m[u - 1];
+    hoff[u] = hoff[u - 1] + hc[u - 1];
+  }
+#pragma unroll
+  for (int u = 0; u < CPT; ++u) {
+    if (c0 + u < c_end) {
+      J.cstart[c0 + u] = start[u];
+      J.count[c0 + u] = 0u;
+    }
+    if (c0 + u == n_c - 1) J.cstart[n_c] = start[u] + cnt[u];
   }
   // work-list entry of the member at slot dst, with hbefore het members in
   // the slots before it: het members in slot order, then the others
@@ -1626,19 +1695,23 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_order(OrderJob ja, OrderJob jb, 
     if (k < J.n_slots) J.work[k] = dst;
   };
   if (mtotal <= (uint32_t)ORDER_LDS) {
-    s_loff[tid] = moff;
-    s_start[tid] = start;
-    s_hoff[tid] = hoff;
-    if (tid == SCAN_BLOCK - 1) s_loff[SCAN_BLOCK] = moff + m;
-    auto put = [&](uint32_t k, float4 v) {
-      s_pos[moff + k] = v;
-      s_id[moff + k] = __float_as_uint(v.w) & ID_MASK;
-      s_cell[moff + k] = (uint8_t)tid;
-    };
 #pragma unroll
-    for (uint32_t k = 0; k < EARLY; ++k)
-      if (k < m) put(k, ev[k]);
-    for (uint32_t k = EARLY; k < m; ++k) put(k, bk[k]);
+    for (int u = 0; u < CPT; ++u) {
+      const int l = tid * CPT + u;
+      s_loff[l] = moff[u];
+      s_start[l] = start[u];
+      s_hoff[l] = hoff[u];
+      if (l == CELLS - 1) s_loff[CELLS] = moff[u] + m[u];
+      auto put = [&](uint32_t k, float4 v) {
+        s_pos[moff[u] + k] = v;
+        s_id[moff[u] + k] = __float_as_uint(v.w) & ID_MASK;
+        s_cell[moff[u] + k] = (std::remove_reference_t<decltype(s_cell[0])>)l;
+      };
+#pragma unroll
+      for (uint32_t k = 0; k < EARLY; ++k)
+        if (k < m[u]) put(k, ev[u][k]);
+      for (uint32_t k = EARLY; k < m[u]; ++k) put(k, bk[u * cap + k]);
+    }
     __syncthreads();
     for (uint32_t e = tid; e < mtotal; e += SCAN_BLOCK) {
       const uint32_t l = s_cell[e], id = s_id[e];
@@ -1661,30 +1734,33 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_order(OrderJob ja, OrderJob jb, 
     }
   } else {
     // dense block (raw initial walks): rank each cell's entries in place
-    for (uint32_t k = 0; k < m; ++k) {
-      const float4 v = bk[k];
-      const uint32_t e = __float_as_uint(v.w) & ID_MASK;
-      uint32_t rank = 0, hr = 0;
-      for (uint32_t s2 = 0; s2 < m; ++s2) {
-        const float4 o = bk[s2];
-        const bool before = (__float_as_uint(o.w) & ID_MASK) < e;
-        rank += before ? 1u : 0u;
-        hr += (before && (wbits(o) & W_HET)) ? 1u : 0u;
+    for (int u = 0; u < CPT; ++u)
+      for (uint32_t k = 0; k < m[u]; ++k) {
+        const float4 v = bk[u * cap + k];
+        const uint32_t e = __float_as_uint(v.w) & ID_MASK;
+        uint32_t rank = 0, hr = 0;
+        for (uint32_t s2 = 0; s2 < m[u]; ++s2) {
+          const float4 o = bk[u * cap + s2];
+          const bool before = (__float_as_uint(o.w) & ID_MASK) < e;
+          rank += before ? 1u : 0u;
+          hr += (before && (wbits(o) & W_HET)) ? 1u : 0u;
+        }
+        J.spos[start[u] + rank] = v;
+        if (J.soi) J.soi[start[u] + rank] = e;
+        if (typed) put_work(start[u] + rank, hoff[u] + hr, (wbits(v) & W_HET) != 0u);
       }
-      J.spos[start + rank] = v;
-      if (J.soi) J.soi[start + rank] = e;
-      if (typed) put_work(start + rank, hoff + hr, (wbits(v) & W_HET) != 0u);
-    }
   }
   // A cell with more members than its bucket holds (flagged above; the host
   // then grows the buckets and rebuilds) keeps its full slot range: the slots
   // past the stored members get a sentinel that every reader skips (index
   // ID_MASK, far outside any grid) instead of stale memory.
-  for (uint32_t k = m; k < cnt; ++k) {
-    J.spos[start + k] = make_float4(1e18f, 1e18f, 1e18f, __uint_as_float(ID_MASK));
-    if (J.soi) J.soi[start + k] = ID_MASK;
-    if (typed) put_work(start + k, hoff + hc, false);
-  }
+#pragma unroll
+  for (int u = 0; u < CPT; ++u)
+    for (uint32_t k = m[u]; k < cnt[u]; ++k) {
+      J.spos[start[u] + k] = make_float4(1e18f, 1e18f, 1e18f, __uint_as_float(ID_MASK));
+      if (J.soi) J.soi[start[u] + k] = ID_MASK;
+      if (typed) put_work(start[u] + k, hoff[u] + hc[u], false);
+    }
 }
 
 // The same terms on their own, before the first stage of a run.
@@ -2170,8 +2246,7 @@ void launch_bin(hipStream_t s, const KParams &p, const GridGeom &g, int n_obj, c
 }
 
 void launch_order(hipStream_t s, const OrderJob &a, const OrderJob *b, uint32_t *flags, uint64_t *step_inc,
-                  const NoiseJob *noise, const KParams *bp, const BondJob *bond) {
-  const OrderJob jb = b ? *b : a;
+                  const NoiseJob *noise, const KParams *bp, const BondJob *bond, OrderTable table) {
   const unsigned blocks = (unsigned)(a.g.nblk + (b ? b->g.nblk : 0));
   NoiseJob nj{};
   KParams p{};
@@ -2181,7 +2256,15 @@ void launch_order(hipStream_t s, const OrderJob &a, const OrderJob *b, uint32_t 
     p = *bp;
     bj = *bond;
   }
-  k_order<<<blocks, SCAN_BLOCK, 0, s>>>(a, jb, flags, step_inc, nj, p, bj);
+  const OrderJobs<1> one{{a}};
+  if (b)
+    k_order<false, 1, true><<<blocks, SCAN_BLOCK, 0, s>>>(OrderJobs<2>{{a, *b}}, nullptr, flags, step_inc, nj, p, bj);
+  else if (!table.blocks)
+    k_order<false, 1, false><<<blocks, SCAN_BLOCK, 0, s>>>(one, nullptr, flags, step_inc, nj, p, bj);
+  else if (table.cells_per_lane == 2)
+    k_order<true, 2, false><<<blocks, SCAN_BLOCK, 0, s>>>(one, table.blocks, flags, step_inc, nj, p, bj);
+  else
+    k_order<true, 1, false><<<blocks, SCAN_BLOCK, 0, s>>>(one, table.blocks, flags, step_inc, nj, p, bj);
 }
 
 __global__ __launch_bounds__(64) void k_signal(const uint32_t *flags, uint32_t *host, uint32_t seq) {

@@ -20,7 +20,7 @@ constexpr uint32_t W_HET = 1u << 31; // the sign bit: a het partner is a negativ
 
 // cells per scan block of the order kernel; each block reads the totals of
 // the blocks before it, so fewer, larger blocks keep that prefix cheap
-constexpr int SCAN_BLOCK = 256;
+constexpr int SCAN_BLOCK = 256, SCAN_SHIFT = 8;
 // threads per block of the bead kernels
 constexpr int BEAD_BLOCK = 256;
 
@@ -32,11 +32,14 @@ enum Mode : int { MODE_CCP = 0, MODE_ICG = 1, MODE_LJ = 2 };
 // Geometry of one uniform cell grid centred on the nucleus (ccp's sugrid,
 // sugrid.cuh:15-54): cell (gx, gy, gz) = floor(r / csl) + cps/2, index
 // coff + gx + cps (gy + cps gz). coff places the grid of one system inside
-// the concatenated cell range of a batch (0 for a single system).
+// the concatenated cell range of a batch, boff its scan blocks inside the
+// batch's (both 0 for a single system).
 struct GridGeom {
   float csl;
   float icsl; // 1/csl for the cell lookup of the step grids; 0: divide by csl (ccp's rule, export grid)
   int cps, half, n_c, cap, nblk, coff;
+  int boff;   // first scan block of the grid: its cells are counted in blocks of their own (0 for a single system)
+  int bshift; // log2 of the cells of a scan block
 };
 
 // Per-system parameters of a batch of independent systems that share one
@@ -130,6 +133,22 @@ struct KPtrs {
   int n_sys;
 };
 
+// One scan block of a batch: its cells [cell0, cell0 + n_cells), all of one
+// system, that system's first block, and the slots and het members of the
+// systems before it.
+struct OrderBlock {
+  int cell0, n_cells;
+  uint32_t blk0, slot0, het0;
+};
+
+// The scan blocks of a batch's ordering (nblk of them, each of SCAN_BLOCK
+// times cells_per_lane cells, 1 or 2); no blocks: block b of a single system
+// holds the cells from b SCAN_BLOCK on.
+struct OrderTable {
+  const OrderBlock *blocks = nullptr;
+  int cells_per_lane = 1;
+};
+
 // One grid's ordering work inside a k_order launch.
 struct OrderJob {
   GridGeom g;
@@ -206,7 +225,8 @@ void launch_bin(hipStream_t s, const KParams &p, const GridGeom &g, int n_obj, c
 // The order pass also fills the next force pass's per-bead terms when given:
 // normals (noise) and bonded + wall forces (bp, bond).
 void launch_order(hipStream_t s, const OrderJob &a, const OrderJob *b, uint32_t *flags, uint64_t *step_inc,
-                  const NoiseJob *noise = nullptr, const KParams *bp = nullptr, const BondJob *bond = nullptr);
+                  const NoiseJob *noise = nullptr, const KParams *bp = nullptr, const BondJob *bond = nullptr,
+                  OrderTable table = {});
 // the same per-bead terms on their own (before the first stage of a run)
 void launch_bead_terms(hipStream_t s, const NoiseJob *noise, const KParams &p, const BondJob *bond);
 // Copy the FLAG_COUNT error flags into host[1..] and then seq into host[0]
