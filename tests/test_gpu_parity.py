@@ -350,3 +350,30 @@ def test_single_chain_16384_steps():
     assert np.allclose(sc, want_sc, rtol=1e-9, atol=1e-9), (sc, want_sc)
     assert np.allclose(rcd, want_rcd, rtol=1e-9, atol=1e-10)
     sim.close()
+
+
+@pytest.mark.parametrize("N,cvf", [(1, 0.05), (3, 0.1), (65, 0.39), (700, 0.002), (5000, 0.3)])
+def test_default_shape_of_ccp_field(N, cvf):
+    # ccp's force field with no shape key: eight lanes over ~1.2 sigma cells,
+    # or the wide cells where the nucleus holds few beads. Forces and overlap
+    # counts (up to the 2 sigma the wide cells allowed) against the oracle,
+    # and the same grid extent as ccp's cells for the outside-the-grid error
+    step(f"default shape N={N} cvf={cvf}")
+    R_n = max(radius_for(N, cvf), 3.0)
+    r = relaxed(N, R_n, seed=N) if N > 3 else np.array([[0.1, 0.2, -0.3], [1.0, 0.4, -0.2], [1.5, 1.2, 0.4]])[:N]
+    fl = pattern(N, N)
+    sim, osys, r64 = make_pair(N, R_n, fl, r)
+    f, want = sim.compute_forces().astype(np.float64), osys.forces(r64)
+    err32 = np.abs(osys.forces(r64, prec=32) - want).max()
+    assert np.abs(f - want).max() <= 3 * err32 + 1e-6 * max(np.abs(want).max(), 1.0)
+    d = np.linalg.norm(r64[:, None] - r64[None], axis=2) if N <= 700 else None
+    for dmin in (0.9, 1.21, 1.95):
+        n = sim.count_overlaps(dmin)
+        if d is not None:
+            i, j = np.triu_indices(N, 2)
+            assert n == int((d[i, j].astype(np.float32) < np.float32(dmin)).sum()), dmin
+    with pytest.raises(tfm_amd.CcpError, match="dmin must be in"):
+        sim.count_overlaps(2.001)
+    info = sim.info
+    assert abs(info.fine_cps / 2 * info.fine_csl - info.cps / 2 * info.csl) < 1e-4
+    sim.close()

@@ -348,7 +348,7 @@ struct ccp_batch {
       KParams k = kp;
       k.N = (int)S.n;
       k.gf = S.g;
-      launch_overlaps(stream, k, grid.spos.p, grid.cstart.p, S.slot, MIS * MIS, dover.p + s);
+      launch_overlaps(stream, k, grid.spos.p, grid.cstart.p, S.slot, MIS, dover.p + s);
     }
     hip_check(hipGetLastError());
     std::vector<unsigned long long> h(n_sys);

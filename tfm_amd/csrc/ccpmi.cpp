@@ -114,9 +114,9 @@ void ccp_sim::configure(const ParMap &par) {
   uint32_t cap_f = par.get<uint32_t>("fine_cell_capacity", 16u);
   if (!(1 <= cap && cap <= 1024)) throw Error(CCP_ERR_PARAM, "cell_capacity out of range");
   if (!(1 <= cap_f && cap_f <= 1024)) throw Error(CCP_ERR_PARAM, "fine_cell_capacity out of range");
-  auto geometry = [&](float side, uint32_t capacity) {
+  auto geometry = [&](float side, uint32_t capacity, float extent) {
     GridGeom g{};
-    uint32_t cps = 2 * (uint32_t)std::ceil(d_m / side);
+    uint32_t cps = 2 * (uint32_t)std::ceil(extent / side);
     if (cps < 4) cps = 4;
     if ((uint64_t)cps * cps * cps >= (1ull << 31)) throw Error(CCP_ERR_PARAM, "cell_size too small for the nucleus");
     g.csl = side;
@@ -129,14 +129,44 @@ void ccp_sim::configure(const ParMap &par) {
     g.bshift = SCAN_SHIFT;
     return g;
   };
-  gh.g = geometry(csl, cap);
+  gh.g = geometry(csl, cap, d_m);
   gx.g = gh.g;
   gx.g.icsl = 0.0f; // the exported cell list divides by csl as ccp does
-  gf.g = geometry(csl_f, split ? cap_f : cap);
+  dmin_max = csl_f;
+  float extent = d_m;
+  lanes = par.get<uint32_t>("lanes_per_bead", 2 * reach + 1);
+  // ccp's force field with no key that bears on the kernels' shape: the step
+  // runs eight lanes per bead over cells just wider than the short cutoff
+  // (1.1547 sigma; the 2 sigma one spans two of them), with the type-ordered work
+  // list. 128 to 2560 steps, us per step against three lanes over 2 sigma
+  // cells: N = 256 25.7 (39.1), 1024 28.1 (44.1), 4096 29.2 (45.1), 16384
+  // 32.4 (44.4), 30386 35.3 (52.3), 32768 at volume fraction 0.25 35.1 (58.1).
+  // Eight lanes over the 2 sigma cells lie between, and above both in the
+  // dense nucleus (64). The order pass pays per cell, so nuclei with few
+  // beads for their size (below a volume fraction of 0.03 or so) keep the
+  // wide cells, and with them the memory of their buckets.
+  if (!lj && !split) {
+    bool plain = true;
+    for (const char *k : {"lanes_per_bead", "cell_reach", "cell_size", "fine_cell_size", "cell_capacity",
+                          "integrate_pass", "group_types", "bal_rounds", "type_order"})
+      plain = plain && !par.has(k);
+    // the same extent as the wide cells' grid (a bead beyond it is an error),
+    // in a whole number of cells
+    extent = gh.g.half * csl;
+    const double n = std::floor((double)extent / STEP_CSL_CCP);
+    if (plain && 8.0 * n * n * n <= 32.0 * N + 32768.0) {
+      csl_f = (float)(extent / n);
+      extent = csl_f * ((float)n - 0.5f); // (n cells, whatever the quotient's rounding)
+      reach = 2;
+      lanes = 8;
+    } else {
+      extent = d_m;
+    }
+  }
+  gf.g = geometry(csl_f, split ? cap_f : cap, extent);
   lg = gf.g;
   fcap = par.get<float>("force_cap", lj ? 0.2f / dt : 0.0f);
   if (!(fcap >= 0.0f)) throw Error(CCP_ERR_PARAM, "force_cap out of range");
-  lanes = par.get<uint32_t>("lanes_per_bead", 2 * reach + 1);
   if (lanes != 1 && lanes != 2 * reach + 1 && lanes != 8) throw Error(CCP_ERR_PARAM, "lanes_per_bead out of range");
   // the balanced kernel scans one grid: the split pair sum has no 8-lane form
   if (lanes == 8 && split) throw Error(CCP_ERR_PARAM, "lanes_per_bead 8 excludes fine_cell_size");
@@ -777,7 +807,7 @@ void ccp_sim::set_particle_positions(HostRng &g) {
 uint64_t ccp_sim::count_overlaps(float dmin) {
   ensure_grids();
   hip_check(hipMemsetAsync(dcount.p, 0, sizeof(unsigned long long), stream));
-  launch_overlaps(stream, kp, gf.spos.p, gf.cstart.p, 0u, dmin * dmin, dcount.p);
+  launch_overlaps(stream, kp, gf.spos.p, gf.cstart.p, 0u, dmin, dcount.p);
   unsigned long long c = 0;
   hip_check(hipMemcpyAsync(&c, dcount.p, sizeof(c), hipMemcpyDeviceToHost, stream));
   hip_check(hipStreamSynchronize(stream));
@@ -1340,7 +1370,7 @@ int ccp_noise(ccp_sim *h, uint64_t step, float *z_xyz, uint32_t *attempts, size_
 int ccp_count_overlaps(ccp_sim *h, float dmin, uint64_t *count) {
   return guarded(h, [&] {
     need(count != nullptr, "null count");
-    need(dmin > 0.0f && dmin <= h->gf.g.csl, "dmin must be in (0, fine_cell_size]");
+    need(dmin > 0.0f && dmin <= h->dmin_max, "dmin must be in (0, fine_cell_size]");
     *count = h->count_overlaps(dmin);
   });
 }

@@ -223,30 +223,6 @@ __device__ __forceinline__ void bin_bead(const KParams &p, const KPtrs &q, uint3
   if (!(isfinite(x) && isfinite(y) && isfinite(z))) atomicAdd(q.flags + FLAG_NONFINITE, 1u);
 }
 
-// Slot ranges of the 9 neighbour rows (x-1..x+1 of rows y+dy, z+dz) of the
-// cell holding (x, y, z); rows outside the grid get an empty range. All 18
-// start lookups are issued together.
-struct Rows {
-  uint32_t lo[9], hi[9];
-  int c0[9], c1[9];
-};
-
-__device__ __forceinline__ void neighbour_rows(const GridGeom &g, const uint32_t *__restrict__ cstart, float x,
-                                               float y, float z, Rows &R) {
-  bool outside = false;
-  const int cx = cell_coord(x, g, outside), cy = cell_coord(y, g, outside), cz = cell_coord(z, g, outside);
-#pragma unroll
-  for (int r = 0; r < 9; ++r) {
-    const int zz = cz + r / 3 - 1, yy = cy + r % 3 - 1;
-    const bool ok = zz >= 0 && zz < g.cps && yy >= 0 && yy < g.cps;
-    const int row = g.coff + (zz * g.cps + yy) * g.cps;
-    R.c0[r] = ok ? row + max(cx - 1, 0) : 0;
-    R.c1[r] = ok ? row + min(cx + 1, g.cps - 1) + 1 : 0;
-    R.lo[r] = cstart[R.c0[r]];
-    R.hi[r] = cstart[R.c1[r]];
-  }
-}
-
 // ---------------------------------------------------------------- forces
 // Short-range pair force on bead i from entry o (every pair type), with
 // |i - j| <= 1 skipped (calc_cell_srf, chrsim.cu:250).
@@ -1834,23 +1810,30 @@ __global__ __launch_bounds__(BEAD_BLOCK) void k_contacts_batch(const SysParams *
                 (S.n + bins - 1) / bins, maps + (size_t)s * bins * bins);
 }
 
-// Non-bonded pairs (|i - j| > 1) closer than dmin <= fine cell side
-// (particle_overlaps, chrsim.cu:805-820), each pair counted once.
+// Non-bonded pairs (|i - j| > 1) closer than dmin (particle_overlaps,
+// chrsim.cu:805-820) on the step grid, rad = ceil(dmin / csl) cells to each
+// side, each pair counted once.
 __global__ __launch_bounds__(BEAD_BLOCK) void k_overlaps(KParams p, const float4 *spos, const uint32_t *cstart,
-                                                         uint32_t slot0, float dmin2, unsigned long long *count) {
+                                                         uint32_t slot0, float dmin2, int rad,
+                                                         unsigned long long *count) {
   const int t = blockIdx.x * BEAD_BLOCK + threadIdx.x;
   uint32_t n = 0;
   if (t < p.N) {
     const float4 me = spos[slot0 + t];
     const uint32_t i = wbits(me) & ID_MASK;
-    Rows R;
-    neighbour_rows(p.gf, cstart, me.x, me.y, me.z, R);
-    for (int r = 0; r < 9; ++r)
-      for (uint32_t k = R.lo[r]; k < R.hi[r]; ++k) {
-        const float4 o = spos[k];
-        const uint32_t j = wbits(o) & ID_MASK;
-        const float dx = me.x - o.x, dy = me.y - o.y, dz = me.z - o.z;
-        if (j > i + 1u && dist2(dx, dy, dz) < dmin2) ++n;
+    const GridGeom &g = p.gf;
+    bool outside = false;
+    const int cx = cell_coord(me.x, g, outside), cy = cell_coord(me.y, g, outside), cz = cell_coord(me.z, g, outside);
+    for (int dz = max(-rad, -cz); dz <= min(rad, g.cps - 1 - cz); ++dz)
+      for (int dy = max(-rad, -cy); dy <= min(rad, g.cps - 1 - cy); ++dy) {
+        const int row = g.coff + ((cz + dz) * g.cps + cy + dy) * g.cps;
+        const uint32_t lo = cstart[row + max(cx - rad, 0)], hi = cstart[row + min(cx + rad, g.cps - 1) + 1];
+        for (uint32_t k = lo; k < hi; ++k) {
+          const float4 o = spos[k];
+          const uint32_t j = wbits(o) & ID_MASK;
+          const float dx = me.x - o.x, dy2 = me.y - o.y, dz2 = me.z - o.z;
+          if (j > i + 1u && dist2(dx, dy2, dz2) < dmin2) ++n;
+        }
       }
   }
   const uint32_t tot = wave_sum(n);
@@ -2409,9 +2392,10 @@ void launch_contacts(hipStream_t s, const KParams &p, const float4 *spos, const 
 }
 
 void launch_overlaps(hipStream_t s, const KParams &p, const float4 *spos, const uint32_t *cstart, uint32_t slot0,
-                     float dmin2, unsigned long long *count) {
+                     float dmin, unsigned long long *count) {
   if (p.N <= 0) return;
-  k_overlaps<<<blocks_for(p.N, BEAD_BLOCK), BEAD_BLOCK, 0, s>>>(p, spos, cstart, slot0, dmin2, count);
+  const int rad = (int)ceilf(dmin / p.gf.csl);
+  k_overlaps<<<blocks_for(p.N, BEAD_BLOCK), BEAD_BLOCK, 0, s>>>(p, spos, cstart, slot0, dmin * dmin, rad, count);
 }
 
 void launch_noise(hipStream_t s, const KParams &p, uint64_t step, float4 *out) {

@@ -244,7 +244,7 @@ void launch_contacts(hipStream_t s, const KParams &p, const float4 *spos, const 
                      uint32_t slot0 = 0, uint32_t id0 = 0);
 // slots [slot0, slot0 + p.N) of spos, pairs counted on p.gf
 void launch_overlaps(hipStream_t s, const KParams &p, const float4 *spos, const uint32_t *cstart, uint32_t slot0,
-                     float dmin2, unsigned long long *count);
+                     float dmin, unsigned long long *count);
 void launch_noise(hipStream_t s, const KParams &p, uint64_t step, float4 *out);
 void launch_observables(hipStream_t s, int N, double R_n, double nod, double a, int n_b, const float4 *pos,
                         double *out);

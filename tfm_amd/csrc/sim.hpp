@@ -85,6 +85,11 @@ using namespace ccpmi;
 using namespace ccpmi::host;
 
 
+// least cell side of the step grid of ccp's force field (when the caller picks
+// no kernel shape): above the short cutoff rco = 1.154701 plus the 1e-3 of the
+// list radii, at least half the long one
+constexpr float STEP_CSL_CCP = 1.2f;
+
 // ---------------------------------------------------------------- handle
 struct ccp_sim {
   // parameters
@@ -100,6 +105,7 @@ struct ccp_sim {
   int ff = CCP_FF_CCP;
   float csl = 0;   // coarse cell side: het grid and ccp-layout export grid
   float csl_f = 0; // cell side of the all-bead grid of the step (fine when split)
+  float dmin_max = 0; // largest overlap distance: fine_cell_size (cell_size when not split)
   bool split = false; // short-range pairs on the fine grid + het-het tail on the het grid
   std::vector<uint32_t> chain_off;
   std::string seq_file;
