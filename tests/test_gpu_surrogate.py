@@ -85,6 +85,35 @@ def test_forward_and_gradients_match_oracle():
         assert err < 2e-2, k
 
 
+@pytest.mark.parametrize("c", [dict(c_in=3, width=36, n_layers=2, d=5, L=13, rd_bins=7, B=5),
+                               dict(c_in=5, width=100, n_layers=3, d=33, L=50, rd_bins=33, B=3),
+                               dict(c_in=17, width=65, n_layers=1, d=16, L=40, rd_bins=1, B=1),
+                               dict(c_in=1, width=256, n_layers=2, d=64, L=129, rd_bins=32, B=2)])
+def test_ragged_sizes_match_oracle(c):
+    # channels, positions, samples and heads off every tile size: outputs and
+    # every gradient against the oracle, with the tolerances above
+    step(f"surrogate sizes {c}")
+    rng = np.random.default_rng(c["width"])
+    p = so.init_params(c["c_in"], c["width"], c["n_layers"], c["d"], c["L"], c["rd_bins"], seed=1)
+    for k in p:
+        p[k] = (p[k] + 0.05 * rng.normal(size=p[k].shape)).astype(np.float32).astype(np.float64)
+    x = rng.normal(size=(c["c_in"], c["B"] * c["L"])).astype(np.float32).astype(np.float64)
+    T = rng.normal(size=(c["B"], c["L"], c["L"])).astype(np.float32)
+    T = (0.5 * (T + T.transpose(0, 2, 1))).astype(np.float64)
+    T_rd = rng.normal(size=(c["rd_bins"], c["B"])).astype(np.float32).astype(np.float64)
+    net = sg.Surrogate(params=p, **c)
+    dev = lambda a: torch.tensor(np.asarray(a, np.float32), device="cuda")
+    S0, rd0 = (t.clone() for t in net.predict(dev(x)))
+    net.zero_grad()
+    loss = net.loss_backward(dev(x), dev(T), dev(T_rd), w_pair=1.0, w_rd=0.5)
+    want_loss, g, S, rd = so.loss_and_grads(p, x, T, T_rd, c["B"], c["L"], c["n_layers"], 1.0, 0.5, round_bf16=True)
+    assert torch.equal(S0, net.S) and torch.equal(rd0, net.rd)
+    assert rel(net.S.cpu().numpy(), S) < 1e-3 and rel(net.rd.cpu().numpy(), rd) < 1e-3
+    assert float(loss.item()) == pytest.approx(want_loss, rel=1e-3)
+    for k in p:
+        assert rel(net.g[k].cpu().numpy(), g[k]) < 2e-2, k
+
+
 def test_training_reduces_loss():
     step("surrogate training")
     c, p, x, T, T_rd = problem(3)

@@ -25,7 +25,25 @@ from .ccp import lib
 NN_EXPORTS = (
     "ccp_nn_gemm", "ccp_nn_im2col", "ccp_nn_col2im", "ccp_nn_bias_gelu", "ccp_nn_gelu_back", "ccp_nn_pair_map",
     "ccp_nn_pair_loss", "ccp_nn_mean_pool", "ccp_nn_pool_back", "ccp_nn_rd_loss", "ccp_nn_cast_bf16", "ccp_nn_adamw",
+    "ccp_nn_input", "ccp_nn_fwd", "ccp_nn_pair", "ccp_nn_pool", "ccp_nn_small", "ccp_nn_pair_bands", "ccp_nn_pair_grad",
+    "ccp_nn_rd_grad", "ccp_nn_duv", "ccp_nn_back", "ccp_nn_wgrad_tiles", "ccp_nn_wgrad", "ccp_nn_reduce", "ccp_nn_pack",
+    "ccp_nn_adamw_flat",
 )
+
+
+def _struct(name, pointers, ints=(), longs=()):
+    return type(name, (ctypes.Structure,), {"_fields_": [(k, ctypes.c_void_p) for k in pointers] +
+                                            [(k, ctypes.c_long) for k in longs] + [(k, ctypes.c_int) for k in ints]})
+
+
+FwdArgs = _struct("FwdArgs", ("A0", "A1", "X", "bias", "res", "pre", "y", "ob", "ot"),
+                  ("M", "M0", "Kp", "Cs", "P", "Ps", "L", "Os", "O1"))
+BackArgs = _struct("BackArgs", ("W", "G", "dpooled", "pre", "dh", "gb", "gt", "dbias"),
+                   ("C", "Cs", "Cr", "Kr", "Gs", "P", "Ps", "L", "B", "V1", "keep"))
+Segment = _struct("Segment", ("src", "dst"), (), ("n", "stride", "parts"))
+WgradJob = _struct("WgradJob", ("G", "X", "dst0", "dst1"), ("M", "M0", "C", "taps", "P", "Ps"))
+Weight = _struct("Weight", ("w", "wb", "fwd", "back"), ("M", "C", "taps", "Kp", "Cr", "Kr"))
+
 
 _bound = False
 
@@ -47,12 +65,32 @@ def _nn():
         L.ccp_nn_rd_loss.argtypes = [vp, vp, vp, vp, vp, vp, vp, i, i, f, vp]
         L.ccp_nn_cast_bf16.argtypes = [vp, vp, lg, vp]
         L.ccp_nn_adamw.argtypes = [vp, vp, vp, vp, vp, lg, f, f, f, f, f, i, vp]
+        L.ccp_nn_input.argtypes = [vp, vp, vp, i, i, i, i, vp, vp]
+        L.ccp_nn_fwd.argtypes = [vp, i, vp]
+        L.ccp_nn_pair.argtypes = [vp, i, vp, vp, vp, i, i, f, vp]
+        L.ccp_nn_pool.argtypes = [vp, vp, vp, i, i, i, i, i, i, vp]
+        L.ccp_nn_small.argtypes = [vp, vp, vp, i, i, i, i, i, i, vp]
+        L.ccp_nn_pair_bands.argtypes = [i]
+        L.ccp_nn_pair_grad.argtypes = [vp, vp, vp, vp, vp, vp, i, i, i, f, vp]
+        L.ccp_nn_rd_grad.argtypes = [vp, vp, vp, vp, vp, vp, vp, i, i, i, i, f, vp]
+        L.ccp_nn_duv.argtypes = [vp, vp, vp, vp, i, i, i, i, i, i, f, vp]
+        L.ccp_nn_back.argtypes = [vp, i, vp]
+        L.ccp_nn_wgrad_tiles.argtypes = [i, i]
+        L.ccp_nn_wgrad.argtypes = [vp, vp, i, i, i, vp]
+        L.ccp_nn_reduce.argtypes = [vp, i, vp]
+        L.ccp_nn_pack.argtypes = [vp, i, vp]
+        L.ccp_nn_adamw_flat.argtypes = [vp, vp, vp, vp, lg, lg, f, f, f, f, f, i, vp]
         _bound = True
     return L
 
 
 def _p(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+
+
+def _a(t):
+    """Device address of a tensor (None for none), for a structure's field."""
+    return t.data_ptr() if t is not None else None
 
 
 def _stream():
@@ -75,9 +113,23 @@ def bf16_like(t):
     return torch.empty(t.shape, dtype=torch.int16, device=t.device)
 
 
+def _up(n, k):
+    return (n + k - 1) // k * k
+
+
+def _table(structs):
+    """The structures as one device array (read by the kernels that take a table)."""
+    raw = b"".join(bytes(t) for t in structs)
+    return torch.frombuffer(bytearray(raw), dtype=torch.uint8).cuda()
+
+
 class Surrogate:
     """Weights (FP32 masters, BF16 copies) and buffers for batches of B
-    sequences of L bins with c_in input channels."""
+    sequences of L bins with c_in input channels.
+
+    The parameters, their gradients and AdamW's moments are views of one flat
+    array each, the weight matrices first (they alone decay). include/ccpmi_nn.h
+    gives the layouts of the activations."""
 
     def __init__(self, c_in=5, width=256, n_layers=6, d=64, L=128, rd_bins=32, B=64, seed=0, params=None):
         self.c_in, self.width, self.n_layers, self.d, self.L, self.rd_bins, self.B = \
@@ -96,47 +148,122 @@ class Surrogate:
             params["dist"] = np.zeros(L)
             params["c0"] = np.zeros(1)
         self.names = list(params.keys())
-        self.p = {k: torch.tensor(np.asarray(v, np.float32), device=dev).contiguous() for k, v in params.items()}
+        host = {k: np.ascontiguousarray(v, np.float32) for k, v in params.items()}
+        order = [k for k in self.names if k.startswith("W")] + [k for k in self.names if not k.startswith("W")]
+        at, off = 0, {}
+        for k in order:
+            off[k] = at
+            at += _up(host[k].size, 64)
+            if k.startswith("W"):
+                self._n_decay = at
+        self._flat = [torch.zeros(at, dtype=torch.float32, device=dev) for _ in range(4)]
+        view = lambda t: {k: t[off[k]:off[k] + host[k].size].view(host[k].shape) for k in self.names}
+        self.p, self.g, self.m, self.v = (view(t) for t in self._flat)
+        for k in self.names:
+            self.p[k].copy_(torch.from_numpy(host[k]))
         self.pb = {k: bf16_like(v) for k, v in self.p.items() if k.startswith("W")}
-        self.g = {k: torch.zeros_like(v) for k, v in self.p.items()}
-        self.m = {k: torch.zeros_like(v) for k, v in self.p.items()}
-        self.v = {k: torch.zeros_like(v) for k, v in self.p.items()}
         self.t = 0
+        self._pack_tables()
         self._cast_weights()
         self._alloc(B)
+
+    def _pack_tables(self):
+        """The packed weight copies and the table that fills them."""
+        W, C1, d = self.width, self.c_in, self.d
+        h = lambda *s: torch.zeros(s, dtype=torch.int16, device="cuda")
+        Cr, Kr, Kd = _up(W, 64), _up(W, 32), _up(d, 32)
+        self._wf = {1: h(Cr, 3 * _up(C1, 16))}
+        self._wt = {}
+        for k in range(2, self.n_layers + 1):
+            self._wf[k], self._wt[k] = h(Cr, 3 * _up(W, 16)), h(3, Cr, Kr)
+        self._wf["u"], self._wf["v"] = h(d, _up(W, 64)), h(d, _up(W, 64))
+        self._wt["uv"] = h(2, Cr, Kd)
+        tab = []
+        for k in range(1, self.n_layers + 1):
+            C, wt = (C1, None) if k == 1 else (W, self._wt[k])
+            tab.append(Weight(_a(self.p[f"W{k}"]), _a(self.pb[f"W{k}"]), _a(self._wf[k]), _a(wt), W, C, 3,
+                              3 * _up(C, 16), Cr, Kr))
+        for j, k in enumerate("uv"):
+            tab.append(Weight(_a(self.p["W" + k]), _a(self.pb["W" + k]), _a(self._wf[k]), _a(self._wt["uv"][j]), d, W,
+                              1, _up(W, 64), Cr, Kd))
+        O = self.rd_bins
+        self._wf["r"], self._wt["r"] = h(O, _up(W, 64)), h(Cr, _up(O, 32))
+        tab.append(Weight(_a(self.p["Wr"]), _a(self.pb["Wr"]), _a(self._wf["r"]), _a(self._wt["r"]), O, W, 1,
+                          _up(W, 64), Cr, _up(O, 32)))
+        self._pack = _table(tab), len(tab)
 
     def _alloc(self, B):
         self.B = B
         dev = torch.device("cuda")
-        P, W, L = B * self.L, self.width, self.L
+        W, L, d, n = self.width, self.L, self.d, self.n_layers
+        Ls, Cs, C1s, ds = _up(L, 8), _up(W, 64), _up(self.c_in, 16), _up(d, 32)
+        P = B * L
+        Ps = _up(P, 16)
+        self._ls, self._ds, self._ps = Ls, ds, Ps
         f = lambda *s: torch.zeros(s, dtype=torch.float32, device=dev)
         h = lambda *s: torch.zeros(s, dtype=torch.int16, device=dev)
-        self.xb = h(self.c_in, P)
-        self.cols = {1: h(3 * self.c_in, P)}
-        for k in range(2, self.n_layers + 1):
-            self.cols[k] = h(3 * W, P)
-        self.pre = {k: f(W, P) for k in range(1, self.n_layers + 1)}
-        self.hs = {k: f(W, P) for k in range(1, self.n_layers + 1)}
-        self.hb = {k: h(W, P) for k in range(1, self.n_layers + 1)}
-        self.Ub, self.Vb = h(self.d, P), h(self.d, P)
-        self.raw = f(B, L, L)
+        # forward; pre and the channel rows are read by the backward pass only
+        self.xb, self.xt = h(self.c_in, Ps), h(P, C1s)
+        self.hs = [f(W, Ps), f(W, Ps)]
+        self.ht = [h(P, Cs), h(P, Cs)]
+        self.pre = {k: f(W, Ps) for k in range(1, n + 1)}
+        self.hb = {k: h(W, Ps) for k in range(1, n + 1)}
+        self.uvb, self.uvt = h(2 * d, Ps), h(P, 2 * ds)
         self.S = f(B, L, L)
-        self.pooled, self.pooledb = f(W, B), h(W, B)
+        Bs, Or = _up(B, 16), _up(self.rd_bins, 32)
+        self._bs, self._or, self._cs = Bs, Or, Cs
+        self.pooledb, self.pooledt = h(W, Bs), h(B, Cs)
         self.rd = f(self.rd_bins, B)
-        # backward
-        self.gS, self.graw, self.grawb = f(B, L, L), f(B, L, L), h(B, L, L)
-        self.dU, self.dUb, self.dV, self.dVb = f(self.d, P), h(self.d, P), f(self.d, P), h(self.d, P)
-        self.dh = f(W, P)
-        self.gp, self.gpb = f(W, P), h(W, P)
-        self.dcols = f(3 * W, P)
-        self.grd, self.grdb = f(self.rd_bins, B), h(self.rd_bins, B)
+        self._fwd = {}
+        for keep in (False, True):
+            for k in range(1, n + 1):
+                first = k == 1
+                self._fwd[keep, k] = FwdArgs(
+                    _a(self._wf[k]), None, _a(self.xt if first else self.ht[k % 2]), _a(self.p[f"b{k}"]),
+                    None if first else _a(self.hs[k % 2]), _a(self.pre[k]) if keep else None,
+                    _a(self.hs[(k + 1) % 2]), _a(self.hb[k]) if keep else None, _a(self.ht[(k + 1) % 2]),
+                    W, W, 3 * _up(self.c_in if first else W, 16), C1s if first else Cs, P, Ps, L, Cs, 0)
+            self._fwd[keep, "uv"] = FwdArgs(
+                _a(self._wf["u"]), _a(self._wf["v"]), _a(self.ht[(n + 1) % 2]), None, None, None, None,
+                _a(self.uvb) if keep else None, _a(self.uvt), 2 * d, d, _up(W, 64), Cs, P, Ps, L, 2 * ds, ds)
+        # backward: every layer keeps its gradient's channel rows for the weight gradients' one launch
+        bands, tiles = _nn().ccp_nn_pair_bands(L), (P + 127) // 128
+        self.grawb = h(B, L, Ls)
+        self.duvb, self.duvt = h(2 * d, Ps), h(P, 2 * ds)
+        self.dh = f(W, Ps)
+        self.gb = {k: h(W, Ps) for k in range(1, n + 1)}
+        self.gt = [h(P, Cs), h(P, Cs)]
+        self.grdb, self.grdt = h(self.rd_bins, Bs), h(B, Or)
         self.dpooled = f(W, B)
         self.loss = f(1)
+        self._gdist, self._gc0 = f(B * bands, L), f(B * bands)
+        self._dbias = {k: f(tiles, W) for k in range(1, n + 1)}
+        Cr = _up(W, 64)
+        self._back = {n: BackArgs(_a(self._wt["uv"]), _a(self.duvt), _a(self.dpooled), _a(self.pre[n]), _a(self.dh),
+                                  _a(self.gb[n]), _a(self.gt[n % 2]), _a(self._dbias[n]), W, Cs, Cr, _up(d, 32),
+                                  2 * ds, P, Ps, L, B, ds, int(n > 1))}
+        for k in range(n - 1, 0, -1):
+            self._back[k] = BackArgs(_a(self._wt[k + 1]), _a(self.gt[(k + 1) % 2]), None, _a(self.pre[k]), _a(self.dh),
+                                     _a(self.gb[k]), _a(self.gt[k % 2]), _a(self._dbias[k]), W, Cs, Cr, _up(W, 32),
+                                     Cs, P, Ps, L, B, 0, int(k > 1))
+        jobs, at = [], [0]
+        for k in list(range(1, n + 1)):
+            X, C = (self.xb, self.c_in) if k == 1 else (self.hb[k - 1], W)
+            jobs.append(WgradJob(_a(self.gb[k]), _a(X), _a(self.g[f"W{k}"]), None, W, W, C, 3, P, Ps))
+        jobs.append(WgradJob(_a(self.duvb), _a(self.hb[n]), _a(self.g["Wu"]), _a(self.g["Wv"]), 2 * d, d, W, 1,
+                             P, Ps))
+        jobs.append(WgradJob(_a(self.grdb), _a(self.pooledb), _a(self.g["Wr"]), None, self.rd_bins, self.rd_bins, W, 1,
+                             B, Bs))
+        for j in jobs:
+            at.append(at[-1] + _nn().ccp_nn_wgrad_tiles(j.M, j.C))
+        self._jobs = _table(jobs), torch.tensor(at, dtype=torch.int32, device=dev), len(jobs), at[-1]
+        seg = [Segment(_a(self._dbias[k]), _a(self.g[f"b{k}"]), W, W, tiles) for k in range(1, n + 1)]
+        seg.append(Segment(_a(self._gdist), _a(self.g["dist"]), L, L, B * bands))
+        seg.append(Segment(_a(self._gc0), _a(self.g["c0"]), 1, 1, B * bands))
+        self._seg = _table(seg), len(seg)
 
     def _cast_weights(self):
-        L = _nn()
-        for k, t in self.pb.items():
-            _ok(L.ccp_nn_cast_bf16(_p(self.p[k]), _p(t), t.numel(), _stream()), "cast")
+        _ok(_nn().ccp_nn_pack(_p(self._pack[0]), self._pack[1], _stream()), "pack")
 
     # ------------------------------------------------------------ forward
     @staticmethod
@@ -144,91 +271,67 @@ class Surrogate:
         if t.dtype != torch.float32 or not t.is_cuda or not t.is_contiguous() or tuple(t.shape) != tuple(shape):
             raise ValueError(f"{name} must be a contiguous float32 cuda tensor of shape {tuple(shape)}")
 
-    def forward(self, x):
-        """x: [c_in, B L] float32 (cuda). Returns (S [B, L, L], rd [rd_bins, B]) on the device."""
+    def forward(self, x, keep=True):
+        """x: [c_in, B L] float32 (cuda). Returns (S [B, L, L], rd [rd_bins, B]) on the device.
+        keep: also store what loss_backward reads."""
         self._check_input(x, (self.c_in, self.B * self.L), "x")
         N = _nn()
         B, L, W, d = self.B, self.L, self.width, self.d
-        P = B * L
         s = _stream()
-        _ok(N.ccp_nn_cast_bf16(_p(x), _p(self.xb), x.numel(), s), "cast")
-        inp_b, inp_f, c_in = self.xb, None, self.c_in
+        _ok(N.ccp_nn_input(_p(x), _p(self.xb) if keep else None, _p(self.xt), self.c_in, _up(self.c_in, 16), B * L,
+                           self._ps, _p(self.loss) if keep else None, s), "input")
         for k in range(1, self.n_layers + 1):
-            _ok(N.ccp_nn_im2col(_p(inp_b), _p(self.cols[k]), c_in, B, L, s), "im2col")
-            K = 3 * c_in
-            gemm(self.pb[f"W{k}"], self.cols[k], W, P, K, (0, K, 1), (0, P, 1), (0, P, 1), C=self.pre[k])
-            _ok(N.ccp_nn_bias_gelu(_p(self.pre[k]), _p(self.p[f"b{k}"]), _p(inp_f), _p(self.hs[k]),
-                                   _p(self.hb[k]), W, P, s), "bias_gelu")
-            inp_b, inp_f, c_in = self.hb[k], self.hs[k], W
-        hb, hf = inp_b, inp_f
-        gemm(self.pb["Wu"], hb, d, P, W, (0, W, 1), (0, P, 1), (0, P, 1), Cb=self.Ub)
-        gemm(self.pb["Wv"], hb, d, P, W, (0, W, 1), (0, P, 1), (0, P, 1), Cb=self.Vb)
-        # raw[b](i, j) = sum_c U[c, b L + i] V[c, b L + j] / sqrt(d)
-        gemm(self.Ub, self.Vb, L, L, d, (L, 1, P), (L, P, 1), (L * L, L, 1), C=self.raw, batch=B,
-             alpha=1.0 / math.sqrt(d))
-        _ok(N.ccp_nn_pair_map(_p(self.raw), _p(self.p["dist"]), _p(self.p["c0"]), _p(self.S), L, B, s), "pair_map")
-        _ok(N.ccp_nn_mean_pool(_p(hf), _p(self.pooled), _p(self.pooledb), W, B, L, s), "pool")
-        gemm(self.pb["Wr"], self.pooledb, self.rd_bins, B, W, (0, W, 1), (0, B, 1), (0, B, 1), C=self.rd)
+            _ok(N.ccp_nn_fwd(ctypes.byref(self._fwd[keep, k]), 1, s), "conv")
+        _ok(N.ccp_nn_fwd(ctypes.byref(self._fwd[keep, "uv"]), 0, s), "heads")
+        # S from raw[b](i, j) = sum_c U[c, b, i] V[c, b, j] / sqrt(d)
+        _ok(N.ccp_nn_pair(_p(self.uvt), self._ds, _p(self.p["dist"]), _p(self.p["c0"]), _p(self.S), L, B,
+                          1.0 / math.sqrt(d), s), "pair")
+        _ok(N.ccp_nn_pool(_p(self.hs[(self.n_layers + 1) % 2]), _p(self.pooledb), _p(self.pooledt), W, B, L, self._ps,
+                          self._bs, self._cs, s), "pool")
+        _ok(N.ccp_nn_small(_p(self._wf["r"]), _p(self.pooledt), _p(self.rd), self.rd_bins, B, self._cs, self._cs,
+                           self._cs, B, s), "radial head")
         return self.S, self.rd
 
     def predict(self, x):
-        S, rd = self.forward(x)
+        S, rd = self.forward(x, keep=False)
         rd = rd + self.p["br"][:, None]
         return S, rd
 
     # ------------------------------------------------------------ backward
     def zero_grad(self):
-        for t in self.g.values():
-            t.zero_()
+        self._flat[1].zero_()
 
     def loss_backward(self, x, T, T_rd, w_pair=1.0, w_rd=1.0):
         """Forward, loss and gradients into self.g; returns the loss (device scalar)."""
         N = _nn()
-        B, L, W, d = self.B, self.L, self.width, self.d
-        P = B * L
+        B, L, W, d, n = self.B, self.L, self.width, self.d, self.n_layers
+        Ls, Ps = self._ls, self._ps
         s = _stream()
         self._check_input(T, (B, L, L), "T")
         self._check_input(T_rd, (self.rd_bins, B), "T_rd")
         self.forward(x)
-        self.loss.zero_()
-        _ok(N.ccp_nn_pair_loss(_p(self.S), _p(T), _p(self.gS), _p(self.graw), _p(self.grawb), _p(self.g["dist"]),
-                               _p(self.g["c0"]), _p(self.loss), L, B, w_pair, s), "pair_loss")
-        _ok(N.ccp_nn_rd_loss(_p(self.rd), _p(self.p["br"]), _p(T_rd), _p(self.grd), _p(self.grdb), _p(self.g["br"]),
-                             _p(self.loss), self.rd_bins, B, w_rd, s), "rd_loss")
-        a = 1.0 / math.sqrt(d)
+        _ok(N.ccp_nn_pair_grad(_p(self.S), _p(T), _p(self.grawb), _p(self._gdist), _p(self._gc0), _p(self.loss), L, Ls,
+                               B, w_pair, s), "pair_grad")
+        _ok(N.ccp_nn_rd_grad(_p(self.rd), _p(self.p["br"]), _p(T_rd), _p(self.grdb), _p(self.grdt), _p(self.g["br"]),
+                             _p(self.loss), self.rd_bins, B, self._bs, self._or, w_rd, s), "rd_grad")
+        _ok(N.ccp_nn_small(_p(self._wt["r"]), _p(self.grdt), _p(self.dpooled), W, B, self._or, self._or, self._or, B,
+                           s), "pooled gradient")
         # dU_b = a V_b graw_b^T, dV_b = a U_b graw_b
-        gemm(self.Vb, self.grawb, d, L, L, (L, P, 1), (L * L, 1, L), (L, P, 1), C=self.dU, Cb=self.dUb, batch=B,
-             alpha=a)
-        gemm(self.Ub, self.grawb, d, L, L, (L, P, 1), (L * L, L, 1), (L, P, 1), C=self.dV, Cb=self.dVb, batch=B,
-             alpha=a)
-        hb, hf = self.hb[self.n_layers], self.hs[self.n_layers]
-        gemm(self.dUb, hb, d, W, P, (0, P, 1), (0, 1, P), (0, W, 1), C=self.g["Wu"], beta=1.0)
-        gemm(self.dVb, hb, d, W, P, (0, P, 1), (0, 1, P), (0, W, 1), C=self.g["Wv"], beta=1.0)
-        gemm(self.pb["Wu"], self.dUb, W, P, d, (0, 1, W), (0, P, 1), (0, P, 1), C=self.dh)
-        gemm(self.pb["Wv"], self.dVb, W, P, d, (0, 1, W), (0, P, 1), (0, P, 1), C=self.dh, beta=1.0)
-        # radial head
-        gemm(self.grdb, self.pooledb, self.rd_bins, W, B, (0, B, 1), (0, 1, B), (0, W, 1), C=self.g["Wr"], beta=1.0)
-        gemm(self.pb["Wr"], self.grdb, W, B, self.rd_bins, (0, 1, W), (0, B, 1), (0, B, 1), C=self.dpooled)
-        _ok(N.ccp_nn_pool_back(_p(self.dpooled), _p(self.dh), W, B, L, s), "pool_back")
-        for k in range(self.n_layers, 0, -1):
-            _ok(N.ccp_nn_gelu_back(_p(self.pre[k]), _p(self.dh), _p(self.gp), _p(self.gpb), _p(self.g[f"b{k}"]), W,
-                                   P, s), "gelu_back")
-            c_in = self.c_in if k == 1 else W
-            K = 3 * c_in
-            gemm(self.gpb, self.cols[k], W, K, P, (0, P, 1), (0, 1, P), (0, K, 1), C=self.g[f"W{k}"], beta=1.0)
-            if k > 1:
-                gemm(self.pb[f"W{k}"], self.gpb, K, P, W, (0, 1, K), (0, P, 1), (0, P, 1), C=self.dcols)
-                _ok(N.ccp_nn_col2im(_p(self.dcols), _p(self.dh), W, B, L, 1.0, s), "col2im")
+        _ok(N.ccp_nn_duv(_p(self.uvb), _p(self.grawb), _p(self.duvb), _p(self.duvt), d, self._ds, L, Ls, B, Ps,
+                         1.0 / math.sqrt(d), s), "duv")
+        for k in range(n, 0, -1):
+            _ok(N.ccp_nn_back(ctypes.byref(self._back[k]), int(k == n), s), "back")
+        _ok(N.ccp_nn_wgrad(_p(self._jobs[0]), _p(self._jobs[1]), self._jobs[2], self._jobs[3], L, s),
+            "wgrad")
+        _ok(N.ccp_nn_reduce(_p(self._seg[0]), self._seg[1], s), "reduce")
         return self.loss
 
     def step(self, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8, wd=1e-4):
-        N = _nn()
         self.t += 1
-        s = _stream()
-        for k in self.names:
-            decay = wd if k.startswith("W") else 0.0
-            _ok(N.ccp_nn_adamw(_p(self.p[k]), _p(self.g[k]), _p(self.m[k]), _p(self.v[k]), _p(self.pb.get(k)),
-                               self.p[k].numel(), lr, b1, b2, eps, decay, self.t, s), "adamw")
+        p, g, m, v = (_p(t) for t in self._flat)
+        _ok(_nn().ccp_nn_adamw_flat(p, g, m, v, self._flat[0].numel(), self._n_decay, lr, b1, b2, eps, wd, self.t,
+                                    _stream()), "adamw")
+        self._cast_weights()
 
     def state_dict(self):
         return {k: v.detach().cpu().numpy() for k, v in self.p.items()}
