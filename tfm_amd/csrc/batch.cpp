@@ -574,7 +574,12 @@ ccp_batch *ccp_batch_create(const char *common_params, const ccp_batch_system *s
     if (b->bond_pass()) b->fbond.alloc(b->N);
     if (b->kp.lanes == 8 && b->integrate_pass) b->fpair.alloc(b->N);
     b->dsys.alloc(n_sys);
-    b->dslot.alloc(n_sys + 1);
+    std::vector<uint32_t> slots = b->slot;
+    for (uint32_t t = 0, s = 0; t < b->N; t += SYS_SLOTS) {
+      while (b->slot[s + 1] <= t) ++s;
+      slots.push_back(s);
+    }
+    b->dslot.alloc(slots.size());
     b->flags.alloc(FLAG_COUNT);
     b->cmaps.alloc((size_t)n_sys * b->bins * b->bins);
     b->dstep.alloc(1);
@@ -582,7 +587,7 @@ ccp_batch *ccp_batch_create(const char *common_params, const ccp_batch_system *s
     b->obs.alloc((6 + 3 * (size_t)b->rd_bins) * n_sys);
     b->grid.alloc(b->N, b->kp.typed != 0);
     hip_check(hipMemcpy(b->dsys.p, b->sys.data(), n_sys * sizeof(SysParams), hipMemcpyHostToDevice));
-    hip_check(hipMemcpy(b->dslot.p, b->slot.data(), (n_sys + 1) * sizeof(uint32_t), hipMemcpyHostToDevice));
+    hip_check(hipMemcpy(b->dslot.p, slots.data(), slots.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
     hip_check(hipMemset(b->flags.p, 0, FLAG_COUNT * sizeof(uint32_t)));
     hip_check(hipMemset(b->cmaps.p, 0, (size_t)n_sys * b->bins * b->bins * sizeof(uint32_t)));
     hip_check(hipMemset(b->dstep.p, 0, sizeof(uint64_t)));

@@ -634,15 +634,14 @@ template <int LANES> struct Lanes {
   static constexpr int BEADS_PER_BLOCK = BEADS_PER_WAVE * (BEAD_BLOCK / 64);
 };
 
-// System of cell-ordered slot t in a batch: the last s with sys_slot[s] <= t.
+// System of slot or bead t in a batch, the last s with sys_slot[s] <= t: from
+// the system of the first of t's 64 slots (the table behind the n_sys + 1
+// starts) on. Two dependent loads where a search of 256 systems took eight,
+// ahead of every other load of a force wavefront.
 __device__ __forceinline__ int system_of(const uint32_t *__restrict__ sys_slot, int n_sys, uint32_t t) {
-  int lo = 0, hi = n_sys - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (sys_slot[mid] <= t) lo = mid;
-    else hi = mid - 1;
-  }
-  return lo;
+  int s = (int)sys_slot[n_sys + 1 + (int)(t / SYS_SLOTS)];
+  while (s + 1 < n_sys && sys_slot[s + 1] <= t) ++s;
+  return s;
 }
 
 // Constants of the batch system holding slot t.

@@ -55,6 +55,9 @@ struct SysParams {
   int frozen; // initial-condition relaxation done: zero force, the beads keep their positions
 };
 
+// slots per entry of the systems' table behind their first slots
+constexpr uint32_t SYS_SLOTS = 64;
+
 // Device buffers of one grid. count/blocksum/bucket receive the binning of
 // the next positions; cstart/spos/soi hold the ordered cell list.
 struct GridBufs {
@@ -129,7 +132,7 @@ struct KPtrs {
   const uint32_t *work;    // type-ordered work list of the fine grid (k_force_typed)
   // batches only (sys == nullptr for a single system)
   const SysParams *sys;    // n_sys systems
-  const uint32_t *sys_slot; // n_sys + 1 first slots
+  const uint32_t *sys_slot; // n_sys + 1 first slots, then the system of every SYS_SLOTS-th slot
   int n_sys;
 };
 
