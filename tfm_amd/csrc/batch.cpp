@@ -284,14 +284,17 @@ struct ccp_batch {
     q.sys = dsys.p;
     q.sys_slot = dslot.p;
     q.n_sys = (int)n_sys;
-    launch_force(stream, mode, stage, k, q);
-    const OrderJob j = grid.order_job((uint32_t)kp.n_het, N);
-    // with the order pass: the next step's normals after the first stage,
-    // the bonded terms of q.out0 after both
+    // the next step's normals: in the tail of the second stage's type-ordered
+    // force launch, else with the order pass after the first stage (as ccp_sim)
     const NoiseJob nj = noise_job(1);
+    const bool typed = grid.work.p != nullptr;
+    const bool drew = launch_force(stream, mode, stage, k, q, typed && stage == 2 ? &nj : nullptr);
+    if (typed && stage == 2 && !drew) throw Error(CCP_ERR_STATE, "type-ordered force launch without its normals");
+    const OrderJob j = grid.order_job((uint32_t)kp.n_het, N);
+    // with the order pass: the bonded terms of q.out0 after both stages
     const BondJob bj = bond_job(q.out0, mode);
-    launch_order(stream, j, nullptr, flags.p, stage == 2 ? dstep.p : nullptr, stage == 1 ? &nj : nullptr, &k,
-                 bond_pass() ? &bj : nullptr, grid.table());
+    launch_order(stream, j, nullptr, flags.p, stage == 2 ? dstep.p : nullptr, stage == 1 && !typed ? &nj : nullptr,
+                 &k, bond_pass() ? &bj : nullptr, grid.table());
     grid.clean ^= 1;
   }
   void run_chunk(uint64_t n) {
