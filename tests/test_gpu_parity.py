@@ -352,6 +352,31 @@ def test_single_chain_16384_steps():
     sim.close()
 
 
+@pytest.mark.parametrize("N,bs,shape", [
+    (4, 1, dict(contact_cutoff=1.2)), (33, 2, dict(contact_cutoff=0.7)), (1003, 7, dict(contact_cutoff=2.5)),
+    (4099, 4099, dict(contact_cutoff=1.5)), (4099, 5, dict(contact_cutoff=2.0, fine_cell_size=1.2)),
+    (4099, 1, dict(contact_cutoff=3.0, cell_size=3.5)),
+    (2051, 3, dict(contact_cutoff=2.4, cell_size=1.25, cell_reach=2, lanes_per_bead=8))])
+def test_contacts_over_reaches(N, bs, shape):
+    # eight lanes over the rows of one, two or three cells to each side: bins
+    # of one bead up to one bin for all, dense enough for rows of several
+    # rounds of loads; whole numbers, equal to the oracle's over all pairs
+    step(f"contacts N={N} {shape}")
+    R_n = max(radius_for(N, 0.3), 3.0)
+    sim = tfm_amd.Simulation({"number_of_particles": N, "nucleus_radius": repr(float(R_n)), "seed": 4,
+                              "number_of_lbs": 0, "force_field": "lj", "contact_bin_size": bs, **shape})
+    r = np.ascontiguousarray(walk(N, R_n, N + 3), np.float32)
+    sim.flags = np.zeros(N, np.uint8)
+    sim.positions = r
+    nb = sim.info.contact_bins
+    sim.contact_reset()
+    sim.contact_sample()
+    m, ns = sim.contact_map()
+    assert ns == 1
+    assert np.array_equal(m, po.contacts(r, np.float32(shape["contact_cutoff"]), bs, nb))
+    sim.close()
+
+
 @pytest.mark.parametrize("N,cvf", [(1, 0.05), (3, 0.1), (65, 0.39), (700, 0.002), (5000, 0.3)])
 def test_default_shape_of_ccp_field(N, cvf):
     # ccp's force field with no shape key: eight lanes over ~1.2 sigma cells,
