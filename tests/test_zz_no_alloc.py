@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 import torch  # before the library: torch's HIP runtime must be the one loaded first
 
+import pyoracle as po
 import tfm_amd
 from gpu_common import step
 from helpers import radius_for, walk
@@ -69,3 +70,19 @@ def test_noalloc_calls_in_a_row_and_limits():
                                  ctypes.cast(dummy, u32p), ctypes.cast(dummy, u32p), None)
     assert rc == tfm_amd.CCP_ERR_ARG
     assert "at most 255" in L.ccp_last_error(None).decode()
+
+
+@pytest.mark.parametrize("N,cps", [(1, 1), (50, 1), (257, 6), (5003, 7), (9001, 63), (9001, 64), (9001, 65), (777, 255)])
+def test_noalloc_block_edges_match_oracle(N, cps):
+    # one block of 256 cells, ragged last blocks, 1024 block sums (added up by
+    # every block) and more (scanned first): the same words as the oracle's
+    step(f"allocation-free cell list N={N} cps={cps}")
+    rng = np.random.default_rng(N + cps)
+    csl = np.float32(1.25)
+    half = cps // 2
+    r = ((rng.random((N, 3)) * cps * 0.999 - half) * csl).astype(np.float32)
+    want = po.cell_list(r, csl, cps)
+    assert not want["bad"]
+    got = noalloc_cell_list(r, csl, cps)
+    for k in ("sci", "soi", "beg", "end"):
+        assert np.array_equal(got[k], want[k]), k

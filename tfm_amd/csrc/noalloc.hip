@@ -13,15 +13,21 @@
 // bit the arrays ccp_cell_list returns for the same positions and geometry.
 //
 // Method (a counting sort that keeps its state in the output arrays):
-//   1. end[c] = 0 (a fill kernel, no memset), flag = 0
+//   1. end[c] = 0 (a fill kernel, no memset), scratch words and flag = 0
 //   2. key of bead i (ccp's floor(r / csl) + cps/2, clamped into the grid;
 //      a bead outside raises the flag) into sci[i], end[key] += 1
-//   3. exclusive scan of the counts: per-256-cell block sums in `scratch`,
-//      one block scans them, then each block's cells get beg[c] = start and
-//      end[c] = start (the scatter cursor)
+//   3. exclusive scan of the counts: a block of 256 cells publishes its sum in
+//      `scratch` and adds up those of the blocks before it (beyond NA_DIRECT
+//      blocks: sums, their scan and the starts as three kernels), then its
+//      cells get beg[c] = start and end[c] = start (the scatter cursor)
 //   4. soi[atomicAdd(end[key], 1)] = i (arbitrary order within a cell)
 //   5. one lane per cell sorts its slots by bead index (the stable order),
 //      writes sci[s] = c over them and sets empty cells to 0/0.
+// What bounds it is launches and their chains of loads, not bytes: at 100003
+// beads over 2 sigma cells the call takes 57 us with five launches, 69 with
+// seven (block sums and their scan as kernels of their own). Block sums added
+// up by atomics in step 2 cost more than both: neighbouring words of a few
+// cache lines, 98 us for that kernel.
 // Calls on one GPU share its scratch array: calls that overlap in time on
 // one GPU race and must not be issued.
 
@@ -37,6 +43,7 @@ constexpr int NA_BLOCK = 256;
 constexpr uint32_t NA_MAX_CELLS = 1u << 24; // cps <= 255
 constexpr uint32_t NA_MAX_BLOCKS = NA_MAX_CELLS / NA_BLOCK;
 constexpr uint32_t NA_FLAG = NA_MAX_BLOCKS; // word of the outside flag
+constexpr uint32_t NA_TICKET = NA_FLAG + 1; // blocks of the scan that have started
 constexpr uint32_t NA_WORDS = NA_MAX_BLOCKS + 64;
 constexpr int NA_MAX_DEVICES = 64;
 
@@ -46,7 +53,8 @@ static __device__ __align__(256) uint32_t scratch[NA_WORDS];
 __global__ __launch_bounds__(NA_BLOCK) void k_na_clear(uint32_t n_c, uint32_t *end, uint32_t *sc) {
   const uint32_t c = blockIdx.x * NA_BLOCK + threadIdx.x;
   if (c < n_c) end[c] = 0u;
-  if (c == 0) sc[NA_FLAG] = 0u;
+  if (threadIdx.x == 0) sc[blockIdx.x] = 0u;
+  if (c < 2u) sc[NA_FLAG + c] = 0u;
 }
 
 // ccp's cell coordinate floor(x / csl) + cps/2 (calc_indexes,
@@ -74,27 +82,23 @@ __global__ __launch_bounds__(NA_BLOCK) void k_na_key(const float *xyz, uint32_t 
 
 // exclusive scan of v over the block's 256 lanes, and the block total
 __device__ __forceinline__ uint32_t na_block_scan(uint32_t v, uint32_t &total) {
-  __shared__ uint32_t s[NA_BLOCK];
-  const int t = threadIdx.x;
-  s[t] = v;
-  __syncthreads();
-  for (int d = 1; d < NA_BLOCK; d <<= 1) {
-    const uint32_t a = t >= d ? s[t - d] : 0u;
-    __syncthreads();
-    s[t] += a;
-    __syncthreads();
+  __shared__ uint32_t sums[NA_BLOCK / 64];
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+  uint32_t incl = v;
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t a = __shfl_up(incl, d);
+    if (lane >= d) incl += a;
   }
-  total = s[NA_BLOCK - 1];
-  const uint32_t incl = s[t];
+  if (lane == 63) sums[wave] = incl;
   __syncthreads();
-  return incl - v;
-}
-
-__global__ __launch_bounds__(NA_BLOCK) void k_na_block_sums(const uint32_t *count, uint32_t n_c, uint32_t *sc) {
-  const uint32_t c = blockIdx.x * NA_BLOCK + threadIdx.x;
-  uint32_t total;
-  na_block_scan(c < n_c ? count[c] : 0u, total);
-  if (threadIdx.x == 0) sc[blockIdx.x] = total;
+  uint32_t before = 0;
+  total = 0;
+  for (int w = 0; w < NA_BLOCK / 64; ++w) {
+    before += w < wave ? sums[w] : 0u;
+    total += sums[w];
+  }
+  __syncthreads();
+  return before + incl - v;
 }
 
 // one block: exclusive scan of the nblk block sums in place, each lane
@@ -113,6 +117,13 @@ __global__ __launch_bounds__(NA_BLOCK) void k_na_scan_sums(uint32_t nblk, uint32
   }
 }
 
+__global__ __launch_bounds__(NA_BLOCK) void k_na_block_sums(const uint32_t *count, uint32_t n_c, uint32_t *sc) {
+  const uint32_t c = blockIdx.x * NA_BLOCK + threadIdx.x;
+  uint32_t total;
+  na_block_scan(c < n_c ? count[c] : 0u, total);
+  if (threadIdx.x == 0) sc[blockIdx.x] = total;
+}
+
 __global__ __launch_bounds__(NA_BLOCK) void k_na_starts(uint32_t *count_cursor, uint32_t n_c, const uint32_t *sc,
                                                         uint32_t *beg) {
   const uint32_t c = blockIdx.x * NA_BLOCK + threadIdx.x;
@@ -122,6 +133,35 @@ __global__ __launch_bounds__(NA_BLOCK) void k_na_starts(uint32_t *count_cursor, 
     const uint32_t start = sc[blockIdx.x] + ex;
     beg[c] = start;
     count_cursor[c] = start;
+  }
+}
+
+// The same in one launch for up to NA_DIRECT blocks (four words a lane, less
+// than the two launches it saves). Blocks are numbered in the order in which
+// they start, and each publishes its sum (below 2^31, bit 31 set: sum and flag
+// are one word) before it waits for the blocks before it, so every wait ends.
+constexpr uint32_t NA_DIRECT = 1024;
+__global__ __launch_bounds__(NA_BLOCK) void k_na_starts_direct(uint32_t *count_cursor, uint32_t n_c, uint32_t *sc,
+                                                               uint32_t *beg) {
+  __shared__ uint32_t ticket;
+  if (threadIdx.x == 0) ticket = atomicAdd(sc + NA_TICKET, 1u);
+  __syncthreads();
+  const uint32_t blk = ticket, c = blk * NA_BLOCK + threadIdx.x;
+  uint32_t total, before;
+  const uint32_t ex = na_block_scan(c < n_c ? count_cursor[c] : 0u, total);
+  if (threadIdx.x == 0)
+    __hip_atomic_store(sc + blk, total | 1u << 31, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  uint32_t part = 0;
+  for (uint32_t b = threadIdx.x; b < blk; b += NA_BLOCK) {
+    uint32_t v;
+    do v = __hip_atomic_load(sc + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    while (!(v >> 31));
+    part += v & ~(1u << 31);
+  }
+  na_block_scan(part, before);
+  if (c < n_c) {
+    beg[c] = before + ex;
+    count_cursor[c] = before + ex;
   }
 }
 
@@ -191,9 +231,13 @@ extern "C" int ccp_cell_list_noalloc(const float *xyz, uint32_t n, float csl, ui
     uint32_t *sc = scratch_ptr();
     k_na_clear<<<nblk, NA_BLOCK, 0, s>>>(n_c, end, sc);
     k_na_key<<<na_blocks(n), NA_BLOCK, 0, s>>>(xyz, n, csl, (int)cps, sci, end, sc);
-    k_na_block_sums<<<nblk, NA_BLOCK, 0, s>>>(end, n_c, sc);
-    k_na_scan_sums<<<1, NA_BLOCK, 0, s>>>(nblk, sc);
-    k_na_starts<<<nblk, NA_BLOCK, 0, s>>>(end, n_c, sc, beg);
+    if (nblk <= NA_DIRECT) {
+      k_na_starts_direct<<<nblk, NA_BLOCK, 0, s>>>(end, n_c, sc, beg);
+    } else {
+      k_na_block_sums<<<nblk, NA_BLOCK, 0, s>>>(end, n_c, sc);
+      k_na_scan_sums<<<1, NA_BLOCK, 0, s>>>(nblk, sc);
+      k_na_starts<<<nblk, NA_BLOCK, 0, s>>>(end, n_c, sc, beg);
+    }
     k_na_scatter<<<na_blocks(n), NA_BLOCK, 0, s>>>(sci, n, end, soi);
     k_na_finish<<<nblk, NA_BLOCK, 0, s>>>(n_c, beg, end, soi, sci);
     host::hip_check(hipGetLastError());
