@@ -162,3 +162,16 @@ def test_frame_contact_map_rounded_rows():
         assert np.array_equal(got[ia], (1000 * n / 16).astype(np.float32)), row
     assert moved > 0
     sim.close()
+
+
+@pytest.mark.parametrize("N", [33, 34, 113, 114, 128, 129, 226, 241])
+def test_distance_contact_ragged_tiles(N):
+    # a last separation and a last starting bead on either side of the edges
+    # of tiles of 16 separations x 112 beads
+    step(f"d(s), P(s) N={N}")
+    R_n = radius_for(N, 0.2)
+    sim = sim_with(N, R_n, walk(N, R_n, seed=N), np.zeros(N, np.uint8))
+    sd, cp = sim.distance_contact(0)
+    wsd, wcp = po.sd_cp(sim.positions, 0)
+    assert np.array_equal(sd, wsd) and np.array_equal(cp, wcp)
+    sim.close()

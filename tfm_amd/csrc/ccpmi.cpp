@@ -1436,10 +1436,12 @@ int ccp_distance_contact(ccp_sim *h, uint32_t chromosome, float *sd, float *cp, 
     const SdCpJob job{i_s, i_e, lsdcp, out.p, out.p + lsdcp, nullptr, nullptr};
     launch_sd_cp(h->stream, h->r.p, h->N, &job, 1);
     hip_check(hipGetLastError());
-    hip_check(hipMemcpyAsync(sd, out.p, lsdcp * sizeof(float), hipMemcpyDeviceToHost, h->stream));
-    hip_check(hipMemcpyAsync(cp, out.p + lsdcp, lsdcp * sizeof(float), hipMemcpyDeviceToHost, h->stream));
+    std::vector<float> both(2 * (size_t)lsdcp);
+    hip_check(hipMemcpyAsync(both.data(), out.p, both.size() * sizeof(float), hipMemcpyDeviceToHost, h->stream));
     hip_check(hipStreamSynchronize(h->stream));
     out.free_();
+    std::copy_n(both.data(), lsdcp, sd);
+    std::copy_n(both.data() + lsdcp, lsdcp, cp);
   });
 }
 

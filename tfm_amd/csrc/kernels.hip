@@ -2006,29 +2006,36 @@ __global__ __launch_bounds__(BEAD_BLOCK) void k_radial_batch(const SysParams *sy
 // of one separation is a serial chain of up to 2 (i_e - i_s) additions and
 // only the distances can be computed in any order. One lane doing both waits
 // for its loads on every pair (180 ns a pair, with 18 to 25 wavefronts on the
-// whole chip). Here a workgroup takes 32 separations: seven wavefronts
-// compute the distances of 64 starting beads x 32 separations into LDS while
-// the first one adds the previous tile's in ccp's order, and the positions of
-// the tile after next are on their way. 32 separations, not 64: the distances of a tile (about 30 VALU
-// instructions each, on one CU) then take as long as its additions.
-// N = 30386, six chromosomes of 2284 to 3170 beads, a launch each: 897 -> 76 us
-// (124 us with 64 separations, the distances then the longer part).
-constexpr int SD_S = 32, SD_P = 64, SD_THREADS = 512;
+// whole chip). Here a workgroup takes SD_S separations: seven wavefronts
+// compute the distances of SD_P starting beads x SD_S separations into LDS and
+// count the contacts among them, while the first one adds the previous tile's
+// in ccp's order, and the positions of the tile after next are on their way.
+// Pairs past the chain's end are distances of 0, which change no sum, so that
+// every tile is added the same way, sixteen read while sixteen are added.
+// 8 separations: the distances of a tile (about 30 VALU instructions each, on
+// one CU) then take no longer than its additions; 112 starting beads: two
+// rounds of the seven wavefronts, none of them partly empty.
+// N = 30386, six chromosomes of 2284 to 3170 beads, a launch each: 897 -> 32 us
+// (124 us with 64 separations, 76 with 32 and the counting among the additions).
+constexpr int SD_S = 8, SD_P = 112, SD_THREADS = 512;
 constexpr int SD_WAVES = SD_THREADS / 64 - 1; // wavefronts that compute distances
+static_assert(64 + SD_P + SD_P + SD_S <= SD_THREADS, "a lane per position of a tile");
+static_assert(SD_P % 16 == 0, "the additions take sixteen at a time");
 __global__ __launch_bounds__(SD_THREADS) void k_sd_cp(const float4 *__restrict__ pos, uint32_t N, SdCpJobs jobs) {
 #pragma clang fp contract(off)
   const SdCpJob J = jobs.job[blockIdx.y];
   const uint32_t s0 = 1u + blockIdx.x * SD_S;
   if (s0 > J.lsdcp) return;
   __shared__ float s_d[2][SD_P][SD_S];
-  // the tile's first beads p0 .. p0 + 63, then those s0 .. s0 + SD_P + SD_S - 1 further on
+  // the tile's first beads p0 .. p0 + SD_P - 1, then those s0 .. s0 + SD_P + SD_S - 1 further on
   __shared__ float4 s_pos[2][SD_P + SD_P + SD_S];
+  __shared__ uint32_t s_n[SD_S]; // contacts by separation
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const uint32_t ncc = (N == 30386u) ? 2u : 1u;
   const uint32_t n_p = J.i_e - J.i_s - s0; // starting beads of the shortest separation
   const uint32_t per = (n_p + SD_P - 1u) / SD_P, tiles = ncc * per;
   auto tile_start = [&](uint32_t t) { return J.i_s + (t / per) * (N / ncc) + (t % per) * SD_P; };
-  // positions of tile t, one per lane of the wavefronts 1 to 3 (clamped: a
+  // positions of tile t, one per lane from the second wavefront on (clamped: a
   // value past the chain belongs to pairs that are not added)
   const bool loads = tid >= 64 && tid < 64 + SD_P + SD_P + SD_S;
   const uint32_t slot = (uint32_t)tid - 64u;
@@ -2036,18 +2043,25 @@ __global__ __launch_bounds__(SD_THREADS) void k_sd_cp(const float4 *__restrict__
     const uint32_t p0 = tile_start(t);
     return pos[min(slot < (uint32_t)SD_P ? p0 + slot : p0 + s0 + (slot - SD_P), N - 1u)];
   };
+  const uint32_t s = s0 + (uint32_t)(lane % SD_S);
+  uint32_t n = 0;
   auto distances = [&](uint32_t t) {
     const float4 *u = s_pos[t & 1u], *v = s_pos[t & 1u] + SD_P;
-    // a wavefront takes two starting beads at a time, half its lanes each
-    const int sep = lane % SD_S;
-#pragma unroll 5
-    for (int r = 2 * (wid - 1) + lane / SD_S; r < SD_P; r += 2 * SD_WAVES) {
+    // a wavefront takes eight starting beads at a time, eight lanes each;
+    // those from `end` on have no partner at this lane's separation
+    constexpr int PER = 64 / SD_S;
+    const int sep = lane % SD_S, end = (int)(J.i_e - J.i_s - s) - (int)((t % per) * SD_P);
+#pragma unroll 4
+    for (int r = PER * (wid - 1) + lane / SD_S; r < SD_P; r += PER * SD_WAVES) {
       const float4 a = u[r], b = v[r + sep];
       const float dx = b.x - a.x, dy = b.y - a.y, dz = b.z - a.z;
       const float xx = dx * dx, yy = dy * dy, zz = dz * dz;
-      s_d[t & 1u][r][sep] = sqrtf((xx + yy) + zz);
+      const float x = r < end ? sqrtf((xx + yy) + zz) : INFINITY;
+      s_d[t & 1u][r][sep] = r < end ? x : 0.0f;
+      n += x < 2.0f ? 1u : 0u;
     }
   };
+  if (tid < SD_S) s_n[tid] = 0u;
   if (loads) {
     s_pos[0][slot] = load_pos(0u);
     if (tiles > 1u) s_pos[1][slot] = load_pos(1u);
@@ -2055,40 +2069,37 @@ __global__ __launch_bounds__(SD_THREADS) void k_sd_cp(const float4 *__restrict__
   __syncthreads();
   if (wid > 0) distances(0u);
   __syncthreads();
-  const uint32_t s = s0 + (uint32_t)(lane % SD_S);
   // ccp adds 1000 per contact in FP32: exact, whatever the order, while the
   // sum is at most 2^24 times 8 (the largest power of two in 1000)
   const bool counts = ncc * (J.i_e - J.i_s) <= (1u << 27) / 1000u;
   float a = 0.0f, c = 0.0f;
-  uint32_t n = 0;
   // the additions are the long chain: their wavefront goes first on its SIMD
   if (wid == 0) __builtin_amdgcn_s_setprio(3);
   for (uint32_t t = 0; t < tiles; ++t) {
     if (wid == 0) {
       const float(*d)[SD_S] = s_d[t & 1u];
-      const uint32_t q = (t % per) * SD_P; // first starting bead of the tile, from the chromosome's first
-      if (counts && q + SD_P + s0 + SD_S - 1u <= J.i_e - J.i_s) {
-        // every pair of the tile is inside the chromosome
+      if (counts) {
+        // the next sixteen are read while these are added
+        float x[16];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) x[r] = d[r][lane % SD_S];
 #pragma unroll
         for (int r0 = 0; r0 < SD_P; r0 += 16) {
-          float x[16];
+          float y[16];
 #pragma unroll
-          for (int r = 0; r < 16; ++r) x[r] = d[r0 + r][lane % SD_S];
+          for (int r = 0; r < 16; ++r) y[r] = d[min(r0 + 16, SD_P - 16) + r][lane % SD_S];
 #pragma unroll
-          for (int r = 0; r < 16; ++r) {
-            a += x[r];
-            n += x[r] < 2.0f ? 1u : 0u;
-          }
+          for (int r = 0; r < 16; ++r) a += x[r];
+#pragma unroll
+          for (int r = 0; r < 16; ++r) x[r] = y[r];
         }
       } else {
+        const uint32_t q = (t % per) * SD_P; // first starting bead of the tile, from the chromosome's first
         for (int r = 0; r < SD_P; ++r) {
           const float x = d[r][lane % SD_S];
           if (q + (uint32_t)r + s < J.i_e - J.i_s) {
             a += x;
-            if (x < 2.0f) {
-              c += 1000.0f;
-              ++n;
-            }
+            if (x < 2.0f) c += 1000.0f;
           }
         }
       }
@@ -2102,9 +2113,11 @@ __global__ __launch_bounds__(SD_THREADS) void k_sd_cp(const float4 *__restrict__
     }
     __syncthreads();
   }
+  if (wid > 0) atomicAdd(&s_n[lane % SD_S], n);
+  __syncthreads();
   if (tid >= SD_S || s > J.lsdcp) return;
   const uint32_t ia = s - 1u;
-  if (counts) c = (float)(1000u * n);
+  if (counts) c = (float)(1000u * s_n[tid]);
   const float m = (float)(ncc * (J.i_e - J.i_s - s));
   a /= m;
   c /= m;
