@@ -346,7 +346,7 @@ class Simulation:
 
     def contact_map(self):
         b = self.info.contact_bins
-        m = np.zeros((b, b), np.uint32)
+        m = np.empty((b, b), np.uint32)
         ns = ctypes.c_uint32()
         self._check(lib().ccp_contact_map(self.h, _ptr(m, ctypes.c_uint32), b * b, ctypes.byref(ns)))
         return m, ns.value
@@ -390,7 +390,7 @@ class Simulation:
 
     def frame_contact_map(self):
         cms = (self.N // 2) // 4 if self.N == 30386 else self.N // 4
-        cm = np.zeros(cms * (cms + 1) // 2, np.float32)
+        cm = np.empty(cms * (cms + 1) // 2, np.float32)
         self._check(lib().ccp_frame_contact_map(self.h, _ptr(cm, ctypes.c_float), cm.size))
         return cm
 
@@ -553,7 +553,7 @@ class Batch:
         self._check(lib().ccp_batch_set_step(self.h, int(value)))
 
     def contact_maps(self):
-        m = np.zeros((self.n_sys, self.bins, self.bins), np.uint32)
+        m = np.empty((self.n_sys, self.bins, self.bins), np.uint32)
         ns = ctypes.c_uint32()
         self._check(lib().ccp_batch_contact_maps(self.h, _ptr(m, ctypes.c_uint32), m.size, ctypes.byref(ns)))
         return m, ns.value

@@ -527,7 +527,9 @@ void plan_batch(ccp_batch &bt, const char *common_params, const ccp_batch_system
       throw Error(CCP_ERR_PARAM, "batch systems must share the kernel shape, timestep and temperature");
     }
     one.hfl.assign(one.N, 0);
-    for (uint32_t i = 0; i < one.N; ++i) b->hbond.push_back(one.wbits(i) & (W_B0 | W_B1 | W_B2 | W_B3));
+    for (size_t c = 0; c + 1 < one.chain_off.size(); ++c)
+      for (uint32_t i = one.chain_off[c]; i < one.chain_off[c + 1]; ++i)
+        b->hbond.push_back(one.wbits(i, one.chain_off[c], one.chain_off[c + 1]) & (W_B0 | W_B1 | W_B2 | W_B3));
     b->sys.push_back(S);
     b->nchain.push_back((uint32_t)one.chain_off.size() - 1);
     // cell indices stay below 2^30 so that their byte offsets (index x 4)

@@ -2189,9 +2189,13 @@ __device__ __forceinline__ bool cm_apart(float4 a, float4 b) {
 // packed pixel evaluating its 32 pairs took 253 us at N = 30386 (7.2 M pixels);
 // this takes 68 us, 16 rows a block (111 us with 64: a block with contacts then
 // holds up the launch).
+//
+// The map goes to `cm`, or its nonzero pixels (index, bits of the value) to
+// `list`, whose first entry counts them; those past `cap` are only counted.
 constexpr int CM_COLS = 256, CM_ROWS = 16;
 __global__ __launch_bounds__(CM_COLS) void k_ccp_cm(uint32_t N, uint32_t cms, uint32_t lcm,
-                                                    const float4 *__restrict__ pos, float *cm, double *sum) {
+                                                    const float4 *__restrict__ pos, float *cm, double *sum,
+                                                    uint2 *list, uint32_t cap) {
   const uint32_t col0 = blockIdx.x * CM_COLS, row0 = blockIdx.y * CM_ROWS;
   if (col0 > row0 + CM_ROWS - 1u) return;
   const uint32_t ncc = (N == 30386u) ? 2u : 1u;
@@ -2228,6 +2232,17 @@ __global__ __launch_bounds__(CM_COLS) void k_ccp_cm(uint32_t N, uint32_t cms, ui
     float v = 0.0f;
     if (!(as_packed && apart)) v = cm_pixel(pos, N, ncc, ix, iy);
     if (cm) cm[ia] = v;
+    if (list) {
+      // one atomic for the pixels of a wavefront
+      const uint64_t hit = __ballot(v != 0.0f);
+      if (v != 0.0f) {
+        const uint32_t before = (uint32_t)__popcll(hit & ((1ull << __lane_id()) - 1ull));
+        uint32_t at = 0;
+        if (before == 0u) at = atomicAdd(&list[0].x, (uint32_t)__popcll(hit));
+        at = __builtin_amdgcn_readfirstlane(at) + before;
+        if (at < cap) list[1u + at] = make_uint2(ia, __float_as_uint(v));
+      }
+    }
     // (an empty pixel adds nothing)
     if (sum && v != 0.0f) sum[ia] += (double)v;
   }
@@ -2453,10 +2468,11 @@ void launch_sd_cp(hipStream_t s, const float4 *pos, uint32_t N, const SdCpJob *j
   k_sd_cp<<<dim3((longest + SD_S - 1) / SD_S, n), SD_THREADS, 0, s>>>(pos, N, all);
 }
 
-void launch_ccp_cm(hipStream_t s, uint32_t N, uint32_t cms, uint32_t lcm, const float4 *pos, float *cm, double *sum) {
+void launch_ccp_cm(hipStream_t s, uint32_t N, uint32_t cms, uint32_t lcm, const float4 *pos, float *cm, double *sum,
+                   uint2 *list, uint32_t cap) {
   if (lcm == 0) return;
   k_ccp_cm<<<dim3((cms + CM_COLS - 1) / CM_COLS, (cms + CM_ROWS - 1) / CM_ROWS), CM_COLS, 0, s>>>(N, cms, lcm, pos,
-                                                                                                cm, sum);
+                                                                                                cm, sum, list, cap);
 }
 
 void launch_bin_batch(hipStream_t s, const SysParams *sys, const uint32_t *sys_slot, int n_sys, int n,

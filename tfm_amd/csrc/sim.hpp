@@ -133,6 +133,7 @@ struct ccp_sim {
   float t = 0.0f;
   uint64_t step = 0;
   std::vector<float> hr, hlr;
+  std::vector<float4> upload_rows; // positions on their way to the device, kept so that a frame allocates nothing
   std::vector<uint8_t> hfl;
   bool lgrid_valid = false, dstep_dirty = true;
   uint32_t n_samples = 0;
@@ -268,7 +269,7 @@ struct ccp_sim {
   void configure(const ParMap &par);
   void allocate();
   void fill_kparams();
-  uint32_t wbits(uint32_t i) const;
+  uint32_t wbits(uint32_t i, uint32_t s, uint32_t e) const;
   void upload_positions();
   void upload_lbs();
   void download_positions();
