@@ -177,18 +177,18 @@ def test_distance_contact_ragged_tiles(N):
     sim.close()
 
 
-@pytest.mark.parametrize("N,scale,pixels", [(2043, 0.6, "whole"), (2048, 1.0, "list"), (2048, 0.6, "whole"),
+@pytest.mark.parametrize("N,scale,pixels", [(2048, 1.0, "whole"), (4092, 1.0, "whole"), (4096, 1.0, "list"),
                                             (8190, 1.0, "list"), (8190, 0.45, "long list"), (8190, 0.05, "whole")])
 def test_frame_contact_map_lists(N, scale, pixels):
     # nearly empty maps, which reach the host as a list of nonzero pixels (one
     # copy up to 32768 of them, then a second), and small or dense ones (more
-    # than a sixteenth), which are copied whole; into an array of other values
+    # than an eighth), which are copied whole; into an array of other values
     step(f"frame contact map N={N} scale={scale}")
     R_n = radius_for(N, 0.3)
     sim = sim_with(N, R_n, walk(N, R_n, seed=5) * np.float32(scale), np.zeros(N, np.uint8))
     want = po.ccp_contact_map(sim.positions)
     n, lcm = int((want != 0).sum()), want.size
-    listed = lcm >= 1 << 17 and n <= lcm // 16
+    listed = lcm >= 1 << 19 and n <= lcm // 8
     assert pixels == ("whole" if not listed else "list" if n <= 32768 else "long list")
     got = np.full(lcm, np.nan, np.float32)
     lib, ptr = tfm_amd.ccp.lib(), tfm_amd.ccp._ptr

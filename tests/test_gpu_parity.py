@@ -377,6 +377,35 @@ def test_contacts_over_reaches(N, bs, shape):
     sim.close()
 
 
+@pytest.mark.parametrize("N,bs,scale,words", [(2172, 3, 1.0, "whole"), (2175, 3, 1.0, "list"), (2000, 2, 1.0, "list"),
+                                              (4100, 4, 0.3, "long list"), (4100, 4, 0.2, "whole")])
+def test_contact_map_lists(N, bs, scale, words):
+    # maps on either side of 2^19 words, of a ragged last 4096, and too dense
+    # for a list (the chain shrunk to a ball): the oracle's whole numbers, into
+    # an array of other values, and the sum of two samples on a second read
+    step(f"contact map N={N} bin={bs} scale={scale}")
+    R_n = radius_for(N, 0.3)
+    sim = tfm_amd.Simulation({"number_of_particles": N, "nucleus_radius": repr(float(R_n)), "seed": 4,
+                              "number_of_lbs": 0, "force_field": "lj", "contact_bin_size": bs, "cell_reach": 2,
+                              "cell_size": 1.25, "lanes_per_bead": 8, "cell_capacity": 1024})
+    r = np.ascontiguousarray(walk(N, R_n, N + 3) * scale, np.float32)
+    sim.flags = np.zeros(N, np.uint8)
+    sim.positions = r
+    nb = sim.info.contact_bins
+    want = po.contacts(r, np.float32(1.5), bs, nb)
+    n = int((want != 0).sum())
+    listed = nb * nb >= 1 << 19 and n <= nb * nb // 8
+    assert words == ("whole" if not listed else "list" if n <= 32768 else "long list")
+    lib, ptr = tfm_amd.ccp.lib(), tfm_amd.ccp._ptr
+    sim.contact_reset()
+    for samples in (1, 2):
+        sim.contact_sample()
+        m = np.full((nb, nb), 7, np.uint32)
+        assert lib.ccp_contact_map(sim.h, ptr(m, tfm_amd.ccp.ctypes.c_uint32), nb * nb, None) == 0
+        assert np.array_equal(m, samples * want)
+    sim.close()
+
+
 @pytest.mark.parametrize("N,cvf", [(1, 0.05), (3, 0.1), (65, 0.39), (700, 0.002), (5000, 0.3)])
 def test_default_shape_of_ccp_field(N, cvf):
     # ccp's force field with no shape key: eight lanes over ~1.2 sigma cells,

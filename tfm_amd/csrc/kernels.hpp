@@ -254,6 +254,7 @@ void launch_observables(hipStream_t s, int N, double R_n, double nod, double a, 
 // d(s) and P(s) of up to SD_CP_JOBS chromosomes in one launch
 void launch_sd_cp(hipStream_t s, const float4 *pos, uint32_t N, const SdCpJob *jobs, int n_jobs);
 // packed map of cms x cms pixels (lcm = cms (cms + 1) / 2 of them)
+void launch_list_words(hipStream_t s, const uint32_t *map, uint32_t n, uint2 *list, uint32_t cap);
 void launch_ccp_cm(hipStream_t s, uint32_t N, uint32_t cms, uint32_t lcm, const float4 *pos, float *cm, double *sum,
                    uint2 *list = nullptr, uint32_t cap = 0);
 void launch_bin_batch(hipStream_t s, const SysParams *sys, const uint32_t *sys_slot, int n_sys, int n,

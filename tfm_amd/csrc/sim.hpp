@@ -133,6 +133,9 @@ struct ccp_sim {
   float t = 0.0f;
   uint64_t step = 0;
   std::vector<float> hr, hlr;
+  DevBuf<uint2> list;          // a map's nonzero words on their way to the host (at most a quarter of the map)
+  uint2 *list_head = nullptr;  // pinned: its count and first entries
+  std::vector<uint2> list_rest;
   std::vector<float4> upload_rows; // positions on their way to the device, kept so that a frame allocates nothing
   std::vector<uint8_t> hfl;
   bool lgrid_valid = false, dstep_dirty = true;
@@ -233,6 +236,7 @@ struct ccp_sim {
     drop_graphs();
     DevBuf<float4> *f4[] = {&r, &er, &pstar, &lr, &lspos, &aux, &fpair, &znoise, &fbond};
     for (auto *b : f4) b->free_();
+    list.free_();
     DevBuf<uint32_t> *u4[] = {&lstart, &flags, &cmap};
     for (auto *b : u4) b->free_();
     gf.free_();
@@ -241,6 +245,7 @@ struct ccp_sim {
     dstep.free_();
     dcount.free_();
     if (hsig) (void)hipHostFree(hsig);
+    if (list_head) (void)hipHostFree(list_head);
     if (stream) (void)hipStreamDestroy(stream);
   }
 
@@ -270,6 +275,8 @@ struct ccp_sim {
   void allocate();
   void fill_kparams();
   uint32_t wbits(uint32_t i, uint32_t s, uint32_t e) const;
+  uint2 *list_space(size_t words);
+  bool take_list(void *map, size_t words);
   void upload_positions();
   void upload_lbs();
   void download_positions();
