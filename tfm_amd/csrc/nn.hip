@@ -552,7 +552,8 @@ template <bool CONV> __global__ __launch_bounds__(NET_THREADS) void k_fwd(ccp_nn
 // (columns ds ..): S = (M + M^T) / 2 + dist[|i - j|] + c0, M = alpha U^T V.
 // One 32 x 32 block of S per wavefront; the transposed block is a second
 // product with U and V exchanged (the same products in the same order), so M
-// is neither stored nor read back.
+// is neither stored nor read back. 64 samples of 128 x 128, d = 64: 8.1 -> 7.6 us
+// with the distance terms loaded ahead and four groups in flight, not two.
 struct PairFrags {
   bf16x8 ui, vi, uj, vj;
 };
@@ -571,50 +572,66 @@ __global__ __launch_bounds__(256) void k_pair(const uint16_t *__restrict__ uv, i
 #pragma unroll
   for (int v = 0; v < 16; ++v) m[v] = mt[v] = 0.0f;
   const int nk = ds / 16;
-  PairFrags ring[2];
+  PairFrags ring[4];
   auto load = [&](PairFrags &t, int k) {
     t.ui = *(const bf16x8 *)(ri + 16 * k);
     t.vi = *(const bf16x8 *)(ri + ds + 16 * k);
     t.uj = *(const bf16x8 *)(rj + 16 * k);
     t.vj = *(const bf16x8 *)(rj + ds + 16 * k);
   };
-  load(ring[0], 0);
-  load(ring[1], min(1, nk - 1));
-  in_rounds<2>(nk, [&](int i, int k) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) load(ring[i], min(i, nk - 1));
+  // the distance terms before the stores: a load behind a store waits for it
+  const int col = j0 + r;
+  const float c = c0[0];
+  float far[16];
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const int d = i0 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3) - col;
+    far[v] = dist[min(d < 0 ? -d : d, L - 1)];
+  }
+  in_rounds<4>(nk, [&](int i, int k) {
     m = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ring[i].ui, ring[i].vj, m, 0, 0, 0);
     mt = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ring[i].vi, ring[i].uj, mt, 0, 0, 0);
-    load(ring[i], min(k + 2, nk - 1));
+    load(ring[i], min(k + 4, nk - 1));
   });
-  const int col = j0 + r;
   if (col >= L) return;
 #pragma unroll
   for (int v = 0; v < 16; ++v) {
     const int row = i0 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
     if (row >= L) continue;
     const float a = alpha * m[v], at_ = alpha * mt[v];
-    const int d = row > col ? row - col : col - row;
-    S[((long)b * L + row) * L + col] = 0.5f * (a + at_) + dist[d] + c0[0];
+    S[((long)b * L + row) * L + col] = 0.5f * (a + at_) + far[v] + c;
   }
 }
 
 // mean over l of h[c, b L + l], summed in order, in BF16 as pb[C][Bs] and pt[B][Cs].
 // A workgroup brings POOL_ROWS of the rows (c, b) into LDS in whole lines,
-// then one lane adds each (a lane reading its own row took 18 us for 16384
-// rows of 128, this 9.5 us).
+// then one lane adds each. 16384 rows of 128: 4.6 us (a lane reading its own row
+// 18 us; with two 64-bit divisions for each value's place 9.5 us).
 constexpr int POOL_ROWS = 32, POOL_SEG = 128;
 __global__ __launch_bounds__(256) void k_pool(const float *h, uint16_t *pb, uint16_t *pt, int C, int B, int L, int Ps,
                                               int Bs, int Cs) {
   __shared__ float s[POOL_ROWS][POOL_SEG + 1];
+  __shared__ long place[POOL_ROWS]; // of a row's first value
   const long rows = (long)C * B, r0 = (long)blockIdx.x * POOL_ROWS;
   float sum = 0.0f;
+  if (threadIdx.x < POOL_ROWS) {
+    const long i = min(r0 + (long)threadIdx.x, rows - 1);
+    place[threadIdx.x] = i / B * Ps + i % B * L;
+  }
   for (int l0 = 0; l0 < L; l0 += POOL_SEG) {
     const int n = min(POOL_SEG, L - l0);
     __syncthreads();
-    for (int e = threadIdx.x; e < POOL_ROWS * POOL_SEG; e += 256) {
-      const int r = e / POOL_SEG, l = e % POOL_SEG;
-      const long i = r0 + r;
-      if (i < rows && l < n) s[r][l] = h[i / B * Ps + i % B * L + l0 + l];
-    }
+    // all of a thread's values in flight together (places past a row's end: its
+    // last value, which is not added)
+    constexpr int STEP = 256 / POOL_SEG, EACH = POOL_ROWS / STEP;
+    const int l = threadIdx.x % POOL_SEG, row = threadIdx.x / POOL_SEG;
+    float v[EACH];
+#pragma unroll
+    for (int k = 0; k < EACH; ++k) v[k] = h[place[row + k * STEP] + min(l0 + l, L - 1)];
+#pragma unroll
+    for (int k = 0; k < EACH; ++k) s[row + k * STEP][l] = v[k];
     __syncthreads();
     if (threadIdx.x < POOL_ROWS) {
       int l = 0;
@@ -675,8 +692,10 @@ __global__ __launch_bounds__(64) void k_small(const uint16_t *__restrict__ A, co
 // off the diagonal and g(r, r) on it, as BF16 rows of Ls entries; the sums of
 // g along each diagonal of the band as a partial of gdist. One workgroup per
 // sample and band of PL_ROWS rows. A lane takes one diagonal for the upper
-// triangle (consecutive lanes read consecutive columns), then one column for
-// the lower one, whose PL_ROWS values lie side by side in that column's row.
+// triangle (consecutive lanes read consecutive columns), or one column for
+// the lower one, whose PL_ROWS values lie side by side in that column's row:
+// at 128 bins each of 256 lanes has one of them, 14.6 us for 64 samples (16.3
+// with the columns behind the diagonals on half the lanes).
 constexpr int PL_ROWS = 16;
 __global__ __launch_bounds__(256) void k_pair_grad(const float *pred, const float *target, uint16_t *graw, float *gdist,
                                                    float *gc0, float *loss, int L, int Ls, int B, float w) {
@@ -688,41 +707,47 @@ __global__ __launch_bounds__(256) void k_pair_grad(const float *pred, const floa
   // (a band's values are loaded together: places past the sample's last are
   // read from it and left out)
   float x[PL_ROWS], y[PL_ROWS];
-  for (int d = threadIdx.x; d < L; d += 256) {
-    float sum = 0.0f;
+  // the band's diagonals, then its columns, from the next whole wavefront on
+  const int cols = (L + 63) / 64 * 64;
+  for (int e = threadIdx.x; e < cols + r1; e += 256) {
+    if (e < cols) {
+      const int d = e;
+      if (d >= L) continue;
+      float sum = 0.0f;
 #pragma unroll
-    for (int i = 0; i < PL_ROWS; ++i) {
-      const long u = base + (long)min(r0 + i, L - 1) * L + min(r0 + i + d, L - 1);
-      x[i] = pred[u];
-      y[i] = target[u];
-    }
+      for (int i = 0; i < PL_ROWS; ++i) {
+        const long u = base + (long)min(r0 + i, L - 1) * L + min(r0 + i + d, L - 1);
+        x[i] = pred[u];
+        y[i] = target[u];
+      }
 #pragma unroll
-    for (int i = 0; i < PL_ROWS; ++i) {
-      const int r = r0 + i;
-      if (r + d >= L) continue;
-      const float e = x[i] - y[i];
-      const float g = 2.0f * w * e / count;
-      sum += g;
-      sq += w * e * e / count;
-      graw[((long)b * L + r) * Ls + r + d] = f2bf(d == 0 ? g : 0.5f * g);
-    }
-    gd[d] = sum;
-    all += sum;
-  }
-  for (int c = threadIdx.x; c < r1; c += 256) {
+      for (int i = 0; i < PL_ROWS; ++i) {
+        const int r = r0 + i;
+        if (r + d >= L) continue;
+        const float e = x[i] - y[i];
+        const float g = 2.0f * w * e / count;
+        sum += g;
+        sq += w * e * e / count;
+        graw[((long)b * L + r) * Ls + r + d] = f2bf(d == 0 ? g : 0.5f * g);
+      }
+      gd[d] = sum;
+      all += sum;
+    } else {
+      const int c = e - cols;
 #pragma unroll
-    for (int i = 0; i < PL_ROWS; ++i) {
-      const long u = base + (long)c * L + min(r0 + i, L - 1);
-      x[i] = pred[u];
-      y[i] = target[u];
-    }
+      for (int i = 0; i < PL_ROWS; ++i) {
+        const long u = base + (long)c * L + min(r0 + i, L - 1);
+        x[i] = pred[u];
+        y[i] = target[u];
+      }
 #pragma unroll
-    for (int i = 0; i < PL_ROWS; ++i) {
-      const int r = r0 + i;
-      if (r <= c || r >= r1) continue;
-      const float e = x[i] - y[i];
-      const float g = 2.0f * w * e / count;
-      graw[((long)b * L + r) * Ls + c] = f2bf(0.5f * g);
+      for (int i = 0; i < PL_ROWS; ++i) {
+        const int r = r0 + i;
+        if (r <= c || r >= r1) continue;
+        const float e = x[i] - y[i];
+        const float g = 2.0f * w * e / count;
+        graw[((long)b * L + r) * Ls + c] = f2bf(0.5f * g);
+      }
     }
   }
   __shared__ float red[2][EW];
