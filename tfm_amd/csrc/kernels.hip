@@ -655,9 +655,11 @@ __device__ __forceinline__ void load_system(KParams &p, const KPtrs &q, uint32_t
 }
 
 // Unit normal triple of bead g (index over all systems) for the job's step.
-__device__ __forceinline__ void fill_noise(const NoiseJob &nj, uint32_t g) {
+// BATCH at compile time, here and in fill_bond: the search for a system in the
+// single system's order pass, never run, cost it registers (0.8 % of a step).
+template <bool BATCH> __device__ __forceinline__ void fill_noise(const NoiseJob &nj, uint32_t g) {
   uint32_t k0 = nj.seed_lo, k1 = nj.seed_hi, local = g;
-  if (nj.sys) {
+  if constexpr (BATCH) {
     const SysParams &S = nj.sys[system_of(nj.sys_slot, nj.n_sys, g)];
     k0 = S.seed_lo;
     k1 = S.seed_hi;
@@ -684,8 +686,9 @@ __device__ __forceinline__ BondNbrs load_bond_nbrs(const BondJob &bj, uint32_t g
   b.p2 = bj.pos[g + 2u < bj.n ? g + 2u : g];
   return b;
 }
+template <bool BATCH>
 __device__ __forceinline__ void fill_bond(KParams p, const BondJob &bj, uint32_t g, const BondNbrs &b) {
-  if (bj.sys) {
+  if constexpr (BATCH) {
     const SysParams &S = bj.sys[system_of(bj.sys_slot, bj.n_sys, g)];
     p.R_n = S.R_n; p.R_o = S.R_o; p.R_b = S.R_b;
     p.noc = S.noc; p.boc = S.boc; p.nod = S.nod; p.bod = S.bod;
@@ -1338,7 +1341,7 @@ __global__ __launch_bounds__(BAL_BLOCK) void k_force_typed(KParams p, KPtrs q, N
   // launch's tail, on SIMDs that the force wavefronts leave idle.
   if (b >= p.het_blocks + t_blocks) {
     const uint32_t g = (uint32_t)(b - p.het_blocks - t_blocks) * BAL_BLOCK + threadIdx.x;
-    if (nj.z && g < nj.n) fill_noise(nj, g);
+    if (nj.z && g < nj.n) fill_noise<BATCH>(nj, g);
     return;
   }
   const bool het_part = b < p.het_blocks;
@@ -1540,8 +1543,8 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_order(OrderJobs<TWO ? 2 : 1> job
       const bool bond = bj.out && g < bj.n;
       BondNbrs nbr;
       if (bond) nbr = load_bond_nbrs(bj, g);
-      if (nj.z && g < nj.n) fill_noise(nj, g);
-      if (bond) fill_bond(bp, bj, g, nbr);
+      if (nj.z && g < nj.n) fill_noise<BATCH>(nj, g);
+      if (bond) fill_bond<BATCH>(bp, bj, g, nbr);
     }
   }
   uint32_t part = (pv[0] + pv[1]) + (pv[2] + pv[3]);
@@ -1739,10 +1742,10 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_order(OrderJobs<TWO ? 2 : 1> job
 }
 
 // The same terms on their own, before the first stage of a run.
-__global__ __launch_bounds__(BEAD_BLOCK) void k_bead_terms(NoiseJob nj, KParams p, BondJob bj) {
+template <bool BATCH> __global__ __launch_bounds__(BEAD_BLOCK) void k_bead_terms(NoiseJob nj, KParams p, BondJob bj) {
   const uint32_t g = blockIdx.x * BEAD_BLOCK + threadIdx.x;
-  if (nj.z && g < nj.n) fill_noise(nj, g);
-  if (bj.out && g < bj.n) fill_bond(p, bj, g, load_bond_nbrs(bj, g));
+  if (nj.z && g < nj.n) fill_noise<BATCH>(nj, g);
+  if (bj.out && g < bj.n) fill_bond<BATCH>(p, bj, g, load_bond_nbrs(bj, g));
 }
 
 // Contact counts on the fine grid: pairs i < j with d < rc within
@@ -2358,7 +2361,8 @@ void launch_bead_terms(hipStream_t s, const NoiseJob *noise, const KParams &p, c
   if (bond) bj = *bond;
   const uint32_t n = nj.z ? nj.n : bj.out ? bj.n : 0u; // both cover every bead
   if (n == 0) return;
-  k_bead_terms<<<blocks_for((int)n, BEAD_BLOCK), BEAD_BLOCK, 0, s>>>(nj, p, bj);
+  if (nj.sys || bj.sys) k_bead_terms<true><<<blocks_for((int)n, BEAD_BLOCK), BEAD_BLOCK, 0, s>>>(nj, p, bj);
+  else k_bead_terms<false><<<blocks_for((int)n, BEAD_BLOCK), BEAD_BLOCK, 0, s>>>(nj, p, bj);
 }
 
 template <int MODE, bool SPLIT, bool BATCH, int R, int LANES>
