@@ -114,8 +114,8 @@ def test_frame_contact_map_two_copies():
 
 @pytest.mark.parametrize("N", [8, 64, 65, 66, 127, 258, 1089, 4223])
 def test_distance_contact_tile_edges(N):
-    # separations and starting beads at the edges of the kernel's tiles (32 x
-    # 64): one separation, a tile and one more or less, many ragged tiles
+    # separations and starting beads at the edges of tiles of 32 x 64:
+    # one separation, a tile and one more or less, many ragged tiles
     step(f"d(s), P(s) N={N}")
     R_n = radius_for(N, 0.2)
     sim = sim_with(N, R_n, walk(N, R_n, seed=N), np.zeros(N, np.uint8))
@@ -167,7 +167,7 @@ def test_frame_contact_map_rounded_rows():
 @pytest.mark.parametrize("N", [33, 34, 113, 114, 128, 129, 226, 241])
 def test_distance_contact_ragged_tiles(N):
     # a last separation and a last starting bead on either side of the edges
-    # of tiles of 16 separations x 112 beads
+    # of tiles of 8 and 16 separations x 112 beads
     step(f"d(s), P(s) N={N}")
     R_n = radius_for(N, 0.2)
     sim = sim_with(N, R_n, walk(N, R_n, seed=N), np.zeros(N, np.uint8))
