@@ -380,9 +380,8 @@ uint2 *ccp_sim::list_space(size_t words) {
     hip_check(hipHostMalloc(&p, (1 + LIST_FIRST) * sizeof(uint2)));
     list_head = static_cast<uint2 *>(p);
   }
-  if (list.n < entries) {
+  if (!list.p || list.n < entries) { // (an allocation that failed leaves no memory but its size)
     list.free_();
-    list.n = 0;
     list.alloc(entries);
   }
   hip_check(hipMemsetAsync(list.p, 0, sizeof(uint2), stream));
