@@ -182,9 +182,9 @@ int ccp_step_grid(ccp_sim *h, uint32_t *cstart, size_t n_c1, uint32_t *soi, size
  * in ccp: it serves callers that cannot allocate device memory (code under
  * hipGraph capture, serving loops, harnesses that forbid hipMalloc). Its
  * only device memory beyond the arguments is a fixed array of 256 KiB per
- * GPU, so cps is at most 255 (CCP_ERR_ARG beyond); calls that overlap in
- * time on one GPU share that array and race. A bead outside the grid gives
- * CCP_ERR_STATE. Errors: ccp_last_error(NULL). */
+ * GPU, so cps is at most 255 (CCP_ERR_ARG beyond); calls on one GPU share
+ * that array and wait for each other, whatever their threads and streams.
+ * A bead outside the grid gives CCP_ERR_STATE. Errors: ccp_last_error(NULL). */
 int ccp_cell_list_noalloc(const float *xyz, uint32_t n, float csl, uint32_t cps, uint32_t *sci, uint32_t *soi,
                           uint32_t *beg, uint32_t *end, void *stream);
 

@@ -1,0 +1,89 @@
+"""What the library's host code asks of the HIP runtime, on the CPU: each test
+runs in a process of its own with tests/host_runtime.cpp in the runtime's
+place (no kernel runs, every launch and wait is logged)."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+
+@pytest.fixture(scope="module")
+def runtime(tmp_path_factory):
+    so = tmp_path_factory.mktemp("rt") / "host_runtime.so"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-pthread", "-o", str(so),
+                    os.path.join(HERE, "host_runtime.cpp")], check=True)
+    return str(so)
+
+
+PRELUDE = """
+import ctypes, sys, threading
+sys.path.insert(0, {root!r})
+rt = ctypes.CDLL({so!r}, mode=ctypes.RTLD_GLOBAL)
+rt.rt_memory_limit.argtypes = [ctypes.c_size_t]
+rt.rt_events.argtypes = [ctypes.c_char_p, ctypes.c_size_t]
+rt.rt_events.restype = ctypes.c_size_t
+def events():
+    buf = ctypes.create_string_buffer(rt.rt_events(None, 0) + (1 << 20))
+    rt.rt_events(buf, len(buf))
+    return [line.split(" ", 1) for line in buf.value.decode().splitlines()]
+import numpy as np
+import tfm_amd
+from tfm_amd import ccp
+L = ccp.lib()
+"""
+
+
+def run(runtime, *parts):
+    code = PRELUDE.format(root=ROOT, so=runtime) + "\n".join(textwrap.dedent(p) for p in parts) + "\nprint('done')"
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and r.stdout.endswith("done\n"), r.stdout + r.stderr
+
+
+CELL_LIST = """
+def call(n=64, cps=8):
+    u = lambda k: (ctypes.c_uint32 * k)()
+    return L.ccp_cell_list_noalloc((ctypes.c_float * (3 * n))(), n, 1.0, cps, u(n), u(n), u(cps ** 3), u(cps ** 3), None)
+"""
+
+
+@pytest.mark.parametrize("cps", [8, 70])
+def test_cell_list_calls_do_not_overlap(runtime, cps):
+    # The calls of a GPU share one array, and the scan's blocks wait for words
+    # of it: one call's launches and its wait come before the next one's first
+    # launch, whatever threads they come from.
+    run(runtime, CELL_LIST, f"""
+    cps = {cps}
+    assert call(cps=cps) == 0
+    per_call = len(events())
+    rt.rt_launch_time(200)
+    rcs = []
+    ts = [threading.Thread(target=lambda: [rcs.append(call(cps=cps)) for _ in range(5)]) for _ in range(4)]
+    for t in ts: t.start()
+    for t in ts: t.join()
+    assert rcs == [0] * 20
+    log = events()
+    assert len(log) == 20 * per_call
+    for k in range(0, len(log), per_call):
+        group = log[k:k + per_call]
+        assert len({{t for t, _ in group}}) == 1, log
+        assert "k_na_clear" in group[0][1] and group[-1][1] == "wait", log
+    """)
+
+
+def test_cell_list_call_that_fails_waits_for_its_launches(runtime):
+    # an error found after the launches: the call ends behind a wait, so that
+    # the next one's launches cannot meet them
+    run(runtime, CELL_LIST, """
+    assert call() == 0
+    events()
+    rt.rt_fail_last_error(1)
+    assert call() == tfm_amd.CCP_ERR_HIP
+    log = events()
+    assert any("k_na_finish" in e for _, e in log) and log[-1][1] == "wait", log
+    assert call() == 0
+    """)

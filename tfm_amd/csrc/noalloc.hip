@@ -28,8 +28,10 @@
 // seven (block sums and their scan as kernels of their own). Block sums added
 // up by atomics in step 2 cost more than both: neighbouring words of a few
 // cache lines, 98 us for that kernel.
-// Calls on one GPU share its scratch array: calls that overlap in time on
-// one GPU race and must not be issued.
+// Calls on one GPU share its scratch array, and a scan block waits for words
+// of it that another call's clearing would erase: a call holds the GPU's lock
+// from its first launch until its stream is done, so that the calls of a
+// process on one GPU run one after another, whatever their threads and streams.
 
 #include "ccpmi.h"
 #include "host.hpp"
@@ -139,7 +141,8 @@ __global__ __launch_bounds__(NA_BLOCK) void k_na_starts(uint32_t *count_cursor, 
 // The same in one launch for up to NA_DIRECT blocks (four words a lane, less
 // than the two launches it saves). Blocks are numbered in the order in which
 // they start, and each publishes its sum (below 2^31, bit 31 set: sum and flag
-// are one word) before it waits for the blocks before it, so every wait ends.
+// are one word) before it waits for the blocks before it, so every wait ends:
+// nothing else writes these words meanwhile (the lock of ccp_cell_list_noalloc).
 constexpr uint32_t NA_DIRECT = 1024;
 __global__ __launch_bounds__(NA_BLOCK) void k_na_starts_direct(uint32_t *count_cursor, uint32_t n_c, uint32_t *sc,
                                                                uint32_t *beg) {
@@ -195,22 +198,40 @@ __global__ __launch_bounds__(NA_BLOCK) void k_na_finish(uint32_t n_c, uint32_t *
   for (uint32_t s = s0; s < s1; ++s) sci[s] = c;
 }
 
-// the address of this GPU's scratch array, looked up once per device
-std::mutex g_na_mutex;
-uint32_t *g_na_ptr[NA_MAX_DEVICES] = {};
+// each GPU's lock and the address of its scratch array, looked up once
+struct NaDevice {
+  std::mutex lock;
+  uint32_t *scratch = nullptr;
+};
+NaDevice g_na[NA_MAX_DEVICES];
 
-uint32_t *scratch_ptr() {
-  int dev = 0;
-  host::hip_check(hipGetDevice(&dev));
-  if (dev < 0 || dev >= NA_MAX_DEVICES) throw host::Error(CCP_ERR_ARG, "device index beyond the supported range");
-  std::lock_guard<std::mutex> lock(g_na_mutex);
-  if (!g_na_ptr[dev]) {
-    void *p = nullptr;
-    host::hip_check(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
-    g_na_ptr[dev] = static_cast<uint32_t *>(p);
+// One call on the current GPU: the lock is held until the launches on the
+// stream are done, also when the call ends with an error behind them.
+struct NaCall {
+  std::unique_lock<std::mutex> lock;
+  uint32_t *sc = nullptr;
+  hipStream_t s;
+  bool waiting = true;
+  explicit NaCall(hipStream_t stream) : s(stream) {
+    int dev = 0;
+    host::hip_check(hipGetDevice(&dev));
+    if (dev < 0 || dev >= NA_MAX_DEVICES) throw host::Error(CCP_ERR_ARG, "device index beyond the supported range");
+    lock = std::unique_lock<std::mutex>(g_na[dev].lock);
+    if (!g_na[dev].scratch) {
+      void *p = nullptr;
+      host::hip_check(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
+      g_na[dev].scratch = static_cast<uint32_t *>(p);
+    }
+    sc = g_na[dev].scratch;
   }
-  return g_na_ptr[dev];
-}
+  void wait() {
+    waiting = false;
+    host::hip_check(hipStreamSynchronize(s));
+  }
+  ~NaCall() {
+    if (waiting) (void)hipStreamSynchronize(s);
+  }
+};
 
 unsigned na_blocks(uint32_t n) { return (n + NA_BLOCK - 1) / NA_BLOCK; }
 
@@ -228,7 +249,8 @@ extern "C" int ccp_cell_list_noalloc(const float *xyz, uint32_t n, float csl, ui
       throw host::Error(CCP_ERR_ARG, "cells per side out of range: at most 255 (2^24 cells) without allocation");
     const uint32_t n_c = cps * cps * cps, nblk = na_blocks(n_c);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    uint32_t *sc = scratch_ptr();
+    NaCall call(s);
+    uint32_t *sc = call.sc;
     k_na_clear<<<nblk, NA_BLOCK, 0, s>>>(n_c, end, sc);
     k_na_key<<<na_blocks(n), NA_BLOCK, 0, s>>>(xyz, n, csl, (int)cps, sci, end, sc);
     if (nblk <= NA_DIRECT) {
@@ -243,7 +265,7 @@ extern "C" int ccp_cell_list_noalloc(const float *xyz, uint32_t n, float csl, ui
     host::hip_check(hipGetLastError());
     uint32_t outside = 0;
     host::hip_check(hipMemcpyAsync(&outside, sc + NA_FLAG, sizeof(outside), hipMemcpyDeviceToHost, s));
-    host::hip_check(hipStreamSynchronize(s));
+    call.wait();
     if (outside) throw host::Error(CCP_ERR_STATE, "bead left the cell grid");
     return CCP_OK;
   } catch (const host::Error &e) {
