@@ -87,3 +87,29 @@ def test_cell_list_call_that_fails_waits_for_its_launches(runtime):
     assert any("k_na_finish" in e for _, e in log) and log[-1][1] == "wait", log
     assert call() == 0
     """)
+
+
+SHAPE = """
+def fine_cells(n, vf, **kw):
+    rco = 1.154701
+    r = rco / 2 + rco / 2 * (n / vf) ** (1 / 3)
+    s = tfm_amd.Simulation({"number_of_particles": n, "nucleus_radius": f"{r:.6f}", "seed": 1, **kw})
+    side, cps = float(s.info.fine_csl), int(s.info.fine_cps)
+    s.close()
+    return side, cps
+"""
+
+
+@pytest.mark.parametrize("n,vf,half", [
+    (1024, 0.2, True), (16384, 0.03, True), (32768, 0.03, False), (65536, 0.1, True), (65536, 0.04, False),
+    (131072, 0.1, True), (131072, 0.06, False), (262144, 0.15, True), (262144, 0.08, False), (524288, 0.2, True),
+    (524288, 0.1, False), (524289, 0.2, False), (600000, 0.3, False)])
+def test_default_cells_of_ccp_field(runtime, n, vf, half):
+    # eight lanes over cells of about 1.2 sigma where they were measured to be
+    # the faster shape, and at no size above the one that has run
+    run(runtime, SHAPE, f"""
+    side, cps = fine_cells({n}, {vf})
+    assert (1.2 <= side < 1.34) if {half} else side == 2.0, (side, cps)
+    assert not {half} or cps ** 3 <= min(32 * {n} + 32768, (2e7 * {n}) ** 0.5)
+    assert fine_cells({n}, {vf}, lanes_per_bead=3)[0] == 2.0
+    """)

@@ -465,13 +465,6 @@ std::string system_text(const std::string &common, const ccp_batch_system &s, ui
   return common + "\n" + buf;
 }
 
-// The half-cutoff cells at eight lanes per bead (reach 2, cells below
-// 1.3 sigma) have run clean in batches of up to this many beads (256 chains of
-// 2048). A command that ran a 1.1M-bead ensemble of this shape for 1e4 steps,
-// after initial conditions generated on 16 host threads, faulted the GPU; its
-// cause is not known, so larger batches of this shape are refused.
-constexpr uint64_t HALF_CELL_BATCH_LIMIT = 524288;
-
 // Everything of a batch that needs no device: each system's parameter text,
 // constants, geometry and place in the shared bead and cell ranges.
 void plan_batch(ccp_batch &bt, const char *common_params, const ccp_batch_system *systems, uint32_t n_sys) {

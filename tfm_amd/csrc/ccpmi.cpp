@@ -142,9 +142,18 @@ void ccp_sim::configure(const ParMap &par) {
   // cells: N = 256 25.7 (39.1), 1024 28.1 (44.1), 4096 29.2 (45.1), 16384
   // 32.4 (44.4), 30386 35.3 (52.3), 32768 at volume fraction 0.25 35.1 (58.1).
   // Eight lanes over the 2 sigma cells lie between, and above both in the
-  // dense nucleus (64). The order pass pays per cell, so nuclei with few
-  // beads for their size (below a volume fraction of 0.03 or so) keep the
-  // wide cells, and with them the memory of their buckets.
+  // dense nucleus (64).
+  // The order pass pays per cell, and each of its blocks reads the totals of
+  // the blocks before it, so its cost has a term in the square of the cells
+  // against a gain per bead: the line n_c^2 = 2e7 N. us per step on its two
+  // sides: 65536 beads, 1.06 M cells 60.0 (70.2), 1.56 M 73.0 (67.4); 131072,
+  // 1.19 M 80.5 (99.9), 2.0 M 107 (94.7); 262144, 1.64 M 128 (162), 2.5 M 162
+  // (155); 524288, 3.24 M 262 (271), 4.74 M 373 (267), 16.8 M 2504 (346).
+  // Up to about 19000 beads the bound of 32 N + 32768 cells comes first, a
+  // volume fraction of 0.03 or so: there the gain is still 1.2 and more, but
+  // the buckets take 512 bytes a cell, so nuclei with fewer beads for their
+  // size keep the wide cells, a fifth as many.
+  // Above HALF_CELL_BATCH_LIMIT beads the shape has not run.
   if (!lj && !split) {
     bool plain = true;
     for (const char *k : {"lanes_per_bead", "cell_reach", "cell_size", "fine_cell_size", "cell_capacity",
@@ -154,7 +163,8 @@ void ccp_sim::configure(const ParMap &par) {
     // in a whole number of cells
     extent = gh.g.half * csl;
     const double n = std::floor((double)extent / STEP_CSL_CCP);
-    if (plain && 8.0 * n * n * n <= 32.0 * N + 32768.0) {
+    const double n_c = 8.0 * n * n * n;
+    if (plain && N <= HALF_CELL_BATCH_LIMIT && n_c <= 32.0 * N + 32768.0 && n_c * n_c <= 2e7 * N) {
       csl_f = (float)(extent / n);
       extent = csl_f * ((float)n - 0.5f); // (n cells, whatever the quotient's rounding)
       reach = 2;

@@ -90,6 +90,14 @@ using namespace ccpmi::host;
 // list radii, at least half the long one
 constexpr float STEP_CSL_CCP = 1.2f;
 
+// The half-cutoff cells at eight lanes per bead (reach 2, cells below
+// 1.3 sigma) have run clean in batches of up to this many beads (256 chains of
+// 2048). A command that ran a 1.1M-bead ensemble of this shape for 1e4 steps,
+// after initial conditions generated on 16 host threads, faulted the GPU; its
+// cause is not known, so larger batches of this shape are refused, and larger
+// single systems do not get it as their default.
+constexpr uint32_t HALF_CELL_BATCH_LIMIT = 524288;
+
 // ---------------------------------------------------------------- handle
 struct ccp_sim {
   // parameters
