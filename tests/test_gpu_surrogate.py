@@ -127,3 +127,19 @@ def test_training_reduces_loss():
         net.step(lr=3e-3)
     assert np.isfinite(losses).all()
     assert losses[-1] < 0.2 * losses[0]
+
+
+def test_loss_outlives_a_forward_pass():
+    # the returned loss is a buffer that the next loss_backward fills; a
+    # forward pass or a prediction in between leaves it alone
+    step("surrogate loss after a forward pass")
+    c, p, x, T, T_rd = problem(4)
+    net = sg.Surrogate(params=p, **c)
+    dev = lambda a: torch.tensor(np.asarray(a, np.float32), device="cuda")
+    loss = net.loss_backward(dev(x), dev(T), dev(T_rd))
+    first = loss.item()
+    assert first > 0
+    net.forward(dev(2 * x))
+    net.predict(dev(x))
+    assert loss.item() == first
+    assert net.loss_backward(dev(x), dev(T), dev(T_rd)).item() == pytest.approx(first, rel=1e-6)

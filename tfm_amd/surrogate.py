@@ -274,12 +274,16 @@ class Surrogate:
     def forward(self, x, keep=True):
         """x: [c_in, B L] float32 (cuda). Returns (S [B, L, L], rd [rd_bins, B]) on the device.
         keep: also store what loss_backward reads."""
+        return self._forward(x, keep)
+
+    def _forward(self, x, keep, loss=None):
+        """forward, with the loss (when given) at zero behind it."""
         self._check_input(x, (self.c_in, self.B * self.L), "x")
         N = _nn()
         B, L, W, d = self.B, self.L, self.width, self.d
         s = _stream()
         _ok(N.ccp_nn_input(_p(x), _p(self.xb) if keep else None, _p(self.xt), self.c_in, _up(self.c_in, 16), B * L,
-                           self._ps, _p(self.loss) if keep else None, s), "input")
+                           self._ps, _p(loss), s), "input")
         for k in range(1, self.n_layers + 1):
             _ok(N.ccp_nn_fwd(ctypes.byref(self._fwd[keep, k]), 1, s), "conv")
         _ok(N.ccp_nn_fwd(ctypes.byref(self._fwd[keep, "uv"]), 0, s), "heads")
@@ -309,7 +313,7 @@ class Surrogate:
         s = _stream()
         self._check_input(T, (B, L, L), "T")
         self._check_input(T_rd, (self.rd_bins, B), "T_rd")
-        self.forward(x)
+        self._forward(x, True, self.loss)
         _ok(N.ccp_nn_pair_grad(_p(self.S), _p(T), _p(self.grawb), _p(self._gdist), _p(self._gc0), _p(self.loss), L, Ls,
                                B, w_pair, s), "pair_grad")
         _ok(N.ccp_nn_rd_grad(_p(self.rd), _p(self.p["br"]), _p(T_rd), _p(self.grdb), _p(self.grdt), _p(self.g["br"]),
