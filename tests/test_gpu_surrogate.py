@@ -143,3 +143,44 @@ def test_loss_outlives_a_forward_pass():
     net.predict(dev(x))
     assert loss.item() == first
     assert net.loss_backward(dev(x), dev(T), dev(T_rd)).item() == pytest.approx(first, rel=1e-6)
+
+
+@pytest.mark.parametrize("how", ["entry", "storage", "dict"])
+def test_replaced_tensors_are_the_ones_used(how):
+    # a parameter, gradient or moment given as another tensor (an entry of its
+    # dict, its storage, a whole dict) is what the kernels read and write: two
+    # steps are bit for bit those of a net that was built with the values
+    step(f"surrogate with replaced tensors ({how})")
+    c, p, x, T, T_rd = problem(5)
+    _, q, _, _, _ = problem(6)
+    dev = lambda a: torch.tensor(np.asarray(a, np.float32), device="cuda")
+    want, net = sg.Surrogate(params=q, **c), sg.Surrogate(params=p, **c)
+    given = {}
+    for group in ("p", "g", "m", "v"):
+        new = {k: torch.full((2 * v.numel() + 1,), -9.0, device="cuda")[1:1 + v.numel()].view(v.shape)
+               for k, v in getattr(net, group).items()}
+        for k, t in new.items():
+            t.copy_(getattr(want, group)[k])
+            if how == "entry":
+                getattr(net, group)[k] = t
+            elif how == "storage":
+                getattr(net, group)[k].data = t
+        if how == "dict":
+            setattr(net, group, new)
+        given[group] = new
+    for n in (want, net):
+        n.step(lr=0.0)  # casts the weights
+        n.t = 0
+    for _ in range(2):
+        for n in (want, net):
+            n.zero_grad()
+            n.loss_backward(dev(x), dev(T), dev(T_rd))
+            n.step(lr=3e-3)
+    assert torch.equal(net.forward(dev(x))[0], want.forward(dev(x))[0])
+    for group, new in given.items():
+        for k, t in new.items():
+            assert torch.equal(t, getattr(want, group)[k]), (group, k)
+    assert all(np.array_equal(a, b) for a, b in zip(net.state_dict().values(), want.state_dict().values()))
+    net.p["b1"] = dev(np.zeros(3))
+    with pytest.raises(ValueError, match="b1 must be"):
+        net.predict(dev(x))

@@ -85,16 +85,12 @@ def _nn():
 
 
 def _p(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
-
-
-def _a(t):
-    """Device address of a tensor (None for none), for a structure's field."""
+    """Device address of a tensor (None for none)."""
     return t.data_ptr() if t is not None else None
 
 
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return torch.cuda.current_stream().cuda_stream
 
 
 def _ok(rc, what):
@@ -123,13 +119,24 @@ def _table(structs):
     return torch.frombuffer(bytearray(raw), dtype=torch.uint8).cuda()
 
 
+def _at(tensors, names):
+    """Addresses of the entries of a dict of tensors."""
+    return [tensors[k].data_ptr() for k in names]
+
+
 class Surrogate:
     """Weights (FP32 masters, BF16 copies) and buffers for batches of B
     sequences of L bins with c_in input channels.
 
     The parameters, their gradients and AdamW's moments are views of one flat
     array each, the weight matrices first (they alone decay). include/ccpmi_nn.h
-    gives the layouts of the activations."""
+    gives the layouts of the activations.
+
+    An entry of p, g, m or v may be given another tensor (or another storage):
+    the kernels' arguments hold addresses, so each call compares those it uses
+    with the entries' and takes the new ones. As ever, new weight matrices
+    reach the products at the next step, which casts them. pb is written then
+    for a caller's own products; the network reads its packed copies."""
 
     def __init__(self, c_in=5, width=256, n_layers=6, d=64, L=128, rd_bins=32, B=64, seed=0, params=None):
         self.c_in, self.width, self.n_layers, self.d, self.L, self.rd_bins, self.B = \
@@ -159,17 +166,26 @@ class Surrogate:
         self._flat = [torch.zeros(at, dtype=torch.float32, device=dev) for _ in range(4)]
         view = lambda t: {k: t[off[k]:off[k] + host[k].size].view(host[k].shape) for k in self.names}
         self.p, self.g, self.m, self.v = (view(t) for t in self._flat)
+        self._numel = {k: host[k].size for k in self.names}
+        self._flat_at = [_at(t, self.names) for t in (self.p, self.g, self.m, self.v)]
         for k in self.names:
             self.p[k].copy_(torch.from_numpy(host[k]))
         self.pb = {k: bf16_like(v) for k, v in self.p.items() if k.startswith("W")}
         self.t = 0
-        self._pack_tables()
+        self._alloc_packed()
         self._cast_weights()
         self._alloc(B)
 
-    def _pack_tables(self):
-        """The packed weight copies and the table that fills them."""
-        W, C1, d = self.width, self.c_in, self.d
+    def _own(self, group, names, dtype=torch.float32):
+        """Entries whose addresses go into a kernel's arguments: whole contiguous device arrays."""
+        for k in names:
+            t = group[k]
+            if t.dtype != dtype or not t.is_cuda or not t.is_contiguous() or t.numel() != self._numel[k]:
+                raise ValueError(f"{k} must be a contiguous {dtype} cuda tensor of {self._numel[k]} entries")
+
+    def _alloc_packed(self):
+        """The packed weight copies."""
+        W, C1, d, O = self.width, self.c_in, self.d, self.rd_bins
         h = lambda *s: torch.zeros(s, dtype=torch.int16, device="cuda")
         Cr, Kr, Kd = _up(W, 64), _up(W, 32), _up(d, 32)
         self._wf = {1: h(Cr, 3 * _up(C1, 16))}
@@ -178,19 +194,28 @@ class Surrogate:
             self._wf[k], self._wt[k] = h(Cr, 3 * _up(W, 16)), h(3, Cr, Kr)
         self._wf["u"], self._wf["v"] = h(d, _up(W, 64)), h(d, _up(W, 64))
         self._wt["uv"] = h(2, Cr, Kd)
+        self._wf["r"], self._wt["r"] = h(O, _up(W, 64)), h(Cr, _up(O, 32))
+        self._weights = [k for k in self.names if k.startswith("W")]
+        self._bind_pack()
+
+    def _bind_pack(self):
+        """The table that fills the packed copies from p."""
+        W, C1, d, O = self.width, self.c_in, self.d, self.rd_bins
+        Cr, Kr, Kd = _up(W, 64), _up(W, 32), _up(d, 32)
+        self._own(self.p, self._weights)
+        self._own(self.pb, self._weights, torch.int16)
         tab = []
         for k in range(1, self.n_layers + 1):
             C, wt = (C1, None) if k == 1 else (W, self._wt[k])
-            tab.append(Weight(_a(self.p[f"W{k}"]), _a(self.pb[f"W{k}"]), _a(self._wf[k]), _a(wt), W, C, 3,
+            tab.append(Weight(_p(self.p[f"W{k}"]), _p(self.pb[f"W{k}"]), _p(self._wf[k]), _p(wt), W, C, 3,
                               3 * _up(C, 16), Cr, Kr))
         for j, k in enumerate("uv"):
-            tab.append(Weight(_a(self.p["W" + k]), _a(self.pb["W" + k]), _a(self._wf[k]), _a(self._wt["uv"][j]), d, W,
+            tab.append(Weight(_p(self.p["W" + k]), _p(self.pb["W" + k]), _p(self._wf[k]), _p(self._wt["uv"][j]), d, W,
                               1, _up(W, 64), Cr, Kd))
-        O = self.rd_bins
-        self._wf["r"], self._wt["r"] = h(O, _up(W, 64)), h(Cr, _up(O, 32))
-        tab.append(Weight(_a(self.p["Wr"]), _a(self.pb["Wr"]), _a(self._wf["r"]), _a(self._wt["r"]), O, W, 1,
+        tab.append(Weight(_p(self.p["Wr"]), _p(self.pb["Wr"]), _p(self._wf["r"]), _p(self._wt["r"]), O, W, 1,
                           _up(W, 64), Cr, _up(O, 32)))
         self._pack = _table(tab), len(tab)
+        self._pack_at = _at(self.p, self._weights) + _at(self.pb, self._weights)
 
     def _alloc(self, B):
         self.B = B
@@ -214,18 +239,8 @@ class Surrogate:
         self._bs, self._or, self._cs = Bs, Or, Cs
         self.pooledb, self.pooledt = h(W, Bs), h(B, Cs)
         self.rd = f(self.rd_bins, B)
-        self._fwd = {}
-        for keep in (False, True):
-            for k in range(1, n + 1):
-                first = k == 1
-                self._fwd[keep, k] = FwdArgs(
-                    _a(self._wf[k]), None, _a(self.xt if first else self.ht[k % 2]), _a(self.p[f"b{k}"]),
-                    None if first else _a(self.hs[k % 2]), _a(self.pre[k]) if keep else None,
-                    _a(self.hs[(k + 1) % 2]), _a(self.hb[k]) if keep else None, _a(self.ht[(k + 1) % 2]),
-                    W, W, 3 * _up(self.c_in if first else W, 16), C1s if first else Cs, P, Ps, L, Cs, 0)
-            self._fwd[keep, "uv"] = FwdArgs(
-                _a(self._wf["u"]), _a(self._wf["v"]), _a(self.ht[(n + 1) % 2]), None, None, None, None,
-                _a(self.uvb) if keep else None, _a(self.uvt), 2 * d, d, _up(W, 64), Cs, P, Ps, L, 2 * ds, ds)
+        self._biases = [f"b{k}" for k in range(1, n + 1)]
+        self._bind_forward()
         # backward: every layer keeps its gradient's channel rows for the weight gradients' one launch
         bands, tiles = _nn().ccp_nn_pair_bands(L), (P + 127) // 128
         self.grawb = h(B, L, Ls)
@@ -239,30 +254,61 @@ class Surrogate:
         self._gdist, self._gc0 = f(B * bands, L), f(B * bands)
         self._dbias = {k: f(tiles, W) for k in range(1, n + 1)}
         Cr = _up(W, 64)
-        self._back = {n: BackArgs(_a(self._wt["uv"]), _a(self.duvt), _a(self.dpooled), _a(self.pre[n]), _a(self.dh),
-                                  _a(self.gb[n]), _a(self.gt[n % 2]), _a(self._dbias[n]), W, Cs, Cr, _up(d, 32),
+        self._back = {n: BackArgs(_p(self._wt["uv"]), _p(self.duvt), _p(self.dpooled), _p(self.pre[n]), _p(self.dh),
+                                  _p(self.gb[n]), _p(self.gt[n % 2]), _p(self._dbias[n]), W, Cs, Cr, _up(d, 32),
                                   2 * ds, P, Ps, L, B, ds, int(n > 1))}
         for k in range(n - 1, 0, -1):
-            self._back[k] = BackArgs(_a(self._wt[k + 1]), _a(self.gt[(k + 1) % 2]), None, _a(self.pre[k]), _a(self.dh),
-                                     _a(self.gb[k]), _a(self.gt[k % 2]), _a(self._dbias[k]), W, Cs, Cr, _up(W, 32),
+            self._back[k] = BackArgs(_p(self._wt[k + 1]), _p(self.gt[(k + 1) % 2]), None, _p(self.pre[k]), _p(self.dh),
+                                     _p(self.gb[k]), _p(self.gt[k % 2]), _p(self._dbias[k]), W, Cs, Cr, _up(W, 32),
                                      Cs, P, Ps, L, B, 0, int(k > 1))
+        self._bind_grads()
+
+    def _bind_forward(self):
+        """Arguments of the layers' products, with the biases of p."""
+        W, L, d, n, B = self.width, self.L, self.d, self.n_layers, self.B
+        C1s, Cs, ds, P, Ps = _up(self.c_in, 16), self._cs, self._ds, B * L, self._ps
+        self._own(self.p, self._biases)
+        self._fwd = {}
+        for keep in (False, True):
+            for k in range(1, n + 1):
+                first = k == 1
+                self._fwd[keep, k] = FwdArgs(
+                    _p(self._wf[k]), None, _p(self.xt if first else self.ht[k % 2]), _p(self.p[f"b{k}"]),
+                    None if first else _p(self.hs[k % 2]), _p(self.pre[k]) if keep else None,
+                    _p(self.hs[(k + 1) % 2]), _p(self.hb[k]) if keep else None, _p(self.ht[(k + 1) % 2]),
+                    W, W, 3 * _up(self.c_in if first else W, 16), C1s if first else Cs, P, Ps, L, Cs, 0)
+            self._fwd[keep, "uv"] = FwdArgs(
+                _p(self._wf["u"]), _p(self._wf["v"]), _p(self.ht[(n + 1) % 2]), None, None, None, None,
+                _p(self.uvb) if keep else None, _p(self.uvt), 2 * d, d, _up(W, 64), Cs, P, Ps, L, 2 * ds, ds)
+        self._bias_at = _at(self.p, self._biases)
+
+    def _bind_grads(self):
+        """Tables of the weight gradients and of the sums that go into g."""
+        W, L, d, n, B = self.width, self.L, self.d, self.n_layers, self.B
+        P, Ps, Bs = B * L, self._ps, self._bs
+        bands, tiles = _nn().ccp_nn_pair_bands(L), (P + 127) // 128
+        dev = torch.device("cuda")
+        self._own(self.g, self.names)
         jobs, at = [], [0]
         for k in list(range(1, n + 1)):
             X, C = (self.xb, self.c_in) if k == 1 else (self.hb[k - 1], W)
-            jobs.append(WgradJob(_a(self.gb[k]), _a(X), _a(self.g[f"W{k}"]), None, W, W, C, 3, P, Ps))
-        jobs.append(WgradJob(_a(self.duvb), _a(self.hb[n]), _a(self.g["Wu"]), _a(self.g["Wv"]), 2 * d, d, W, 1,
+            jobs.append(WgradJob(_p(self.gb[k]), _p(X), _p(self.g[f"W{k}"]), None, W, W, C, 3, P, Ps))
+        jobs.append(WgradJob(_p(self.duvb), _p(self.hb[n]), _p(self.g["Wu"]), _p(self.g["Wv"]), 2 * d, d, W, 1,
                              P, Ps))
-        jobs.append(WgradJob(_a(self.grdb), _a(self.pooledb), _a(self.g["Wr"]), None, self.rd_bins, self.rd_bins, W, 1,
+        jobs.append(WgradJob(_p(self.grdb), _p(self.pooledb), _p(self.g["Wr"]), None, self.rd_bins, self.rd_bins, W, 1,
                              B, Bs))
         for j in jobs:
             at.append(at[-1] + _nn().ccp_nn_wgrad_tiles(j.M, j.C))
         self._jobs = _table(jobs), torch.tensor(at, dtype=torch.int32, device=dev), len(jobs), at[-1]
-        seg = [Segment(_a(self._dbias[k]), _a(self.g[f"b{k}"]), W, W, tiles) for k in range(1, n + 1)]
-        seg.append(Segment(_a(self._gdist), _a(self.g["dist"]), L, L, B * bands))
-        seg.append(Segment(_a(self._gc0), _a(self.g["c0"]), 1, 1, B * bands))
+        seg = [Segment(_p(self._dbias[k]), _p(self.g[f"b{k}"]), W, W, tiles) for k in range(1, n + 1)]
+        seg.append(Segment(_p(self._gdist), _p(self.g["dist"]), L, L, B * bands))
+        seg.append(Segment(_p(self._gc0), _p(self.g["c0"]), 1, 1, B * bands))
         self._seg = _table(seg), len(seg)
+        self._grad_at = _at(self.g, self.names)
 
     def _cast_weights(self):
+        if _at(self.p, self._weights) + _at(self.pb, self._weights) != self._pack_at:
+            self._bind_pack()
         _ok(_nn().ccp_nn_pack(_p(self._pack[0]), self._pack[1], _stream()), "pack")
 
     # ------------------------------------------------------------ forward
@@ -281,6 +327,8 @@ class Surrogate:
         self._check_input(x, (self.c_in, self.B * self.L), "x")
         N = _nn()
         B, L, W, d = self.B, self.L, self.width, self.d
+        if _at(self.p, self._biases) != self._bias_at:
+            self._bind_forward()
         s = _stream()
         _ok(N.ccp_nn_input(_p(x), _p(self.xb) if keep else None, _p(self.xt), self.c_in, _up(self.c_in, 16), B * L,
                            self._ps, _p(loss), s), "input")
@@ -304,6 +352,9 @@ class Surrogate:
     # ------------------------------------------------------------ backward
     def zero_grad(self):
         self._flat[1].zero_()
+        for k, at in zip(self.names, self._flat_at[1]):
+            if self.g[k].data_ptr() != at:
+                self.g[k].zero_()
 
     def loss_backward(self, x, T, T_rd, w_pair=1.0, w_rd=1.0):
         """Forward, loss and gradients into self.g; returns the loss (device scalar)."""
@@ -313,6 +364,8 @@ class Surrogate:
         s = _stream()
         self._check_input(T, (B, L, L), "T")
         self._check_input(T_rd, (self.rd_bins, B), "T_rd")
+        if _at(self.g, self.names) != self._grad_at:
+            self._bind_grads()
         self._forward(x, True, self.loss)
         _ok(N.ccp_nn_pair_grad(_p(self.S), _p(T), _p(self.grawb), _p(self._gdist), _p(self._gc0), _p(self.loss), L, Ls,
                                B, w_pair, s), "pair_grad")
@@ -332,9 +385,18 @@ class Surrogate:
 
     def step(self, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8, wd=1e-4):
         self.t += 1
-        p, g, m, v = (_p(t) for t in self._flat)
-        _ok(_nn().ccp_nn_adamw_flat(p, g, m, v, self._flat[0].numel(), self._n_decay, lr, b1, b2, eps, wd, self.t,
-                                    _stream()), "adamw")
+        groups = self.p, self.g, self.m, self.v
+        if [_at(t, self.names) for t in groups] == self._flat_at:
+            p, g, m, v = (_p(t) for t in self._flat)
+            _ok(_nn().ccp_nn_adamw_flat(p, g, m, v, self._flat[0].numel(), self._n_decay, lr, b1, b2, eps, wd, self.t,
+                                        _stream()), "adamw")
+        else:
+            for t in groups:
+                self._own(t, self.names)
+            for k in self.names:
+                p, g, m, v = (_p(t[k]) for t in groups)
+                _ok(_nn().ccp_nn_adamw(p, g, m, v, None, self._numel[k], lr, b1, b2, eps,
+                                       wd if k.startswith("W") else 0.0, self.t, _stream()), "adamw")
         self._cast_weights()
 
     def state_dict(self):
