@@ -2,6 +2,8 @@
 matrix cores against float64 products of the same bfloat16 values, and the
 network's forward pass and every gradient against the numpy oracle with the
 same bfloat16 rounding points; then a short training run."""
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -184,3 +186,33 @@ def test_replaced_tensors_are_the_ones_used(how):
     net.p["b1"] = dev(np.zeros(3))
     with pytest.raises(ValueError, match="b1 must be"):
         net.predict(dev(x))
+
+
+@pytest.mark.parametrize("L,B", [(3, 65536), (16, 65535 + 70)])
+def test_more_samples_than_a_grid_dimension(L, B):
+    # the pair map and its gradients go out in several launches: outputs and
+    # gradients against the oracle, with the tolerances above
+    step(f"surrogate with {B} samples of {L} bins")
+    c = dict(c_in=2, width=8, n_layers=1, d=4, L=L, rd_bins=3, B=B)
+    rng = np.random.default_rng(L)
+    p = so.init_params(c["c_in"], c["width"], c["n_layers"], c["d"], c["L"], c["rd_bins"], seed=2)
+    f32 = lambda a: a.astype(np.float32).astype(np.float64)
+    p = {k: f32(v + 0.05 * rng.normal(size=v.shape)) for k, v in p.items()}
+    # the last samples weigh as much in the loss as all others
+    scale = np.where(np.arange(B) >= 65535, math.sqrt(65535 / (B - 65535)), 1.0)
+    x = f32(rng.normal(size=(c["c_in"], B * L)))
+    T = rng.normal(size=(B, L, L)) * scale[:, None, None]
+    T = f32(0.5 * (T + T.transpose(0, 2, 1)))
+    T_rd = f32(rng.normal(size=(c["rd_bins"], B)))
+    net = sg.Surrogate(params=p, **c)
+    dev = lambda a: torch.tensor(np.asarray(a, np.float32), device="cuda")
+    net.zero_grad()
+    loss = net.loss_backward(dev(x), dev(T), dev(T_rd), w_pair=1.0, w_rd=0.5)
+    want_loss, g, S, rd = so.loss_and_grads(p, x, T, T_rd, B, L, c["n_layers"], 1.0, 0.5, round_bf16=True)
+    got = net.S.cpu().numpy()
+    assert rel(got, S) < 1e-3 and rel(got[65535:], S[65535:]) < 1e-3 and rel(net.rd.cpu().numpy(), rd) < 1e-3
+    assert float(loss.item()) == pytest.approx(want_loss, rel=1e-3)
+    for k in p:
+        err = rel(net.g[k].cpu().numpy(), g[k])
+        step(f"  grad {k}: rel err {err:.2e}")
+        assert err < 2e-2, k

@@ -1191,6 +1191,13 @@ __global__ __launch_bounds__(256) void k_pack(const ccp_nn_weight *tab) {
   }
 }
 
+// launch(first sample, samples) for B samples, as many as a grid's second
+// dimension takes at a time
+template <class F> void in_samples(int B, F &&launch) {
+  constexpr int MOST = 65535;
+  for (int b = 0; b < B; b += MOST) launch((long)b, (unsigned)(B - b < MOST ? B - b : MOST));
+}
+
 // k_adamw over one flat run of parameters, decay on the first n_decay
 __global__ void k_adamw_flat(float *p, const float *g, float *m, float *v, long n, long n_decay, float lr, float b1,
                              float b2, float eps, float wd, float c1, float c2) {
@@ -1307,10 +1314,12 @@ int ccp_nn_fwd(const ccp_nn_fwd_args *a, int conv, void *stream) {
 
 int ccp_nn_pair(const void *uv, int d, const float *dist, const float *c0, float *S, int L, int B, float alpha,
                 void *stream) {
-  if (d <= 0 || d % 16 || L <= 0 || B <= 0 || B > 65535) return 1;
+  if (d <= 0 || d % 16 || L <= 0 || B <= 0) return 1;
   const unsigned nt = (unsigned)((L + 31) / 32);
-  k_pair<<<dim3((nt * nt + 3) / 4, (unsigned)B), 256, 0, (hipStream_t)stream>>>((const uint16_t *)uv, d, 2 * d, dist,
-                                                                               c0, S, L, alpha);
+  in_samples(B, [&](long b, unsigned n) {
+    k_pair<<<dim3((nt * nt + 3) / 4, n), 256, 0, (hipStream_t)stream>>>((const uint16_t *)uv + b * L * 2 * d, d, 2 * d,
+                                                                       dist, c0, S + b * L * L, L, alpha);
+  });
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 
@@ -1333,9 +1342,13 @@ int ccp_nn_pair_bands(int L) { return (L + PL_ROWS - 1) / PL_ROWS; }
 
 int ccp_nn_pair_grad(const float *pred, const float *target, void *graw, float *gdist, float *gc0, float *loss, int L,
                      int Ls, int B, float w, void *stream) {
-  if (L <= 0 || Ls % 8 || Ls < L || B <= 0 || B > 65535) return 1;
-  k_pair_grad<<<dim3((unsigned)ccp_nn_pair_bands(L), (unsigned)B), EW, 0, (hipStream_t)stream>>>(
-      pred, target, (uint16_t *)graw, gdist, gc0, loss, L, Ls, B, w);
+  if (L <= 0 || Ls % 8 || Ls < L || B <= 0) return 1;
+  const int bands = ccp_nn_pair_bands(L);
+  in_samples(B, [&](long b, unsigned n) {
+    k_pair_grad<<<dim3((unsigned)bands, n), EW, 0, (hipStream_t)stream>>>(
+        pred + b * L * L, target + b * L * L, (uint16_t *)graw + b * L * Ls, gdist + b * bands * L, gc0 + b * bands,
+        loss, L, Ls, B, w);
+  });
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 
@@ -1349,12 +1362,13 @@ int ccp_nn_rd_grad(float *pred, const float *bias, const float *target, void *gb
 
 int ccp_nn_duv(const void *uvb, const void *graw, void *db, void *dt, int d, int ds, int L, int Ls, int B, int Ps,
                float alpha, void *stream) {
-  if (d <= 0 || ds % 8 || ds < d || L <= 0 || Ls % 8 || Ls < L || B <= 0 || B > 65535 || Ps % 8 || Ps < (long)B * L)
-    return 1;
-  const unsigned n = (unsigned)((2 * d + 31) / 32 * ((L + 31) / 32));
-  k_duv<<<dim3((n + 3) / 4, (unsigned)B), 256, 0, (hipStream_t)stream>>>((const uint16_t *)uvb, (const uint16_t *)graw,
-                                                                        (uint16_t *)db, (uint16_t *)dt, d, ds, L, Ls,
-                                                                        Ps, 2 * ds, alpha);
+  if (d <= 0 || ds % 8 || ds < d || L <= 0 || Ls % 8 || Ls < L || B <= 0 || Ps % 8 || Ps < (long)B * L) return 1;
+  const unsigned blocks = (unsigned)((2 * d + 31) / 32 * ((L + 31) / 32));
+  in_samples(B, [&](long b, unsigned n) {
+    k_duv<<<dim3((blocks + 3) / 4, n), 256, 0, (hipStream_t)stream>>>(
+        (const uint16_t *)uvb + b * L, (const uint16_t *)graw + b * L * Ls, (uint16_t *)db + b * L,
+        (uint16_t *)dt + b * L * 2 * ds, d, ds, L, Ls, Ps, 2 * ds, alpha);
+  });
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 
