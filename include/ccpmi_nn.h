@@ -118,8 +118,9 @@ int ccp_nn_back(const ccp_nn_back_args *a, int head, void *stream);
 /* Weight gradients of n_jobs products in one launch (tables in device memory):
  * dst[m][taps c + t] += sum over p of G[m, p] X[c, p + t - 1] (taps 3, nothing
  * across a sample's ends) or G[m, p] X[c, p] (taps 1), p < P, rows of Ps (P
- * rounded up to 16, below 2^26, zero beyond P); rows from M0 on go to dst1. first: each job's first tile, jobs in order, ccp_nn_wgrad_tiles of
- * each, n_tiles in all. */
+ * rounded up to 16, below 2^26, zero beyond P); rows from M0 on go to dst1.
+ * first: each job's first tile, jobs in order, ccp_nn_wgrad_tiles of each,
+ * n_tiles in all. */
 typedef struct ccp_nn_wgrad_job {
   const void *G, *X;
   float *dst0, *dst1;
@@ -127,6 +128,8 @@ typedef struct ccp_nn_wgrad_job {
 } ccp_nn_wgrad_job;
 int ccp_nn_wgrad_tiles(int M, int C);
 int ccp_nn_wgrad(const ccp_nn_wgrad_job *tab, const int *first, int n_jobs, int n_tiles, int L, void *stream);
+/* the same where a job's rows have 2^26 entries or more (addresses of 64 bits) */
+int ccp_nn_wgrad_far(const ccp_nn_wgrad_job *tab, const int *first, int n_jobs, int n_tiles, int L, void *stream);
 
 /* dst[i] += sum over parts of src[k stride + i], i < n, for n segments of a
  * table in device memory, in a fixed order */

@@ -216,3 +216,35 @@ def test_more_samples_than_a_grid_dimension(L, B):
         err = rel(net.g[k].cpu().numpy(), g[k])
         step(f"  grad {k}: rel err {err:.2e}")
         assert err < 2e-2, k
+
+
+@pytest.mark.parametrize("taps,L", [(1, 64), (3, 64), (3, 13)])
+@pytest.mark.parametrize("Ps", [96, (1 << 26) + 5 * (1 << 20)])
+def test_weight_gradients_of_long_rows(taps, L, Ps):
+    # rows so long that the last of a tile of 32 lie more than 32 bits of bytes
+    # behind the first: small whole numbers in the first P columns, exact sums
+    step(f"weight gradients, {taps} taps, samples of {L}, rows of {Ps}")
+    M, C, P = 33, 34, 64
+    rng = np.random.default_rng(taps * L)
+    far = Ps >= 1 << 26
+    G, X = (torch.empty((n, Ps), dtype=torch.int16, device="cuda") for n in (M, C))
+    g, x = rng.integers(-4, 5, (M, P)).astype(float), rng.integers(-4, 5, (C, P)).astype(float)
+    for t, v in ((G, g), (X, x)):
+        t[:, :96] = 0
+        t[:, :P] = to_bf16_dev(v)[0]
+    dst = torch.full((M, taps * C), 3.0, device="cuda")
+    nn = sg._nn()
+    n_tiles = nn.ccp_nn_wgrad_tiles(M, C)
+    tab = sg._table([sg.WgradJob(G.data_ptr(), X.data_ptr(), dst.data_ptr(), None, M, M, C, taps, P, Ps)])
+    first = torch.tensor([0, n_tiles], dtype=torch.int32, device="cuda")
+    run = nn.ccp_nn_wgrad_far if far else nn.ccp_nn_wgrad
+    assert run(tab.data_ptr(), first.data_ptr(), 1, n_tiles, L, sg._stream()) == 0
+    want = np.full((M, C, taps), 3.0)
+    for t in range(taps):
+        for p in range(P):
+            q = p + t - 1 if taps == 3 else p
+            if 0 <= q < P and q // L == p // L:
+                want[:, :, t] += np.outer(g[:, p], x[:, q])
+    assert np.array_equal(dst.cpu().numpy(), want.reshape(M, taps * C))
+    del G, X
+    torch.cuda.empty_cache()

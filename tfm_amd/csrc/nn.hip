@@ -1023,16 +1023,17 @@ typedef __attribute__((address_space(1))) uint16_t global_u16;
 typedef __attribute__((address_space(1))) float global_f32;
 typedef __attribute__((address_space(1))) u32x4 global_u32x4;
 __device__ __forceinline__ uint32_t other_half(uint32_t v) { return (uint32_t)__shfl_xor((int)v, 32); }
-// ALIGNED: samples of a multiple of 8 positions
-template <int TAPS, bool ALIGNED>
+// ALIGNED: samples of a multiple of 8 positions. OFF: the lane's byte offset
+// from a tile's first row, 32 bits on a scalar base so that a load needs no
+// address arithmetic, while 31 rows lie within them (Ps below 2^26)
+template <int TAPS, bool ALIGNED, class OFF>
 __device__ __forceinline__ void wgrad_tile(const ccp_nn_wgrad_job &J, int m0, int c0, int L) {
   const int P = J.P, Ps = J.Ps;
   const int lane = threadIdx.x, r = lane & 31, half = lane >> 5;
-  // this lane's byte offset from the tile's first row of each matrix (rows past
-  // the last: its values, for results that are not stored); a 32-bit offset on
-  // a scalar base, so that a load needs no address arithmetic
-  const uint32_t go = ((uint32_t)(min(m0 + r, J.M - 1) - m0) * (uint32_t)Ps + 8u * half) * 2u;
-  const uint32_t xo = ((uint32_t)(min(c0 + r, J.C - 1) - c0) * (uint32_t)Ps + 8u * half) * 2u;
+  // this lane's offset from the tile's first row of each matrix (rows past the
+  // last: its values, for results that are not stored)
+  const OFF go = ((OFF)(min(m0 + r, J.M - 1) - m0) * (OFF)Ps + 8u * half) * 2u;
+  const OFF xo = ((OFF)(min(c0 + r, J.C - 1) - c0) * (OFF)Ps + 8u * half) * 2u;
   const global_u16 *G = (const global_u16 *)J.G + (long)m0 * Ps, *X = (const global_u16 *)J.X + (long)c0 * Ps;
   union Frag {
     u32x4 u;
@@ -1116,6 +1117,7 @@ __device__ __forceinline__ void wgrad_tile(const ccp_nn_wgrad_job &J, int m0, in
       if (m < J.M) d[n + t] = acc[t][v] + old[t][v];
     }
 }
+template <class OFF>
 __global__ __launch_bounds__(64) void k_wgrad(const ccp_nn_wgrad_job *tab, const int *first, int n_jobs, int L) {
   // Workgroups go round-robin over the 8 XCDs: each XCD takes a run of tiles,
   // so the rows that a layer's tiles share stay in one or two L2s.
@@ -1126,9 +1128,9 @@ __global__ __launch_bounds__(64) void k_wgrad(const ccp_nn_wgrad_job *tab, const
   const ccp_nn_wgrad_job J = tab[job];
   const int nc = (J.C + 31) / 32, tile = bid - first[job];
   const int m0 = tile / nc * 32, c0 = tile % nc * 32;
-  if (J.taps == 1) wgrad_tile<1, true>(J, m0, c0, L);
-  else if (L % 8 == 0) wgrad_tile<3, true>(J, m0, c0, L);
-  else wgrad_tile<3, false>(J, m0, c0, L);
+  if (J.taps == 1) wgrad_tile<1, true, OFF>(J, m0, c0, L);
+  else if (L % 8 == 0) wgrad_tile<3, true, OFF>(J, m0, c0, L);
+  else wgrad_tile<3, false, OFF>(J, m0, c0, L);
 }
 
 // dst[i] += sum over parts of src[s stride + i], for every segment of the
@@ -1387,7 +1389,13 @@ int ccp_nn_wgrad_tiles(int M, int C) { return (M + 31) / 32 * ((C + 31) / 32); }
 
 int ccp_nn_wgrad(const ccp_nn_wgrad_job *tab, const int *first, int n_jobs, int n_tiles, int L, void *stream) {
   if (!tab || !first || n_jobs <= 0 || n_tiles <= 0 || L <= 0) return 1;
-  k_wgrad<<<(unsigned)n_tiles, 64, 0, (hipStream_t)stream>>>(tab, first, n_jobs, L);
+  k_wgrad<uint32_t><<<(unsigned)n_tiles, 64, 0, (hipStream_t)stream>>>(tab, first, n_jobs, L);
+  return hipGetLastError() == hipSuccess ? 0 : 2;
+}
+
+int ccp_nn_wgrad_far(const ccp_nn_wgrad_job *tab, const int *first, int n_jobs, int n_tiles, int L, void *stream) {
+  if (!tab || !first || n_jobs <= 0 || n_tiles <= 0 || L <= 0) return 1;
+  k_wgrad<uint64_t><<<(unsigned)n_tiles, 64, 0, (hipStream_t)stream>>>(tab, first, n_jobs, L);
   return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 

@@ -26,8 +26,8 @@ NN_EXPORTS = (
     "ccp_nn_gemm", "ccp_nn_im2col", "ccp_nn_col2im", "ccp_nn_bias_gelu", "ccp_nn_gelu_back", "ccp_nn_pair_map",
     "ccp_nn_pair_loss", "ccp_nn_mean_pool", "ccp_nn_pool_back", "ccp_nn_rd_loss", "ccp_nn_cast_bf16", "ccp_nn_adamw",
     "ccp_nn_input", "ccp_nn_fwd", "ccp_nn_pair", "ccp_nn_pool", "ccp_nn_small", "ccp_nn_pair_bands", "ccp_nn_pair_grad",
-    "ccp_nn_rd_grad", "ccp_nn_duv", "ccp_nn_back", "ccp_nn_wgrad_tiles", "ccp_nn_wgrad", "ccp_nn_reduce", "ccp_nn_pack",
-    "ccp_nn_adamw_flat",
+    "ccp_nn_rd_grad", "ccp_nn_duv", "ccp_nn_back", "ccp_nn_wgrad_tiles", "ccp_nn_wgrad", "ccp_nn_wgrad_far", "ccp_nn_reduce",
+    "ccp_nn_pack", "ccp_nn_adamw_flat",
 )
 
 
@@ -76,7 +76,7 @@ def _nn():
         L.ccp_nn_duv.argtypes = [vp, vp, vp, vp, i, i, i, i, i, i, f, vp]
         L.ccp_nn_back.argtypes = [vp, i, vp]
         L.ccp_nn_wgrad_tiles.argtypes = [i, i]
-        L.ccp_nn_wgrad.argtypes = [vp, vp, i, i, i, vp]
+        L.ccp_nn_wgrad.argtypes = L.ccp_nn_wgrad_far.argtypes = [vp, vp, i, i, i, vp]
         L.ccp_nn_reduce.argtypes = [vp, i, vp]
         L.ccp_nn_pack.argtypes = [vp, i, vp]
         L.ccp_nn_adamw_flat.argtypes = [vp, vp, vp, vp, lg, lg, f, f, f, f, f, i, vp]
@@ -378,8 +378,8 @@ class Surrogate:
                          1.0 / math.sqrt(d), s), "duv")
         for k in range(n, 0, -1):
             _ok(N.ccp_nn_back(ctypes.byref(self._back[k]), int(k == n), s), "back")
-        _ok(N.ccp_nn_wgrad(_p(self._jobs[0]), _p(self._jobs[1]), self._jobs[2], self._jobs[3], L, s),
-            "wgrad")
+        wgrad = N.ccp_nn_wgrad if Ps < 1 << 26 else N.ccp_nn_wgrad_far
+        _ok(wgrad(_p(self._jobs[0]), _p(self._jobs[1]), self._jobs[2], self._jobs[3], L, s), "wgrad")
         _ok(N.ccp_nn_reduce(_p(self._seg[0]), self._seg[1], s), "reduce")
         return self.loss
 
