@@ -159,3 +159,16 @@ def test_half_cell_batches_above_the_tested_size_are_refused():
     shapes = autotune.candidates(2.5, sum(s["n_beads"] for s in systems))
     assert {"lanes_per_bead": 8, "cell_reach": 2, "cell_size": 1.25} not in shapes and len(shapes) == 5
     assert len(autotune.candidates(2.5, 524288)) == 6
+
+
+def test_batches_take_no_default_shape_of_ccp_field():
+    # systems run the WCA/LJ set on one shared cell side: "force_field ccp" in
+    # the common text must not bring in the cells that ccp's field would choose
+    # for each nucleus on its own
+    systems = [dict(n_beads=n, volume_fraction=v, eps_het=0.6, eps_lam=1.0, het_fraction=0.3, lad_fraction=0.1,
+                    seed=7) for n, v in ((4000, 0.3), (700, 0.2), (1500, 0.1))]
+    lay = tfm_amd.batch_layout(systems, {"timestep": 0.001, "force_field": "ccp"})
+    for k, s in enumerate(systems):
+        rco = float(np.float32(1.154701))
+        R_n = np.float32(float(f"{rco / 2 + rco / 2 * (s['n_beads'] / s['volume_fraction']) ** (1 / 3):.6f}"))
+        assert lay["cell_offsets"][k + 1] - lay["cell_offsets"][k] == (2 * int(np.ceil(R_n / np.float32(2.0)))) ** 3

@@ -488,6 +488,7 @@ void plan_batch(ccp_batch &bt, const char *common_params, const ccp_batch_system
     // the system's own configuration gives its geometry and constants
     ccp_sim one;
     one.log_fn = quiet;
+    one.in_batch = true;
     ParMap par(b->text.back().c_str());
     one.configure(par);
     one.fill_kparams();

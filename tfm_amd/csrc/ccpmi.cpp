@@ -154,7 +154,7 @@ void ccp_sim::configure(const ParMap &par) {
   // the buckets take 512 bytes a cell, so nuclei with fewer beads for their
   // size keep the wide cells, a fifth as many.
   // Above HALF_CELL_BATCH_LIMIT beads the shape has not run.
-  if (!lj && !split) {
+  if (!lj && !split && !in_batch) {
     bool plain = true;
     for (const char *k : {"lanes_per_bead", "cell_reach", "cell_size", "fine_cell_size", "cell_capacity",
                           "integrate_pass", "group_types", "bal_rounds", "type_order"})

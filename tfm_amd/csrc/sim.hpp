@@ -114,6 +114,7 @@ struct ccp_sim {
   float csl = 0;   // coarse cell side: het grid and ccp-layout export grid
   float csl_f = 0; // cell side of the all-bead grid of the step (fine when split)
   float dmin_max = 0; // largest overlap distance: fine_cell_size (cell_size when not split)
+  bool in_batch = false; // configured as a system of a batch, whose systems share one cell side
   bool split = false; // short-range pairs on the fine grid + het-het tail on the het grid
   std::vector<uint32_t> chain_off;
   std::string seq_file;
