@@ -195,3 +195,28 @@ def test_frame_contact_map_lists(N, scale, pixels):
     assert lib.ccp_frame_contact_map(sim.h, ptr(got, tfm_amd.ccp.ctypes.c_float), lcm) == 0
     assert np.array_equal(got, want)
     sim.close()
+
+
+@pytest.mark.parametrize("N,scale", [(140000, 1.0), (140000, 0.01), (340000, 1.0), (340002, 1.0)])
+def test_distance_contact_long_chain(N, scale):
+    # more contacts at a separation than 2^27 / 1000: ccp's FP32 sum of 1000 per
+    # contact rounds at each addition from there on (bonded neighbours, and
+    # every separation of the shrunk chain), against sums in order in numpy; and
+    # both sides of 170000 separations, above which a lane takes each
+    step(f"d(s), P(s) N={N} scale={scale}")
+    R_n = radius_for(N, 0.2)
+    sim = sim_with(N, R_n, walk(N, R_n, seed=6) * np.float32(scale), np.zeros(N, np.uint8))
+    r = sim.positions
+    sd, cp = sim.distance_contact(0)
+    assert len(sd) == N // 2
+    over = 0
+    for s in (1, 2, 3, 8, 9, 112, 5000, N // 2 - 1, N // 2):
+        d = r[s:] - r[:-s]
+        d = np.sqrt((d[:, 0] * d[:, 0] + d[:, 1] * d[:, 1]) + d[:, 2] * d[:, 2])
+        a = np.add.accumulate(d, dtype=np.float32)[-1] / np.float32(N - s)
+        hit = np.where(d < np.float32(2.0), np.float32(1000.0), np.float32(0.0))
+        c = np.add.accumulate(hit, dtype=np.float32)[-1] / np.float32(N - s)
+        over += int((d < 2.0).sum() > 134217)
+        assert sd[s - 1] == a and cp[s - 1] == c, s
+    assert over >= (1 if scale == 1.0 else 6)
+    sim.close()

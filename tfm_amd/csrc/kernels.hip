@@ -2041,6 +2041,18 @@ __global__ __launch_bounds__(BEAD_BLOCK) void k_radial_batch(const SysParams *sy
       if (s_acc[k] != 0.0) atomicAdd(out + (size_t)first * n_b + k, s_acc[k]);
 }
 
+// ccp's FP32 sum of 1000 per contact, a function of their number n alone: the
+// whole number while it is at most 2^24 times 8 (the largest power of two in
+// 1000), and from there on rounded at each addition
+__device__ __forceinline__ float contact_sum(uint32_t n) {
+#pragma clang fp contract(off)
+  constexpr uint32_t EXACT = (1u << 27) / 1000u;
+  float c = (float)(1000u * min(n, EXACT));
+#pragma unroll 16
+  for (uint32_t k = EXACT; k < n; ++k) c += 1000.0f;
+  return c;
+}
+
 // ccp's d(s) and 1000 P(s) of one or several chromosomes (calc_sd_cp,
 // chrana.cu:13-45): FP32 sums over the pairs (p, p+s) of beads [i_s, i_e)
 // and, when N = 30386, of the homologue N/2 further on, for every separation
@@ -2115,39 +2127,25 @@ __global__ __launch_bounds__(SD_THREADS) void k_sd_cp(const float4 *__restrict__
   __syncthreads();
   if (wid > 0) distances(0u);
   __syncthreads();
-  // ccp adds 1000 per contact in FP32: exact, whatever the order, while the
-  // sum is at most 2^24 times 8 (the largest power of two in 1000)
-  const bool counts = ncc * (J.i_e - J.i_s) <= (1u << 27) / 1000u;
-  float a = 0.0f, c = 0.0f;
+  float a = 0.0f;
   // the additions are the long chain: their wavefront goes first on its SIMD
   if (wid == 0) __builtin_amdgcn_s_setprio(3);
   for (uint32_t t = 0; t < tiles; ++t) {
     if (wid == 0) {
       const float(*d)[SD_S] = s_d[t & 1u];
-      if (counts) {
-        // the next sixteen are read while these are added
-        float x[16];
+      // the next sixteen are read while these are added
+      float x[16];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) x[r] = d[r][lane % SD_S];
+      for (int r = 0; r < 16; ++r) x[r] = d[r][lane % SD_S];
 #pragma unroll
-        for (int r0 = 0; r0 < SD_P; r0 += 16) {
-          float y[16];
+      for (int r0 = 0; r0 < SD_P; r0 += 16) {
+        float y[16];
 #pragma unroll
-          for (int r = 0; r < 16; ++r) y[r] = d[min(r0 + 16, SD_P - 16) + r][lane % SD_S];
+        for (int r = 0; r < 16; ++r) y[r] = d[min(r0 + 16, SD_P - 16) + r][lane % SD_S];
 #pragma unroll
-          for (int r = 0; r < 16; ++r) a += x[r];
+        for (int r = 0; r < 16; ++r) a += x[r];
 #pragma unroll
-          for (int r = 0; r < 16; ++r) x[r] = y[r];
-        }
-      } else {
-        const uint32_t q = (t % per) * SD_P; // first starting bead of the tile, from the chromosome's first
-        for (int r = 0; r < SD_P; ++r) {
-          const float x = d[r][lane % SD_S];
-          if (q + (uint32_t)r + s < J.i_e - J.i_s) {
-            a += x;
-            if (x < 2.0f) c += 1000.0f;
-          }
-        }
+        for (int r = 0; r < 16; ++r) x[r] = y[r];
       }
     } else {
       float4 next = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -2163,7 +2161,43 @@ __global__ __launch_bounds__(SD_THREADS) void k_sd_cp(const float4 *__restrict__
   __syncthreads();
   if (tid >= SD_S || s > J.lsdcp) return;
   const uint32_t ia = s - 1u;
-  if (counts) c = (float)(1000u * s_n[tid]);
+  const float m = (float)(ncc * (J.i_e - J.i_s - s));
+  a /= m;
+  const float c = contact_sum(s_n[tid]) / m;
+  if (J.sd) {
+    J.sd[ia] = a;
+    J.cp[ia] = c;
+  }
+  if (J.sum_sd) {
+    J.sum_sd[ia] += (double)a;
+    J.sum_cp[ia] += (double)c;
+  }
+}
+
+// The same with one lane a separation, for chromosomes of so many of them that
+// lanes fill the chip by themselves: the tiles' detour through LDS then only
+// costs. One chain of 131072, 200000 and 400000 beads: tiles 7.8, 18.0 and 71.6
+// ms, lanes 22.7, 31.0 and 62.4; they cross at about 340000 beads.
+constexpr uint32_t SD_LANES = 170000; // separations
+__global__ __launch_bounds__(BEAD_BLOCK) void k_sd_cp_lanes(const float4 *pos, uint32_t N, SdCpJob J) {
+#pragma clang fp contract(off)
+  const uint32_t ia = blockIdx.x * BEAD_BLOCK + threadIdx.x;
+  if (ia >= J.lsdcp) return;
+  const uint32_t s = ia + 1u, ncc = (N == 30386u) ? 2u : 1u;
+  uint32_t i_s = J.i_s, i_e = J.i_e;
+  float a = 0.0f, c = 0.0f;
+  for (uint32_t k = 0; k < ncc; ++k) {
+    for (uint32_t p = i_s; p < i_e - s; ++p) {
+      const float4 u = pos[p], v = pos[p + s];
+      const float dx = v.x - u.x, dy = v.y - u.y, dz = v.z - u.z;
+      const float xx = dx * dx, yy = dy * dy, zz = dz * dz;
+      const float d = sqrtf((xx + yy) + zz);
+      a += d;
+      if (d < 2.0f) c += 1000.0f;
+    }
+    i_s += N / ncc;
+    i_e += N / ncc;
+  }
   const float m = (float)(ncc * (J.i_e - J.i_s - s));
   a /= m;
   c /= m;
@@ -2507,7 +2541,9 @@ void launch_sd_cp(hipStream_t s, const float4 *pos, uint32_t N, const SdCpJob *j
   SdCpJobs all{};
   uint32_t n = 0, longest = 0;
   for (int k = 0; k < n_jobs; ++k)
-    if (jobs[k].lsdcp) {
+    if (jobs[k].lsdcp > SD_LANES) {
+      k_sd_cp_lanes<<<blocks_for((int)jobs[k].lsdcp, BEAD_BLOCK), BEAD_BLOCK, 0, s>>>(pos, N, jobs[k]);
+    } else if (jobs[k].lsdcp) {
       all.job[n++] = jobs[k];
       longest = jobs[k].lsdcp > longest ? jobs[k].lsdcp : longest;
     }
