@@ -220,3 +220,15 @@ def test_distance_contact_long_chain(N, scale):
         assert sd[s - 1] == a and cp[s - 1] == c, s
     assert over >= (1 if scale == 1.0 else 6)
     sim.close()
+
+
+@pytest.mark.parametrize("N,scale", [(1000, 0.3), (4095, 0.3), (4096, 0.3), (4100, 1.0), (4124, 1.0), (4128, 0.3),
+                                     (4132, 1.0), (6000, 0.1)])
+def test_frame_contact_map_rows_of_a_block(N, scale):
+    # one row a block below 1024 rows and eight from there on, whole and ragged
+    # last blocks, with few and with many pixels in contact
+    step(f"frame contact map N={N} scale={scale}")
+    R_n = radius_for(N, 0.3)
+    sim = sim_with(N, R_n, walk(N, R_n, seed=N) * np.float32(scale), np.zeros(N, np.uint8))
+    assert np.array_equal(sim.frame_contact_map(), po.ccp_contact_map(sim.positions))
+    sim.close()

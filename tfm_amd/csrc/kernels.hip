@@ -2219,8 +2219,8 @@ __global__ __launch_bounds__(BEAD_BLOCK) void k_sd_cp_lanes(const float4 *pos, u
 //
 // sqrtf(x) < 2 and x < 4 select the same FP32 values x (the root is rounded
 // correctly, and the root of the largest float below 4 rounds below 2).
-__device__ __forceinline__ float cm_pixel(const float4 *__restrict__ pos, uint32_t N, uint32_t ncc, uint32_t ix,
-                                          uint32_t iy) {
+__device__ __forceinline__ uint32_t cm_pixel(const float4 *__restrict__ pos, uint32_t N, uint32_t ncc, uint32_t ix,
+                                             uint32_t iy) {
 #pragma clang fp contract(off)
   uint32_t n = 0;
   for (uint32_t c = 0; c < ncc; ++c) {
@@ -2234,8 +2234,7 @@ __device__ __forceinline__ float cm_pixel(const float4 *__restrict__ pos, uint32
         n += ((xx + yy) + zz) < 4.0f ? 1u : 0u;
       }
   }
-  // whole thousands of at most 32 contacts: exact in FP32, as ccp's sum of them
-  return (float)(1000u * n) / (float)(ncc * 16u);
+  return n;
 }
 
 // First bead and the distance of the farthest of a pixel's other three, with
@@ -2261,70 +2260,127 @@ __device__ __forceinline__ bool cm_apart(float4 a, float4 b) {
   return dist2(a.x - b.x, a.y - b.y, a.z - b.z) > t * t;
 }
 
-// One lane per column pixel of a block of CM_COLS columns x CM_ROWS rows. A
-// packed row is contiguous, so the stores are coalesced, and a column's
-// bound is loaded once for CM_ROWS pixels. Nearly every pixel is empty (a
-// contact reaches 2 sigma in a nucleus of tens), so the test of the bounds
-// decides all but a few per cent of the wavefronts' pixels; one lane per
-// packed pixel evaluating its 32 pairs took 253 us at N = 30386 (7.2 M pixels);
-// this takes 68 us, 16 rows a block (111 us with 64: a block with contacts then
-// holds up the launch).
+// Contacts of the pixel of the four beads u (in registers) and v.
+__device__ __forceinline__ uint32_t cm_pairs(const float4 u[4], const float4 *v) {
+#pragma clang fp contract(off)
+  uint32_t n = 0;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float4 o = v[q];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const float dx = o.x - u[p].x, dy = o.y - u[p].y, dz = o.z - u[p].z;
+      const float xx = dx * dx, yy = dy * dy, zz = dz * dz;
+      n += ((xx + yy) + zz) < 4.0f ? 1u : 0u;
+    }
+  }
+  return n;
+}
+
+// One lane per column pixel of a block of CM_COLS columns x ROWS rows. A
+// packed row is contiguous, so the stores are coalesced, and a column's beads
+// and bound are loaded once for ROWS pixels, the rows' once for a block. Nearly
+// every pixel is empty (a contact reaches 2 sigma in a nucleus of tens), so the
+// test of the bounds decides all but a few per cent of the wavefronts' pixels;
+// one lane per packed pixel evaluating its 32 pairs took 253 us at N = 30386
+// (7.2 M pixels); this takes 72 us, 8 rows a block (171, 94, 78 and 78 us with
+// 1, 2, 4 and 16; medians over maps of 1 % to all pixels). Maps of less than 1024 rows leave most of the chip idle and
+// take one row a block: 3.7 us for 16 rows, 5.7 for 100 (8 rows: 10.5, 12.4).
 //
 // The map goes to `cm`, or its nonzero pixels (index, bits of the value) to
-// `list`, whose first entry counts them; those past `cap` are only counted.
-constexpr int CM_COLS = 256, CM_ROWS = 16;
+// `list`, whose first entry counts them; those past `cap` are only counted. A
+// lane keeps its rows' contacts, a byte each, and a block takes its entries
+// with one atomic: with one for each wavefront's row, and pixels that loaded
+// their beads, a full map of 7.2 M pixels took 3.15 ms instead of 1.9.
+constexpr int CM_COLS = 256, CM_ROWS = 8;
+template <int ROWS>
 __global__ __launch_bounds__(CM_COLS) void k_ccp_cm(uint32_t N, uint32_t cms, uint32_t lcm,
                                                     const float4 *__restrict__ pos, float *cm, double *sum,
                                                     uint2 *list, uint32_t cap) {
-  const uint32_t col0 = blockIdx.x * CM_COLS, row0 = blockIdx.y * CM_ROWS;
-  if (col0 > row0 + CM_ROWS - 1u) return;
+  static_assert(ROWS <= 8, "a lane keeps a byte for each of its rows");
+  const uint32_t col0 = blockIdx.x * CM_COLS, row0 = blockIdx.y * ROWS;
+  if (col0 > row0 + ROWS - 1u) return;
   const uint32_t ncc = (N == 30386u) ? 2u : 1u;
-  __shared__ float4 s_row[2][CM_ROWS];
-  for (uint32_t k = threadIdx.x; k < ncc * CM_ROWS; k += CM_COLS) {
-    const uint32_t c = k / CM_ROWS, r = min(row0 + k % CM_ROWS, cms - 1u);
-    s_row[c][k % CM_ROWS] = cm_bound(pos + c * (N / ncc) + 4u * r);
-  }
-  const uint32_t col = col0 + threadIdx.x;
-  float4 mine[2];
+  __shared__ float4 s_row[2][ROWS], s_bead[2][ROWS][4];
+  __shared__ uint32_t s_sum[CM_COLS / 64], s_base;
+  const uint32_t tid = threadIdx.x;
+  if (tid < ncc * ROWS) {
+    const uint32_t c = tid / ROWS, k = tid % ROWS;
+    const float4 *p = pos + c * (N / ncc) + 4u * min(row0 + k, cms - 1u);
+    s_row[c][k] = cm_bound(p);
 #pragma unroll
-  for (uint32_t c = 0; c < 2u; ++c)
-    mine[c] = cm_bound(pos + (c < ncc ? c : 0u) * (N / ncc) + 4u * min(col, cms - 1u));
+    for (int q = 0; q < 4; ++q) s_bead[c][k][q] = p[q];
+  }
+  const uint32_t col = col0 + tid;
+  float4 mine[2], bead[2][4];
+#pragma unroll
+  for (uint32_t c = 0; c < 2u; ++c) {
+    const float4 *p = pos + (c < ncc ? c : 0u) * (N / ncc) + 4u * min(col, cms - 1u);
+    mine[c] = cm_bound(p);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) bead[c][q] = p[q];
+  }
   __syncthreads();
-  for (uint32_t k = 0; k < (uint32_t)CM_ROWS; ++k) {
+  // whole thousands of at most 32 contacts over 16 or 32 pairs: exact in FP32,
+  // as ccp's sum of them and its quotient
+  const float unit = ncc == 2u ? 1.0f / 32.0f : 1.0f / 16.0f;
+  uint64_t kept = 0;
+  for (uint32_t k = 0; k < (uint32_t)ROWS; ++k) {
     const uint32_t row = row0 + k;
     if (row >= cms) break;
     if (col > row) continue;
     const uint32_t ia = (uint32_t)((uint64_t)row * (row + 1u) / 2u) + col;
-    uint32_t ix = row, iy = col;
     // ccp finds the row as an FP32 root of the packed index, which near a
     // row's ends may round to a neighbouring row (by less than 0.008 of the
     // row's length up to 65535 rows). The pixels close to an end take ccp's
     // row and column; the clamps keep the reads inside the chain where the
     // root would round past the last row.
     const float edge = 0.01f * (float)(row + 1u) + 1.0f;
+    uint32_t ix = row, iy = col;
     if ((float)col < edge || (float)(row - col) < edge) {
       ix = min((uint32_t)((double)sqrtf((float)(2.0 * ia + 0.25)) - 0.5), cms - 1u);
       iy = min((uint32_t)(ia - ix * (ix + 1.0) / 2.0), cms - 1u);
     }
-    const bool as_packed = ix == row && iy == col;
-    bool apart = cm_apart(mine[0], s_row[0][k]);
-    if (ncc == 2u) apart = apart && cm_apart(mine[1], s_row[1][k]);
-    float v = 0.0f;
-    if (!(as_packed && apart)) v = cm_pixel(pos, N, ncc, ix, iy);
-    if (cm) cm[ia] = v;
-    if (list) {
-      // one atomic for the pixels of a wavefront
-      const uint64_t hit = __ballot(v != 0.0f);
-      if (v != 0.0f) {
-        const uint32_t before = (uint32_t)__popcll(hit & ((1ull << __lane_id()) - 1ull));
-        uint32_t at = 0;
-        if (before == 0u) at = atomicAdd(&list[0].x, (uint32_t)__popcll(hit));
-        at = __builtin_amdgcn_readfirstlane(at) + before;
-        if (at < cap) list[1u + at] = make_uint2(ia, __float_as_uint(v));
+    uint32_t n = 0;
+    if (ix == row && iy == col) {
+      bool apart = cm_apart(mine[0], s_row[0][k]);
+      if (ncc == 2u) apart = apart && cm_apart(mine[1], s_row[1][k]);
+      if (!apart) {
+        n = cm_pairs(bead[0], s_bead[0][k]);
+        if (ncc == 2u) n += cm_pairs(bead[1], s_bead[1][k]);
       }
+    } else {
+      n = cm_pixel(pos, N, ncc, ix, iy);
     }
+    const float v = (float)(1000u * n) * unit;
+    if (cm) cm[ia] = v;
+    kept |= (uint64_t)n << (8u * k);
     // (an empty pixel adds nothing)
     if (sum && v != 0.0f) sum[ia] += (double)v;
+  }
+  if (!list) return;
+  uint32_t count = 0;
+  for (uint32_t k = 0; k < (uint32_t)ROWS; ++k)
+    count += ((uint32_t)(kept >> (8u * k)) & 255u) ? 1u : 0u;
+  const uint32_t incl = wave_incl_scan(count);
+  if (__lane_id() == 63) s_sum[tid >> 6] = incl;
+  __syncthreads();
+  uint32_t at = incl - count, total = 0;
+#pragma unroll
+  for (uint32_t w = 0; w < CM_COLS / 64; ++w) {
+    at += w < tid >> 6 ? s_sum[w] : 0u;
+    total += s_sum[w];
+  }
+  if (tid == 0) s_base = total ? atomicAdd(&list[0].x, total) : 0u;
+  __syncthreads();
+  at += s_base;
+  if (count == 0u) return;
+  for (uint32_t k = 0; k < (uint32_t)ROWS; ++k) {
+    const uint32_t n = (uint32_t)(kept >> (8u * k)) & 255u, row = row0 + k;
+    if (n == 0u) continue;
+    const uint32_t ia = (uint32_t)((uint64_t)row * (row + 1u) / 2u) + col;
+    if (at < cap) list[1u + at] = make_uint2(ia, __float_as_uint((float)(1000u * n) * unit));
+    ++at;
   }
 }
 
@@ -2559,8 +2615,12 @@ void launch_list_words(hipStream_t s, const uint32_t *map, uint32_t n, uint2 *li
 void launch_ccp_cm(hipStream_t s, uint32_t N, uint32_t cms, uint32_t lcm, const float4 *pos, float *cm, double *sum,
                    uint2 *list, uint32_t cap) {
   if (lcm == 0) return;
-  k_ccp_cm<<<dim3((cms + CM_COLS - 1) / CM_COLS, (cms + CM_ROWS - 1) / CM_ROWS), CM_COLS, 0, s>>>(N, cms, lcm, pos,
-                                                                                                cm, sum, list, cap);
+  const unsigned cols = (cms + CM_COLS - 1) / CM_COLS;
+  if (cms < 1024)
+    k_ccp_cm<1><<<dim3(cols, cms), CM_COLS, 0, s>>>(N, cms, lcm, pos, cm, sum, list, cap);
+  else
+    k_ccp_cm<CM_ROWS><<<dim3(cols, (cms + CM_ROWS - 1) / CM_ROWS), CM_COLS, 0, s>>>(N, cms, lcm, pos, cm, sum, list,
+                                                                                  cap);
 }
 
 void launch_bin_batch(hipStream_t s, const SysParams *sys, const uint32_t *sys_slot, int n_sys, int n,
