@@ -257,3 +257,32 @@ def test_batch_scan_blocks_at_system_edges(size):
         assert np.array_equal(m, maps[s][:len(m), :len(m)]), s
         sim.close()
     b.close()
+
+
+@pytest.mark.parametrize("n_empty", [12, 13])
+def test_batch_scan_blocks_of_two_cells_a_lane(n_empty):
+    # the sizes above among systems of a few beads in a large nucleus, on either
+    # side of 2^20 cells: each system's positions and contact map equal the
+    # single run's
+    systems = [dict(n_beads=n, volume_fraction=v, eps_het=0.6, eps_lam=1.0, het_fraction=0.3, lad_fraction=0.1,
+                    seed=6000 + n) for n, v in [(5, 0.1), (40, 0.3), (33, 0.02), (700, 0.25), (12, 0.2)] +
+               [(41 + k, 0.0005) for k in range(n_empty)]]
+    shape = dict(timestep=0.001, contact_interval=20, graph_steps=10, lanes_per_bead=8, cell_reach=2, cell_size=1.25)
+    cells = int(tfm_amd.batch_layout(systems, shape)["cells"])
+    step(f"batch of {cells} cells")
+    assert (cells >= 1 << 20) == (n_empty == 13)
+    b = tfm_amd.Batch(systems, shape)
+    b.generate_initial_conditions()
+    xyz0, fl0 = b.state()
+    b.run_steps(40)
+    xyz, _ = b.state()
+    maps, _ = b.contact_maps()
+    for s in list(range(6)) + [len(systems) - 1]:
+        sim = single_from(b, s, xyz0, fl0)
+        sim.run_steps(40)
+        o0, o1 = b.offsets[s], b.offsets[s + 1]
+        assert np.array_equal(sim.positions, xyz[o0:o1]), s
+        m, _ = sim.contact_map()
+        assert np.array_equal(m, maps[s][:len(m), :len(m)]), s
+        sim.close()
+    b.close()

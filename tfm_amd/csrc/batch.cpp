@@ -478,7 +478,7 @@ void plan_batch(ccp_batch &bt, const char *common_params, const ccp_batch_system
   if (!(1 <= b->rd_bins && b->rd_bins <= 1024)) throw Error(CCP_ERR_PARAM, "radial_bins out of range");
   b->n_sys = n_sys;
   b->slot.push_back(0);
-  int coff = 0, boff = 0;
+  int coff = 0;
   uint64_t total = 0;
   for (uint32_t s = 0; s < n_sys; ++s) {
     const ccp_batch_system &in = systems[s];
@@ -503,12 +503,6 @@ void plan_batch(ccp_batch &bt, const char *common_params, const ccp_batch_system
     S.n = one.N;
     S.g = one.gf.g;
     S.g.coff = coff;
-    S.g.boff = boff;
-    // Two cells per lane of the order pass for cells of about a bead each, so
-    // that a block's members still fit its LDS (1024) with room to spare;
-    // larger cells (2.5 sigma: six beads) keep one.
-    S.g.bshift = S.g.csl < 1.5f ? SCAN_SHIFT + 1 : SCAN_SHIFT;
-    S.g.nblk = (S.g.n_c + (1 << S.g.bshift) - 1) >> S.g.bshift;
     if (s == 0) {
       b->kp = one.kp;
       b->contact_rc = one.contact_rc;
@@ -530,7 +524,6 @@ void plan_batch(ccp_batch &bt, const char *common_params, const ccp_batch_system
     // fit the 32-bit offsets of the force kernels' row loads
     if ((uint64_t)coff + (uint64_t)one.gf.g.n_c >= (1ull << 30)) throw Error(CCP_ERR_PARAM, "batch too large");
     coff += one.gf.g.n_c;
-    boff += S.g.nblk;
     total += one.N;
     if (total >= (1ull << ID_BITS)) throw Error(CCP_ERR_PARAM, "batch too large");
     b->slot.push_back((uint32_t)total);
@@ -539,6 +532,21 @@ void plan_batch(ccp_batch &bt, const char *common_params, const ccp_batch_system
     throw Error(CCP_ERR_PARAM, "lanes_per_bead 8 with cell_reach 2 and cells below 1.3 sigma is limited to "
                                "524288 beads per batch: a larger run of this shape faulted the GPU and the cause "
                                "is not yet found");
+  // Two cells per lane of the order pass for cells of about a bead each, so
+  // that a block's members still fit its LDS (1024) with room to spare; larger
+  // cells (2.5 sigma: six beads) keep one. So do batches of less than 2^20
+  // cells, whose blocks are few enough for the chip: us a step with one and two
+  // cells a lane, 46656 cells 34.3 (39.0), 373248 57.8 (61.3), 512000 57.4
+  // (57.3), 1.10 M 95.7 (96.6), 1.15 M 64.5 (61.3), 1.40 M 93.6 (91.3), 2.73 M
+  // 163.4 (157.9).
+  const int shift = b->kp.gf.csl < 1.5f && coff >= (1 << 20) ? SCAN_SHIFT + 1 : SCAN_SHIFT;
+  int boff = 0;
+  for (SysParams &S : b->sys) {
+    S.g.boff = boff;
+    S.g.bshift = shift;
+    S.g.nblk = (S.g.n_c + (1 << shift) - 1) >> shift;
+    boff += S.g.nblk;
+  }
   b->N = (uint32_t)total;
   b->kp.N = (int)b->N;
   b->kp.n_l = 0;
@@ -548,7 +556,7 @@ void plan_batch(ccp_batch &bt, const char *common_params, const ccp_batch_system
   b->grid.g.n_c = coff;
   b->grid.g.coff = 0;
   b->grid.g.nblk = boff;
-  b->grid.g.bshift = b->sys[0].g.bshift;
+  b->grid.g.bshift = shift;
   b->hr.assign(3 * (size_t)b->N, 0.0f);
   b->hfl.assign(b->N, 0);
   b->rd_sum.assign((size_t)n_sys * b->rd_bins, 0.0);
