@@ -286,3 +286,28 @@ def test_batch_scan_blocks_of_two_cells_a_lane(n_empty):
         assert np.array_equal(m, maps[s][:len(m), :len(m)]), s
         sim.close()
     b.close()
+
+
+@pytest.mark.parametrize("shape", [{}, dict(lanes_per_bead=8, cell_reach=2, cell_size=1.25)])
+def test_batch_of_tiny_systems(shape):
+    # several systems in a scan block and runs that end inside one, with a
+    # system of many blocks among them: each equals the single run
+    step(f"batch of tiny systems {shape}")
+    sizes = [5, 9, 4, 16, 7] * 12 + [2000] + [4, 6, 30] * 30
+    systems = [dict(n_beads=n, volume_fraction=(0.1, 0.3)[k % 2], eps_het=0.6, eps_lam=1.0, het_fraction=0.3,
+                    lad_fraction=0.1, seed=7000 + k) for k, n in enumerate(sizes)]
+    b = tfm_amd.Batch(systems, dict(timestep=0.001, contact_interval=20, graph_steps=10, **shape))
+    b.generate_initial_conditions()
+    xyz0, fl0 = b.state()
+    b.run_steps(40)
+    xyz, _ = b.state()
+    maps, _ = b.contact_maps()
+    for s in [0, 1, 17, 33, 59, 60, 61, 62, 100, len(systems) - 2, len(systems) - 1]:
+        sim = single_from(b, s, xyz0, fl0)
+        sim.run_steps(40)
+        o0, o1 = b.offsets[s], b.offsets[s + 1]
+        assert np.array_equal(sim.positions, xyz[o0:o1]), s
+        m, _ = sim.contact_map()
+        assert np.array_equal(m, maps[s][:len(m), :len(m)]), s
+        sim.close()
+    b.close()

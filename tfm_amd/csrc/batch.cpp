@@ -30,7 +30,7 @@ struct BatchGrid {
   DevBuf<uint32_t> count, bs0, bs1, cstart;
   DevBuf<float4> bucket, spos; // bucket: members' positions, index in the w bits
   DevBuf<uint32_t> hbs0, hbs1, work; // type-ordered work list (k_force_typed)
-  DevBuf<OrderBlock> blocks;         // g.nblk scan blocks, each of one system
+  DevBuf<OrderBlock> blocks;         // g.nblk scan blocks, each of one run of systems
   int clean = 0;
   bool valid = false;
   uint32_t *bs(int k) { return k ? bs1.p : bs0.p; }
@@ -156,17 +156,23 @@ struct ccp_batch {
     hip_check(hipStreamSynchronize(stream));
     grid.valid = false;
   }
-  // the scan blocks of every system's cells, with the slots and the het beads
-  // of the systems before it
+  // the scan blocks of every run's cells, with the slots and the het beads of
+  // the systems before it; a run starts with a system that starts a block
   std::vector<OrderBlock> order_blocks() const {
     std::vector<OrderBlock> ob;
     ob.reserve(grid.g.nblk);
+    const int cells = 1 << grid.g.bshift;
     uint32_t het = 0;
-    for (const SysParams &S : sys) {
-      const int cells = 1 << S.g.bshift;
-      for (int c = 0; c < S.g.n_c; c += cells)
-        ob.push_back({S.g.coff + c, std::min(cells, S.g.n_c - c), (uint32_t)S.g.boff, S.slot, het});
-      for (uint32_t i = S.slot; i < S.slot + S.n; ++i) het += (hfl[i] & CCP_HET) ? 1u : 0u;
+    for (size_t s = 0; s < sys.size();) {
+      const SysParams &S = sys[s];
+      const uint32_t blk0 = (uint32_t)ob.size(), het0 = het;
+      int end = S.g.coff;
+      do {
+        end += sys[s].g.n_c;
+        for (uint32_t i = sys[s].slot; i < sys[s].slot + sys[s].n; ++i) het += (hfl[i] & CCP_HET) ? 1u : 0u;
+        ++s;
+      } while (s < sys.size() && (sys[s].g.coff + sys[s].g.bbias) % cells != 0);
+      for (int c = S.g.coff; c < end; c += cells) ob.push_back({c, std::min(cells, end - c), blk0, S.slot, het0});
     }
     return ob;
   }
@@ -540,13 +546,23 @@ void plan_batch(ccp_batch &bt, const char *common_params, const ccp_batch_system
   // (57.3), 1.10 M 95.7 (96.6), 1.15 M 64.5 (61.3), 1.40 M 93.6 (91.3), 2.73 M
   // 163.4 (157.9).
   const int shift = b->kp.gf.csl < 1.5f && coff >= (1 << 20) ? SCAN_SHIFT + 1 : SCAN_SHIFT;
-  int boff = 0;
+  // Systems follow each other in the blocks until a run has RUN_CELLS cells:
+  // a block holds several tiny systems (8192 of 64 cells in blocks of their own
+  // 58.1 us a step, 44.2 before there were any runs), and no block reads
+  // more than a few totals before its own, or those of its one large system.
+  constexpr int RUN_CELLS = 4096;
+  const int block = 1 << shift;
+  int at = 0, run = 0; // cells before in whole blocks, those of the run
   for (SysParams &S : b->sys) {
-    S.g.boff = boff;
+    if (run >= RUN_CELLS) {
+      at += (run + block - 1) / block * block;
+      run = 0;
+    }
+    S.g.bbias = at + run - S.g.coff;
     S.g.bshift = shift;
-    S.g.nblk = (S.g.n_c + (1 << shift) - 1) >> shift;
-    boff += S.g.nblk;
+    run += S.g.n_c;
   }
+  const int nblk = (at + run + block - 1) / block;
   b->N = (uint32_t)total;
   b->kp.N = (int)b->N;
   b->kp.n_l = 0;
@@ -555,7 +571,7 @@ void plan_batch(ccp_batch &bt, const char *common_params, const ccp_batch_system
   b->grid.g = b->kp.gf;
   b->grid.g.n_c = coff;
   b->grid.g.coff = 0;
-  b->grid.g.nblk = boff;
+  b->grid.g.nblk = nblk;
   b->grid.g.bshift = shift;
   b->hr.assign(3 * (size_t)b->N, 0.0f);
   b->hfl.assign(b->N, 0);

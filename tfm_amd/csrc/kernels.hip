@@ -203,11 +203,11 @@ __device__ __forceinline__ void bin_into(const GridGeom &g, uint32_t *count, uin
                                          uint32_t *flags, float4 v, uint32_t *hblocksum = nullptr) {
   bool outside = false;
   const int gx = cell_coord(v.x, g, outside), gy = cell_coord(v.y, g, outside), gz = cell_coord(v.z, g, outside);
-  const uint32_t cell = (uint32_t)((gz * g.cps + gy) * g.cps + gx), key = (uint32_t)g.coff + cell;
+  const uint32_t key = (uint32_t)(g.coff + (gz * g.cps + gy) * g.cps + gx);
   // beads of one wavefront mostly sit in distinct cells: plain atomics
   const uint32_t slot = atomicAdd(count + key, 1u);
   // the block totals and the flag need no slot: done while it returns
-  const uint32_t blk = (uint32_t)g.boff + (cell >> g.bshift);
+  const uint32_t blk = (key + (uint32_t)g.bbias) >> g.bshift;
   agg_add_noret(blocksum, blk);
   if (hblocksum && (wbits(v) & W_HET)) agg_add_noret(hblocksum, blk);
   if (outside) atomicAdd(flags + FLAG_OUTSIDE, 1u);
@@ -1467,10 +1467,11 @@ __global__ __launch_bounds__(BEAD_BLOCK) void k_bin_batch(const SysParams *sys, 
 // within its cell (number of smaller indices) is then found in parallel and
 // the entry written to its sorted slot.
 //
-// BATCH: the scan blocks come from a table, each holding cells of one system
-// (CPT per lane). That system's first slot is known, so a block's prefix
-// starts at the system's first block, and a block with no members (nearly
-// half lie outside the nucleus) only writes its starts. With one run of
+// BATCH: the scan blocks come from a table, each holding cells of one run of
+// systems (CPT per lane; a large system is a run of its own). The run's first
+// slot is known, so a block's prefix starts at the run's first block, and a
+// block with no members (nearly half lie outside the nucleus) only writes its
+// starts. With one run of
 // 256-cell blocks over all systems every block read the totals of all blocks
 // before it; 256 systems of 2048 beads over 1.375 sigma cells (3.3 M cells)
 // took 46.6 us a launch, 30 us with the table, 27.4 us with two cells per lane

@@ -32,13 +32,13 @@ enum Mode : int { MODE_CCP = 0, MODE_ICG = 1, MODE_LJ = 2 };
 // Geometry of one uniform cell grid centred on the nucleus (ccp's sugrid,
 // sugrid.cuh:15-54): cell (gx, gy, gz) = floor(r / csl) + cps/2, index
 // coff + gx + cps (gy + cps gz). coff places the grid of one system inside
-// the concatenated cell range of a batch, boff its scan blocks inside the
-// batch's (both 0 for a single system).
+// the concatenated cell range of a batch, and its cells are numbered bbias
+// further on in the batch's scan blocks (both 0 for a single system).
 struct GridGeom {
   float csl;
   float icsl; // 1/csl for the cell lookup of the step grids; 0: divide by csl (ccp's rule, export grid)
   int cps, half, n_c, cap, nblk, coff;
-  int boff;   // first scan block of the grid: its cells are counted in blocks of their own (0 for a single system)
+  int bbias;  // cell c of the batch is counted in scan block (c + bbias) >> bshift
   int bshift; // log2 of the cells of a scan block
 };
 
@@ -136,9 +136,9 @@ struct KPtrs {
   int n_sys;
 };
 
-// One scan block of a batch: its cells [cell0, cell0 + n_cells), all of one
-// system, that system's first block, and the slots and het members of the
-// systems before it.
+// One scan block of a batch: its cells [cell0, cell0 + n_cells), all of one run
+// of systems, that run's first block, and the slots and het members of the
+// systems before the run.
 struct OrderBlock {
   int cell0, n_cells;
   uint32_t blk0, slot0, het0;
