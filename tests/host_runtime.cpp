@@ -24,7 +24,7 @@ std::map<const void *, std::string> kernels; // host stub -> device name
 std::map<const void *, void *> symbols;      // host shadow of a device variable -> its memory
 std::map<void *, size_t> blocks;             // device memory
 size_t in_use = 0, limit = SIZE_MAX;
-int launch_us = 0, fail_last_error = 0;
+int launch_us = 0, fail_last_error = 0, last_error = OK, fill_copies = 0;
 std::map<std::thread::id, int> threads;
 std::string events;
 void note(const char *what) { // (mu held)
@@ -42,6 +42,7 @@ void rt_memory_limit(size_t bytes) {
 size_t rt_in_use() { return in_use; }
 void rt_launch_time(int us) { launch_us = us; }
 void rt_fail_last_error(int n) { fail_last_error = n; }
+void rt_fill_copies(int on) { fill_copies = on; }
 size_t rt_events(char *buf, size_t len) {
   std::lock_guard<std::mutex> l(mu);
   const size_t n = events.size();
@@ -84,7 +85,7 @@ int hipMalloc(void **p, size_t n) {
   std::lock_guard<std::mutex> l(mu);
   if (in_use + n > limit) {
     *p = nullptr;
-    return NO_MEMORY;
+    return last_error = NO_MEMORY;
   }
   *p = std::calloc(1, n);
   blocks[*p] = n;
@@ -114,8 +115,9 @@ int hipMemcpy(void *d, const void *s, size_t n, int) {
   std::memcpy(d, s, n);
   return OK;
 }
-int hipMemcpyAsync(void *d, const void *s, size_t n, int, void *) {
+int hipMemcpyAsync(void *d, const void *s, size_t n, int kind, void *) {
   std::memcpy(d, s, n);
+  if (fill_copies && kind == 2) std::memset(d, 0xff, n); // what kernels would have left, device to host
   return OK;
 }
 int hipMemset(void *d, int v, size_t n) {
@@ -137,7 +139,10 @@ int hipGetSymbolAddress(void **p, const void *shadow) {
 }
 int hipGetLastError() {
   std::lock_guard<std::mutex> l(mu);
-  return fail_last_error > 0 && fail_last_error-- == 1 ? UNKNOWN : OK;
+  if (fail_last_error > 0 && fail_last_error-- == 1) return UNKNOWN;
+  const int e = last_error;
+  last_error = OK;
+  return e;
 }
 const char *hipGetErrorString(int e) { return e == NO_MEMORY ? "out of memory" : "unknown error"; }
 int hipStreamCreateWithFlags(void **s, unsigned) {

@@ -113,3 +113,41 @@ def test_default_cells_of_ccp_field(runtime, n, vf, half):
     assert not {half} or cps ** 3 <= min(32 * {n} + 32768, (2e7 * {n}) ** 0.5)
     assert fine_cells({n}, {vf}, lanes_per_bead=3)[0] == 2.0
     """)
+
+
+MAPS = """
+def sim(n):
+    r = 0.577 + 0.577 * (n / 0.2) ** (1 / 3)
+    return tfm_amd.Simulation({"number_of_particles": n, "nucleus_radius": f"{r:.6f}", "seed": 1,
+                               "contact_bin_size": 1, "contact_cutoff": 1.5})
+"""
+
+
+def test_maps_need_no_memory_beyond_their_own(runtime):
+    # the list of a map's nonzero words is a faster way to the host: where the
+    # GPU has no memory for it, maps come as they did without it
+    run(runtime, MAPS, """
+    s = sim(4096)
+    rt.rt_memory_limit(0)
+    m, _ = s.contact_map()  # the map is on the device already
+    assert m.shape == (4096, 4096)
+    rt.rt_memory_limit(4 * (1024 * 1025 // 2) + 64)  # the frame's map itself, without its list
+    assert s.frame_contact_map().size == 1024 * 1025 // 2
+    assert s.contact_map()[0].shape == (4096, 4096)
+    rt.rt_memory_limit(2**64 - 1)
+    assert s.frame_contact_map().size == 1024 * 1025 // 2
+    s.close()
+    """)
+
+
+def test_dense_frame_map_takes_back_the_lists_memory(runtime):
+    # a frame's map of too many pixels for its list, with memory for either
+    run(runtime, MAPS, """
+    s = sim(4096)
+    words = 1024 * 1025 // 2
+    rt.rt_memory_limit(4 * words + 64)
+    rt.rt_fill_copies(1)  # the list's count comes back as 2^32 - 1
+    assert s.frame_contact_map().size == words
+    assert s.frame_contact_map().size == words
+    s.close()
+    """)

@@ -382,17 +382,22 @@ void ccp_sim::upload_positions() {
 // way for a frame's at 2^17, and 77 us against 189 at 2^19.
 constexpr size_t LIST_MIN = 1u << 19, LIST_SHARE = 8, LIST_FIRST = 32768;
 
-// Device memory for the list of a map, its count (the first entry) at zero.
+// Device memory for the list of a map, its count (the first entry) at zero;
+// nullptr for a map of too few words, or where there is no memory for a list.
 uint2 *ccp_sim::list_space(size_t words) {
+  if (words < LIST_MIN) return nullptr;
   const size_t entries = 1 + words / LIST_SHARE;
   if (!list_head) {
     void *p = nullptr;
-    hip_check(hipHostMalloc(&p, (1 + LIST_FIRST) * sizeof(uint2)));
+    if (hipHostMalloc(&p, (1 + LIST_FIRST) * sizeof(uint2)) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
     list_head = static_cast<uint2 *>(p);
   }
-  if (!list.p || list.n < entries) { // (an allocation that failed leaves no memory but its size)
+  if (!list.p || list.n < entries) {
     list.free_();
-    list.alloc(entries);
+    if (!list.try_alloc(entries)) return nullptr;
   }
   hip_check(hipMemsetAsync(list.p, 0, sizeof(uint2), stream));
   return list.p;
@@ -1474,9 +1479,8 @@ int ccp_contact_map(ccp_sim *h, uint32_t *map, size_t n_bins2, uint32_t *n_sampl
   return guarded(h, [&] {
     need(map && n_bins2 == (size_t)h->cbins * h->cbins, "contact map size mismatch");
     bool taken = false;
-    if (n_bins2 >= LIST_MIN) {
-      launch_list_words(h->stream, h->cmap.p, (uint32_t)n_bins2, h->list_space(n_bins2),
-                        (uint32_t)(n_bins2 / LIST_SHARE));
+    if (uint2 *list = h->list_space(n_bins2)) {
+      launch_list_words(h->stream, h->cmap.p, (uint32_t)n_bins2, list, (uint32_t)(n_bins2 / LIST_SHARE));
       taken = h->take_list(map, n_bins2);
     }
     if (!taken) {
@@ -1535,13 +1539,15 @@ int ccp_frame_contact_map(ccp_sim *h, float *cm, size_t lcm) {
   return guarded(h, [&] {
     const uint32_t cms = (h->N == N_DEF) ? (h->N / 2) / 4 : h->N / 4;
     need(cm && lcm == (size_t)cms * (cms + 1) / 2, "contact map size mismatch");
-    if (lcm >= LIST_MIN) {
-      launch_ccp_cm(h->stream, h->N, cms, (uint32_t)lcm, h->r.p, nullptr, nullptr, h->list_space(lcm),
-                    (uint32_t)(lcm / LIST_SHARE));
+    if (uint2 *list = h->list_space(lcm)) {
+      launch_ccp_cm(h->stream, h->N, cms, (uint32_t)lcm, h->r.p, nullptr, nullptr, list, (uint32_t)(lcm / LIST_SHARE));
       if (h->take_list(cm, lcm)) return;
     }
     DevBuf<float> out;
-    out.alloc(lcm);
+    if (!out.try_alloc(lcm)) { // (the list's memory may be what is missing)
+      h->list.free_();
+      out.alloc(lcm);
+    }
     launch_ccp_cm(h->stream, h->N, cms, (uint32_t)lcm, h->r.p, out.p, nullptr);
     hip_check(hipGetLastError());
     hip_check(hipMemcpyAsync(cm, out.p, lcm * sizeof(float), hipMemcpyDeviceToHost, h->stream));

@@ -81,6 +81,16 @@ template <class T> struct DevBuf {
     n = count;
     hip_check(hipMalloc(&p, std::max<size_t>(count, 1) * sizeof(T)));
   }
+  // false where the device has no memory for it
+  bool try_alloc(size_t count) {
+    n = count;
+    const hipError_t e = hipMalloc(&p, std::max<size_t>(count, 1) * sizeof(T));
+    if (e == hipSuccess) return true;
+    p = nullptr;
+    (void)hipGetLastError(); // (no error of the next launch's)
+    if (e != hipErrorOutOfMemory) hip_check(e);
+    return false;
+  }
   void free_() {
     if (p) (void)hipFree(p);
     p = nullptr;
