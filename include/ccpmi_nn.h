@@ -2,9 +2,11 @@
  * ccpmi_nn — kernels of the contact-map surrogate (no counterpart in ccp).
  *
  * A 1-D convolutional encoder over the binned het/LAD sequence with a
- * pairwise outer-product head, trained and evaluated with these kernels:
- * a strided batched BF16 GEMM on the matrix cores with FP32 accumulation,
- * and the element-wise steps around it. Activations are stored
+ * pairwise outer-product head. Two sets of kernels compute it: single
+ * operations (a strided batched BF16 GEMM on the matrix cores with FP32
+ * accumulation, and the element-wise steps around it), for a caller's own
+ * composition, and the network's own kernels further down, which fuse them
+ * and give the same bits in outputs and weight gradients. Activations are stored
  * channel-major: x[c, b L + l] for channel c, sample b, bin l. BF16 values
  * are passed as raw 16-bit words (void pointers). Every call is
  * asynchronous on `stream` (a hipStream_t) and returns 0, 1 for bad sizes,

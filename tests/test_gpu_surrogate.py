@@ -248,3 +248,103 @@ def test_weight_gradients_of_long_rows(taps, L, Ps):
     assert np.array_equal(dst.cpu().numpy(), want.reshape(M, taps * C))
     del G, X
     torch.cuda.empty_cache()
+
+
+def single_operations(net, x, T, T_rd, w_pair, w_rd):
+    """The network's step from the library's single operations (an im2col matrix
+    and one product a layer): outputs, loss and gradients. Weights as net's."""
+    N, B, L, W, d, n, O = sg._nn(), net.B, net.L, net.width, net.d, net.n_layers, net.rd_bins
+    P, st = B * L, sg._stream()
+    f = lambda *s: torch.zeros(s, dtype=torch.float32, device="cuda")
+    h = lambda *s: torch.zeros(s, dtype=torch.int16, device="cuda")
+    a = lambda *t: [None if v is None else v.data_ptr() if torch.is_tensor(v) else v for v in t]
+
+    def call(name, *args):
+        assert getattr(N, "ccp_nn_" + name)(*a(*args), st) == 0, name
+
+    pb = {k: h(*net.p[k].shape) for k in net.names if k.startswith("W")}
+    for k, t in pb.items():
+        call("cast_bf16", net.p[k], t, t.numel())
+    xb = h(*x.shape)
+    call("cast_bf16", x, xb, x.numel())
+    inp, res, c = xb, None, net.c_in
+    cols, pre = {}, {}
+    for k in range(1, n + 1):
+        cols[k], pre[k], y, yb = h(3 * c, P), f(W, P), f(W, P), h(W, P)
+        call("im2col", inp, cols[k], c, B, L)
+        sg.gemm(pb[f"W{k}"], cols[k], W, P, 3 * c, (0, 3 * c, 1), (0, P, 1), (0, P, 1), C=pre[k])
+        call("bias_gelu", pre[k], net.p[f"b{k}"], res, y, yb, W, P)
+        inp, res, c = yb, y, W
+    U, V, raw, S = h(d, P), h(d, P), f(B, L, L), f(B, L, L)
+    for k, t in (("Wu", U), ("Wv", V)):
+        sg.gemm(pb[k], inp, d, P, W, (0, W, 1), (0, P, 1), (0, P, 1), Cb=t)
+    alpha = 1.0 / math.sqrt(d)
+    sg.gemm(U, V, L, L, d, (L, 1, P), (L, P, 1), (L * L, L, 1), C=raw, batch=B, alpha=alpha)
+    call("pair_map", raw, net.p["dist"], net.p["c0"], S, L, B)
+    pooled, pooledb, rd = f(W, B), h(W, B), f(O, B)
+    call("mean_pool", res, pooled, pooledb, W, B, L)
+    sg.gemm(pb["Wr"], pooledb, O, B, W, (0, W, 1), (0, B, 1), (0, B, 1), C=rd)
+    g, loss = {k: f(*net.p[k].shape) for k in net.names}, f(1)
+    gS, graw, grawb, grd, grdb = f(B, L, L), f(B, L, L), h(B, L, L), f(O, B), h(O, B)
+    call("pair_loss", S, T, gS, graw, grawb, g["dist"], g["c0"], loss, L, B, w_pair)
+    call("rd_loss", rd, net.p["br"], T_rd, grd, grdb, g["br"], loss, O, B, w_rd)
+    dU, dV, dh = h(d, P), h(d, P), f(W, P)
+    sg.gemm(V, grawb, d, L, L, (L, P, 1), (L * L, 1, L), (L, P, 1), Cb=dU, batch=B, alpha=alpha)
+    sg.gemm(U, grawb, d, L, L, (L, P, 1), (L * L, L, 1), (L, P, 1), Cb=dV, batch=B, alpha=alpha)
+    for k, t in (("Wu", dU), ("Wv", dV)):
+        sg.gemm(t, inp, d, W, P, (0, P, 1), (0, 1, P), (0, W, 1), C=g[k], beta=1.0)
+    sg.gemm(pb["Wu"], dU, W, P, d, (0, 1, W), (0, P, 1), (0, P, 1), C=dh)
+    sg.gemm(pb["Wv"], dV, W, P, d, (0, 1, W), (0, P, 1), (0, P, 1), C=dh, beta=1.0)
+    sg.gemm(grdb, pooledb, O, W, B, (0, B, 1), (0, 1, B), (0, W, 1), C=g["Wr"], beta=1.0)
+    dpooled = f(W, B)
+    sg.gemm(pb["Wr"], grdb, W, B, O, (0, 1, W), (0, B, 1), (0, B, 1), C=dpooled)
+    call("pool_back", dpooled, dh, W, B, L)
+    gp, gpb, dcols = f(W, P), h(W, P), f(3 * W, P)
+    for k in range(n, 0, -1):
+        call("gelu_back", pre[k], dh, gp, gpb, g[f"b{k}"], W, P)
+        K = 3 * (net.c_in if k == 1 else W)
+        sg.gemm(gpb, cols[k], W, K, P, (0, P, 1), (0, 1, P), (0, K, 1), C=g[f"W{k}"], beta=1.0)
+        if k > 1:
+            sg.gemm(pb[f"W{k}"], gpb, K, P, W, (0, 1, K), (0, P, 1), (0, P, 1), C=dcols)
+            call("col2im", dcols, dh, W, B, L, 1.0)
+    return S, rd, loss, g
+
+
+@pytest.mark.parametrize("c", [cfg(), dict(c_in=3, width=36, n_layers=2, d=5, L=13, rd_bins=7, B=5),
+                               dict(c_in=5, width=100, n_layers=4, d=33, L=64, rd_bins=33, B=9)])
+def test_single_operations_give_the_networks_numbers(c):
+    # the library's single operations and the network's fused kernels contract
+    # in the same order: outputs and weight gradients bit for bit, the sums over
+    # positions (biases, distance terms) as FP32 sums in two orders, and one step
+    # of AdamW tensor by tensor
+    step(f"single operations, sizes {c}")
+    rng = np.random.default_rng(c["width"])
+    p = so.init_params(c["c_in"], c["width"], c["n_layers"], c["d"], c["L"], c["rd_bins"], seed=3)
+    p = {k: v + 0.05 * rng.normal(size=v.shape) for k, v in p.items()}
+    dev = lambda a: torch.tensor(np.asarray(a, np.float32), device="cuda")
+    x, T_rd = dev(rng.normal(size=(c["c_in"], c["B"] * c["L"]))), dev(rng.normal(size=(c["rd_bins"], c["B"])))
+    T = rng.normal(size=(c["B"], c["L"], c["L"]))
+    T = dev(0.5 * (T + T.transpose(0, 2, 1)))
+    net = sg.Surrogate(params=p, **c)
+    S, rd, loss, g = single_operations(net, x, T, T_rd, 1.0, 0.5)
+    net.zero_grad()
+    got = net.loss_backward(x, T, T_rd, w_pair=1.0, w_rd=0.5)
+    assert torch.equal(net.S, S) and torch.equal(net.rd, rd)
+    assert got.item() == pytest.approx(loss.item(), rel=1e-5)
+    for k in net.names:
+        if k.startswith("W"):
+            assert torch.equal(net.g[k], g[k]), k
+        else:
+            assert rel(net.g[k].cpu().numpy(), g[k].cpu().numpy()) < 1e-5, k
+    for k in net.names:
+        w, m, v, wb = net.p[k].clone(), torch.zeros_like(g[k]), torch.zeros_like(g[k]), sg.bf16_like(g[k])
+        grad = net.g[k].contiguous()
+        args = [t.data_ptr() for t in (w, grad, m, v, wb)]
+        assert sg._nn().ccp_nn_adamw(*args, w.numel(), 1e-3, 0.9, 0.999, 1e-8, 1e-4 if k.startswith("W") else 0.0, 1,
+                                     sg._stream()) == 0
+        p[k] = w, wb
+    net.step()
+    for k in net.names:
+        assert torch.equal(net.p[k], p[k][0]), k
+        if k.startswith("W"):
+            assert torch.equal(net.pb[k], p[k][1]), k
