@@ -232,3 +232,21 @@ def test_frame_contact_map_rows_of_a_block(N, scale):
     sim = sim_with(N, R_n, walk(N, R_n, seed=N) * np.float32(scale), np.zeros(N, np.uint8))
     assert np.array_equal(sim.frame_contact_map(), po.ccp_contact_map(sim.positions))
     sim.close()
+
+
+@pytest.mark.parametrize("N,n_b", [(700, 1024), (700, 1025), (300, 4096), (5, 2500)])
+def test_observables_of_many_bins(N, n_b):
+    # up to 1024 bins the workgroup holds the shells' radii in a table, above
+    # each is computed where it is used; the tolerances above
+    step(f"observables N={N} n_b={n_b}")
+    R_n = max(radius_for(N, 0.2), 4.0)
+    r = walk(N, R_n, seed=N + n_b)
+    flags = (np.random.default_rng(N).random(N) < 0.4).astype(np.uint8)
+    sim = sim_with(N, R_n, r, flags)
+    sc, rcd = sim.observables(n_b)
+    R_nf, R_of = float(np.float32(R_n)), float(sim.info.R_o)
+    nod = float(np.float32(np.sqrt(R_nf * R_nf - R_of * R_of)))
+    want, want_rcd = po.observables(sim.positions.astype(np.float64), flags, R_nf, nod=nod, n_b=n_b)
+    assert np.allclose(sc, want, rtol=1e-9, atol=1e-9), (sc, want)
+    assert np.allclose(rcd, want_rcd, rtol=1e-9, atol=1e-10)
+    sim.close()

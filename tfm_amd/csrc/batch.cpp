@@ -481,7 +481,7 @@ void plan_batch(ccp_batch &bt, const char *common_params, const ccp_batch_system
   b->bins = cpar.get<uint32_t>("contact_bins", 128u);
   b->rd_bins = cpar.get<uint32_t>("radial_bins", 32u);
   if (!(1 <= b->bins && b->bins <= 4096)) throw Error(CCP_ERR_PARAM, "contact_bins out of range");
-  if (!(1 <= b->rd_bins && b->rd_bins <= 1024)) throw Error(CCP_ERR_PARAM, "radial_bins out of range");
+  if (!(1 <= b->rd_bins && b->rd_bins <= (uint32_t)LENS_TABLE)) throw Error(CCP_ERR_PARAM, "radial_bins out of range");
   b->n_sys = n_sys;
   b->slot.push_back(0);
   int coff = 0;

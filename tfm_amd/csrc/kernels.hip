@@ -1944,7 +1944,6 @@ __device__ __forceinline__ void lens_bins(double d, double a, double R_n, int n_
 }
 // the bins' cube roots, once per workgroup where they fit its table (an FP64
 // cube root per bead and bin was most of the kernels' time)
-constexpr int LENS_TABLE = 1024;
 struct LensRoots {
   const double *table; // n_b entries, or nullptr: more bins than the table holds
   int n_b;
@@ -2014,7 +2013,8 @@ __global__ __launch_bounds__(BEAD_BLOCK) void k_observables(int N, double R_n, d
 // Radial density of every system of a batch (the all-bead row of
 // k_observables), one lane per bead, FP64 sums into out[s n_b + k]. The
 // workgroup's beads mostly belong to one system: that of its first bead is
-// summed in LDS and added once per bin, the others' beads go out directly.
+// summed in LDS and added once per bin, the others' beads go out directly. All
+// bins of a batch fit the table.
 __global__ __launch_bounds__(BEAD_BLOCK) void k_radial_batch(const SysParams *sys, const uint32_t *sys_slot,
                                                              int n_sys, int n, double a, int n_b, const float4 *pos,
                                                              double *out) {
@@ -2022,24 +2022,21 @@ __global__ __launch_bounds__(BEAD_BLOCK) void k_radial_batch(const SysParams *sy
   const int i = blockIdx.x * BEAD_BLOCK + threadIdx.x;
   const int first = system_of(sys_slot, n_sys, (uint32_t)(blockIdx.x * BEAD_BLOCK));
   const LensRoots root = lens_roots(s_root, n_b);
-  const bool local = n_b <= LENS_TABLE;
-  if (local)
-    for (int k = threadIdx.x; k < n_b; k += BEAD_BLOCK) s_acc[k] = 0.0;
+  for (int k = threadIdx.x; k < n_b; k += BEAD_BLOCK) s_acc[k] = 0.0;
   __syncthreads();
   if (i < n) {
     const int s = system_of(sys_slot, n_sys, (uint32_t)i);
     const float4 q = pos[i];
     const double x = q.x, y = q.y, z = q.z;
-    const bool here = local && s == first;
+    const bool here = s == first;
     lens_bins(sqrt(x * x + y * y + z * z), a, (double)sys[s].R_n, n_b, root, [&](int k, double net) {
       if (here) atomicAdd(&s_acc[k], net);
       else atomicAdd(out + (size_t)s * n_b + k, net);
     });
   }
   __syncthreads();
-  if (local)
-    for (int k = threadIdx.x; k < n_b; k += BEAD_BLOCK)
-      if (s_acc[k] != 0.0) atomicAdd(out + (size_t)first * n_b + k, s_acc[k]);
+  for (int k = threadIdx.x; k < n_b; k += BEAD_BLOCK)
+    if (s_acc[k] != 0.0) atomicAdd(out + (size_t)first * n_b + k, s_acc[k]);
 }
 
 // ccp's FP32 sum of 1000 per contact, a function of their number n alone: the

@@ -21,6 +21,9 @@ constexpr uint32_t W_HET = 1u << 31; // the sign bit: a het partner is a negativ
 // cells per scan block of the order kernel; each block reads the totals of
 // the blocks before it, so fewer, larger blocks keep that prefix cheap
 constexpr int SCAN_BLOCK = 256, SCAN_SHIFT = 8;
+// shells of a radial density whose radii a workgroup keeps in a table; a batch
+// has no more
+constexpr int LENS_TABLE = 1024;
 // threads per block of the bead kernels
 constexpr int BEAD_BLOCK = 256;
 
