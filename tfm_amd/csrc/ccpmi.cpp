@@ -107,7 +107,7 @@ void ccp_sim::configure(const ParMap &par) {
   split = csl_f < csl;
   if (split && !(csl_f >= short_cut && csl_f >= LCO && csl_f >= MIS && csl_f >= contact_rc / 2.0f))
     throw Error(CCP_ERR_PARAM, "fine_cell_size below the short-range cutoff");
-  // the overlap count of the initial condition scans one cell around each bead
+  // the initial condition counts overlaps on the step's grid
   if (!(csl_f >= MIS)) throw Error(CCP_ERR_PARAM, "cell_size below the overlap distance");
   if (split && reach != 1) throw Error(CCP_ERR_PARAM, "fine_cell_size needs cell_reach 1");
   uint32_t cap = par.get<uint32_t>("cell_capacity", 32u);
@@ -1453,7 +1453,8 @@ int ccp_noise(ccp_sim *h, uint64_t step, float *z_xyz, uint32_t *attempts, size_
 int ccp_count_overlaps(ccp_sim *h, float dmin, uint64_t *count) {
   return guarded(h, [&] {
     need(count != nullptr, "null count");
-    need(dmin > 0.0f && dmin <= h->dmin_max, "dmin must be in (0, fine_cell_size]");
+    if (!(dmin > 0.0f && dmin <= h->dmin_max))
+      throw Error(CCP_ERR_ARG, "dmin must be in (0, fine_cell_size], here " + cnfs(h->dmin_max));
     *count = h->count_overlaps(dmin);
   });
 }
