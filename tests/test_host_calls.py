@@ -151,3 +151,24 @@ def test_dense_frame_map_takes_back_the_lists_memory(runtime):
     assert s.frame_contact_map().size == words
     s.close()
     """)
+
+
+def test_full_contact_map_is_listed_once(runtime):
+    # a summed map with too many nonzero words for its list keeps them until it
+    # is cleared: only the first read tries the list
+    run(runtime, MAPS, """
+    s = sim(4096)
+    def listed():
+        events()
+        assert s.contact_map()[0].shape == (4096, 4096)
+        return sum("k_list_words" in e for _, e in events())
+    assert [listed(), listed()] == [1, 1]
+    rt.rt_fill_copies(1)  # the list's count comes back as 2^32 - 1
+    assert [listed(), listed(), listed()] == [1, 0, 0]
+    rt.rt_fill_copies(0)
+    s.contact_sample()
+    assert listed() == 0
+    s.contact_reset()
+    assert [listed(), listed()] == [1, 1]
+    s.close()
+    """)

@@ -377,8 +377,9 @@ void ccp_sim::upload_positions() {
 // the caller's array here, which is cleared while the kernel runs: 1712 -> 207
 // us (most of it the clearing) and 227 -> 42 us. At 1 M words a list of a ninth
 // takes 101 us and the whole map 247; a longer list is given up for the whole
-// map as soon as its count is here, which then takes 288 us (a map summed over
-// a long run, read once). Maps below 2^19 words are copied whole: 63 us either
+// map as soon as its count is here, which then takes 288 us. A map that is
+// summed over a run only fills up, so its further reads take the whole map at
+// once, until it is cleared. Maps below 2^19 words are copied whole: 63 us either
 // way for a frame's at 2^17, and 77 us against 189 at 2^19.
 constexpr size_t LIST_MIN = 1u << 19, LIST_SHARE = 8, LIST_FIRST = 32768;
 
@@ -1473,6 +1474,7 @@ int ccp_contact_reset(ccp_sim *h) {
     hip_check(hipMemsetAsync(h->cmap.p, 0, (size_t)h->cbins * h->cbins * 4, h->stream));
     hip_check(hipStreamSynchronize(h->stream));
     h->n_samples = 0;
+    h->cmap_full = false;
   });
 }
 
@@ -1480,9 +1482,10 @@ int ccp_contact_map(ccp_sim *h, uint32_t *map, size_t n_bins2, uint32_t *n_sampl
   return guarded(h, [&] {
     need(map && n_bins2 == (size_t)h->cbins * h->cbins, "contact map size mismatch");
     bool taken = false;
-    if (uint2 *list = h->list_space(n_bins2)) {
+    if (uint2 *list = h->cmap_full ? nullptr : h->list_space(n_bins2)) {
       launch_list_words(h->stream, h->cmap.p, (uint32_t)n_bins2, list, (uint32_t)(n_bins2 / LIST_SHARE));
       taken = h->take_list(map, n_bins2);
+      h->cmap_full = !taken;
     }
     if (!taken) {
       hip_check(hipMemcpyAsync(map, h->cmap.p, 4 * n_bins2, hipMemcpyDeviceToHost, h->stream));

@@ -145,6 +145,7 @@ struct ccp_sim {
   DevBuf<uint2> list;          // a map's nonzero words on their way to the host (at most a quarter of the map)
   uint2 *list_head = nullptr;  // pinned: its count and first entries
   std::vector<uint2> list_rest;
+  bool cmap_full = false;      // too many nonzero words for a list; so it stays until the map is cleared
   std::vector<float4> upload_rows; // positions on their way to the device, kept so that a frame allocates nothing
   std::vector<uint8_t> hfl;
   bool lgrid_valid = false, dstep_dirty = true;
