@@ -2,7 +2,9 @@
 matrix cores against float64 products of the same bfloat16 values, and the
 network's forward pass and every gradient against the numpy oracle with the
 same bfloat16 rounding points; then a short training run."""
+import copy
 import math
+import pickle
 
 import numpy as np
 import pytest
@@ -348,3 +350,34 @@ def test_single_operations_give_the_networks_numbers(c):
         assert torch.equal(net.p[k], p[k][0]), k
         if k.startswith("W"):
             assert torch.equal(net.pb[k], p[k][1]), k
+
+
+@pytest.mark.parametrize("how", ["deepcopy", "pickle"])
+def test_a_copied_net_is_a_net_of_its_own(how):
+    # a copy trains on its own tensors, bit for bit as a net built from the same
+    # parameters, and leaves the original's alone
+    step(f"surrogate copied by {how}")
+    c, p, x, T, T_rd = problem(7)
+    dev = lambda a: torch.tensor(np.asarray(a, np.float32), device="cuda")
+    X, TT, TR = dev(x), dev(T), dev(T_rd)
+    net, want = sg.Surrogate(params=p, **c), sg.Surrogate(params=p, **c)
+
+    def train(n):
+        n.zero_grad()
+        n.loss_backward(X, TT, TR)
+        n.step(lr=3e-3)
+
+    train(net)
+    train(want)
+    before = net.state_dict()
+    out = net.predict(X)[0].clone()
+    other = copy.deepcopy(net) if how == "deepcopy" else pickle.loads(pickle.dumps(net))
+    for n in (other, want):
+        for _ in range(2):
+            train(n)
+    for group in ("p", "g", "m", "v"):
+        for k in net.names:
+            assert torch.equal(getattr(other, group)[k], getattr(want, group)[k]), (group, k)
+    assert torch.equal(other.predict(X)[0], want.predict(X)[0])
+    assert all(np.array_equal(a, b) for a, b in zip(net.state_dict().values(), before.values()))
+    assert torch.equal(net.predict(X)[0], out)

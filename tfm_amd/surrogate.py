@@ -166,15 +166,31 @@ class Surrogate:
         self._flat = [torch.zeros(at, dtype=torch.float32, device=dev) for _ in range(4)]
         view = lambda t: {k: t[off[k]:off[k] + host[k].size].view(host[k].shape) for k in self.names}
         self.p, self.g, self.m, self.v = (view(t) for t in self._flat)
-        self._numel = {k: host[k].size for k in self.names}
-        self._flat_at = [_at(t, self.names) for t in (self.p, self.g, self.m, self.v)]
+        self._numel, self._off = {k: host[k].size for k in self.names}, off
         for k in self.names:
             self.p[k].copy_(torch.from_numpy(host[k]))
         self.pb = {k: bf16_like(v) for k, v in self.p.items() if k.startswith("W")}
         self.t = 0
         self._alloc_packed()
-        self._cast_weights()
         self._alloc(B)
+        self._cast_weights()
+
+    # what holds addresses: left out of copies and made anew for them
+    _BOUND = ("_flat_at", "_pack", "_pack_at", "_fwd", "_bias_at", "_back", "_jobs", "_seg", "_grad_at")
+
+    def __getstate__(self):
+        return {k: v for k, v in self.__dict__.items() if k not in self._BOUND}
+
+    def __setstate__(self, state):
+        self.__dict__.update(state)
+        self._bind()
+
+    def _bind(self):
+        self._flat_at = [[t.data_ptr() + 4 * self._off[k] for k in self.names] for t in self._flat]
+        self._bind_pack()
+        self._bind_forward()
+        self._bind_backward()
+        self._bind_grads()
 
     def _own(self, group, names, dtype=torch.float32):
         """Entries whose addresses go into a kernel's arguments: whole contiguous device arrays."""
@@ -196,7 +212,6 @@ class Surrogate:
         self._wt["uv"] = h(2, Cr, Kd)
         self._wf["r"], self._wt["r"] = h(O, _up(W, 64)), h(Cr, _up(O, 32))
         self._weights = [k for k in self.names if k.startswith("W")]
-        self._bind_pack()
 
     def _bind_pack(self):
         """The table that fills the packed copies from p."""
@@ -240,7 +255,6 @@ class Surrogate:
         self.pooledb, self.pooledt = h(W, Bs), h(B, Cs)
         self.rd = f(self.rd_bins, B)
         self._biases = [f"b{k}" for k in range(1, n + 1)]
-        self._bind_forward()
         # backward: every layer keeps its gradient's channel rows for the weight gradients' one launch
         bands, tiles = _nn().ccp_nn_pair_bands(L), (P + 127) // 128
         self.grawb = h(B, L, Ls)
@@ -253,15 +267,7 @@ class Surrogate:
         self.loss = f(1)
         self._gdist, self._gc0 = f(B * bands, L), f(B * bands)
         self._dbias = {k: f(tiles, W) for k in range(1, n + 1)}
-        Cr = _up(W, 64)
-        self._back = {n: BackArgs(_p(self._wt["uv"]), _p(self.duvt), _p(self.dpooled), _p(self.pre[n]), _p(self.dh),
-                                  _p(self.gb[n]), _p(self.gt[n % 2]), _p(self._dbias[n]), W, Cs, Cr, _up(d, 32),
-                                  2 * ds, P, Ps, L, B, ds, int(n > 1))}
-        for k in range(n - 1, 0, -1):
-            self._back[k] = BackArgs(_p(self._wt[k + 1]), _p(self.gt[(k + 1) % 2]), None, _p(self.pre[k]), _p(self.dh),
-                                     _p(self.gb[k]), _p(self.gt[k % 2]), _p(self._dbias[k]), W, Cs, Cr, _up(W, 32),
-                                     Cs, P, Ps, L, B, 0, int(k > 1))
-        self._bind_grads()
+        self._bind()
 
     def _bind_forward(self):
         """Arguments of the layers' products, with the biases of p."""
@@ -281,6 +287,19 @@ class Surrogate:
                 _p(self._wf["u"]), _p(self._wf["v"]), _p(self.ht[(n + 1) % 2]), None, None, None, None,
                 _p(self.uvb) if keep else None, _p(self.uvt), 2 * d, d, _up(W, 64), Cs, P, Ps, L, 2 * ds, ds)
         self._bias_at = _at(self.p, self._biases)
+
+    def _bind_backward(self):
+        """Arguments of the layers' gradients."""
+        W, L, d, n, B = self.width, self.L, self.d, self.n_layers, self.B
+        Cs, ds, P, Ps = self._cs, self._ds, B * L, self._ps
+        Cr = _up(W, 64)
+        self._back = {n: BackArgs(_p(self._wt["uv"]), _p(self.duvt), _p(self.dpooled), _p(self.pre[n]), _p(self.dh),
+                                  _p(self.gb[n]), _p(self.gt[n % 2]), _p(self._dbias[n]), W, Cs, Cr, _up(d, 32),
+                                  2 * ds, P, Ps, L, B, ds, int(n > 1))}
+        for k in range(n - 1, 0, -1):
+            self._back[k] = BackArgs(_p(self._wt[k + 1]), _p(self.gt[(k + 1) % 2]), None, _p(self.pre[k]), _p(self.dh),
+                                     _p(self.gb[k]), _p(self.gt[k % 2]), _p(self._dbias[k]), W, Cs, Cr, _up(W, 32),
+                                     Cs, P, Ps, L, B, 0, int(k > 1))
 
     def _bind_grads(self):
         """Tables of the weight gradients and of the sums that go into g."""
