@@ -109,6 +109,7 @@ struct ccp_batch {
   DevBuf<unsigned long long> dover; // overlap count per system
   DevBuf<double> obs;
   BatchGrid grid;
+  std::vector<OrderBlock> blocks; // what grid.blocks holds
   hipGraphExec_t graphs[2] = {nullptr, nullptr};
   std::string err;
 
@@ -151,9 +152,16 @@ struct ccp_batch {
       h[i] = make_float4(hr[3 * i], hr[3 * i + 1], hr[3 * i + 2], wf);
     }
     hip_check(hipMemcpyAsync(r.p, h.data(), (size_t)N * sizeof(float4), hipMemcpyHostToDevice, stream));
-    const std::vector<OrderBlock> ob = order_blocks();
-    hip_check(hipMemcpyAsync(grid.blocks.p, ob.data(), ob.size() * sizeof(OrderBlock), hipMemcpyHostToDevice, stream));
+    // (new positions of the same beads leave the table as it is)
+    std::vector<OrderBlock> ob = order_blocks();
+    const size_t bytes = ob.size() * sizeof(OrderBlock);
+    const bool same = ob.size() == blocks.size() && std::memcmp(ob.data(), blocks.data(), bytes) == 0;
+    if (!same) {
+      blocks.clear(); // (until the copy is done)
+      hip_check(hipMemcpyAsync(grid.blocks.p, ob.data(), bytes, hipMemcpyHostToDevice, stream));
+    }
     hip_check(hipStreamSynchronize(stream));
+    blocks = std::move(ob);
     grid.valid = false;
   }
   // the scan blocks of every run's cells, with the slots and the het beads of
