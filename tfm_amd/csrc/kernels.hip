@@ -2281,9 +2281,10 @@ __device__ __forceinline__ uint32_t cm_pairs(const float4 u[4], const float4 *v)
 // every pixel is empty (a contact reaches 2 sigma in a nucleus of tens), so the
 // test of the bounds decides all but a few per cent of the wavefronts' pixels;
 // one lane per packed pixel evaluating its 32 pairs took 253 us at N = 30386
-// (7.2 M pixels); this takes 72 us, 8 rows a block (171, 94, 78 and 78 us with
-// 1, 2, 4 and 16; medians over maps of 1 % to all pixels). Maps of less than 1024 rows leave most of the chip idle and
-// take one row a block: 3.7 us for 16 rows, 5.7 for 100 (8 rows: 10.5, 12.4).
+// (7.2 M pixels); this takes 42 us, and over maps of 1 % to all pixels a median
+// of 72 with 8 rows a block (171, 94, 78 and 78 with 1, 2, 4 and 16). Maps of
+// less than 1024 rows leave most of the chip idle and take one row a block: 3.7
+// us for 16 rows, 5.7 for 100 (8 rows: 10.5, 12.4).
 //
 // The map goes to `cm`, or its nonzero pixels (index, bits of the value) to
 // `list`, whose first entry counts them; those past `cap` are only counted. A
