@@ -311,3 +311,36 @@ def test_batch_of_tiny_systems(shape):
         assert np.array_equal(m, maps[s][:len(m), :len(m)]), s
         sim.close()
     b.close()
+
+
+@pytest.mark.parametrize("shape,size,phi", [
+    (dict(lanes_per_bead=8, cell_reach=1, cell_size=2.5), 400, 0.005),
+    (dict(lanes_per_bead=8, cell_reach=2, cell_size=1.25), 400, 0.005),
+    (dict(lanes_per_bead=8, cell_reach=2, cell_size=1.25), 700, 0.0005),  # two cells a lane
+    (dict(lanes_per_bead=3), 400, 0.005),
+])
+def test_batch_short_block_before_a_small_last_system(shape, size, phi):
+    # a run of cells whose last scan block is short by more cells than the last
+    # run has: the starts' end entry is still the last system's own
+    step(f"batch with a small last system {shape} {size}")
+    systems = [dict(n_beads=n, volume_fraction=v, eps_het=0.6, eps_lam=1.0, het_fraction=0.3, lad_fraction=0.1,
+                    seed=8000 + n) for n, v in [(size, phi), (4, 0.35)]]
+    common = dict(timestep=0.001, contact_interval=20, graph_steps=10, **shape)
+    first, total = (int(c) for c in tfm_amd.batch_layout(systems, common)["cell_offsets"][1:])
+    block = 512 if total >= 1 << 20 else 256
+    assert first >= 4096 and 0 < first % block and total <= first - first % block + block
+    b = tfm_amd.Batch(systems, common)
+    b.generate_initial_conditions()
+    xyz0, fl0 = b.state()
+    b.run_steps(40)
+    xyz, _ = b.state()
+    maps, _ = b.contact_maps()
+    for s in range(2):
+        sim = single_from(b, s, xyz0, fl0)
+        sim.run_steps(40)
+        o0, o1 = b.offsets[s], b.offsets[s + 1]
+        assert np.array_equal(sim.positions, xyz[o0:o1]), s
+        m, _ = sim.contact_map()
+        assert np.array_equal(m, maps[s][:len(m), :len(m)]), s
+        sim.close()
+    b.close()

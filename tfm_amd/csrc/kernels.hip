@@ -1581,8 +1581,10 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_order(OrderJobs<TWO ? 2 : 1> job
       for (int k = 0; k < SCAN_BLOCK / 64; ++k) prefix += red[k];
 #pragma unroll
       for (int u = 0; u < CPT; ++u) {
-        if (c0 + u < c_end) J.cstart[c0 + u] = prefix;
-        if (c0 + u == n_c - 1) J.cstart[n_c] = prefix;
+        if (c0 + u < c_end) {
+          J.cstart[c0 + u] = prefix;
+          if (c0 + u == n_c - 1) J.cstart[n_c] = prefix;
+        }
       }
       return;
     }
@@ -1664,8 +1666,9 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_order(OrderJobs<TWO ? 2 : 1> job
     if (c0 + u < c_end) {
       J.cstart[c0 + u] = start[u];
       J.count[c0 + u] = 0u;
+      // (the lanes past a short block's cells hold numbers of the next run's)
+      if (c0 + u == n_c - 1) J.cstart[n_c] = start[u] + cnt[u];
     }
-    if (c0 + u == n_c - 1) J.cstart[n_c] = start[u] + cnt[u];
   }
   // work-list entry of the member at slot dst, with hbefore het members in
   // the slots before it: het members in slot order, then the others
