@@ -344,3 +344,29 @@ def test_batch_short_block_before_a_small_last_system(shape, size, phi):
         assert np.array_equal(m, maps[s][:len(m), :len(m)]), s
         sim.close()
     b.close()
+
+
+@pytest.mark.parametrize("shape", [dict(lanes_per_bead=8, cell_reach=2, cell_size=1.25),
+                                   dict(lanes_per_bead=5, cell_reach=2, cell_size=1.25)])
+def test_batch_steps_past_an_overflowing_cell(shape):
+    # stretched chains, one bead a cell, contract in cells that hold one bead:
+    # the steps queued behind the first overflow run, then the error comes
+    step(f"batch with one bead a cell {shape}")
+    sizes = [(12, 0.05), (40, 0.005), (24, 0.05), (60, 0.005), (16, 0.05)]
+    systems = [dict(n_beads=n, volume_fraction=v, eps_het=0.6, eps_lam=1.0, het_fraction=0.3, lad_fraction=0.1,
+                    seed=9200 + k) for k, (n, v) in enumerate(sizes)]
+    b = tfm_amd.Batch(systems, dict(timestep=0.001, cell_capacity=1, graph_steps=16, **shape))
+    xyz, flags = [], []
+    for n, _ in sizes:
+        m = int(np.ceil(np.cbrt(n)))
+        i = np.arange(n)
+        z, y, x = i // (m * m), i // m % m, i % m
+        y = np.where(z % 2, m - 1 - y, y)  # (a snake: neighbours along the chain are neighbours in space)
+        x = np.where((i // m) % 2, m - 1 - x, x)
+        xyz.append((np.stack([x, y, z], 1) - m // 2 + 0.5) * 1.25)
+        flags.append((i % 3 == 0).astype(np.uint8))
+    b.set_state(np.concatenate(xyz).astype(np.float32), np.concatenate(flags))
+    with pytest.raises(tfm_amd.CcpError):
+        b.run_steps(400)
+        b.synchronize()
+    b.close()

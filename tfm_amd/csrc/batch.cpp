@@ -180,7 +180,8 @@ struct ccp_batch {
         for (uint32_t i = sys[s].slot; i < sys[s].slot + sys[s].n; ++i) het += (hfl[i] & CCP_HET) ? 1u : 0u;
         ++s;
       } while (s < sys.size() && (sys[s].g.coff + sys[s].g.bbias) % cells != 0);
-      for (int c = S.g.coff; c < end; c += cells) ob.push_back({c, std::min(cells, end - c), blk0, S.slot, het0});
+      for (int c = S.g.coff; c < end; c += cells)
+        ob.push_back({c, std::min(cells, end - c), blk0, S.slot, slot[s], het0});
     }
     return ob;
   }

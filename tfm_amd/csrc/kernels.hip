@@ -1477,6 +1477,10 @@ __global__ __launch_bounds__(BEAD_BLOCK) void k_bin_batch(const SysParams *sys, 
 // took 46.6 us a launch, 30 us with the table, 27.4 us with two cells per lane
 // (cells below 1.5 sigma, about one bead each: half as many workgroups, each
 // waiting out the same chain of loads) and the early end of empty blocks.
+// After an overflowing cell (reported, but steps already queued go on) the
+// work list can name a run's beads more often than it has them, so starts and
+// slots stop at the run's end: nothing is written past it, and no start lies
+// beyond the arrays.
 constexpr int ORDER_LDS = 1024;
 
 //
@@ -1506,7 +1510,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_order(OrderJobs<TWO ? 2 : 1> job
   const OrderJob &J = jobs.j[second ? 1 : 0];
   const int b = second ? bx - jobs.j[0].g.nblk : bx;
   const int tid = threadIdx.x, lane = __lane_id(), wid = tid >> 6;
-  OrderBlock ob{b * CELLS, CELLS, 0u, 0u, 0u};
+  OrderBlock ob{b * CELLS, CELLS, 0u, 0u, 0u, 0u};
   if constexpr (BATCH) ob = blocks[b];
   const int cap = J.g.cap, n_c = J.g.n_c;
   // this lane's cells c0 .. c0 + CPT - 1, those below c_end
@@ -1579,6 +1583,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_order(OrderJobs<TWO ? 2 : 1> job
       uint32_t prefix = ob.slot0;
 #pragma unroll
       for (int k = 0; k < SCAN_BLOCK / 64; ++k) prefix += red[k];
+      prefix = min(prefix, ob.slot1);
 #pragma unroll
       for (int u = 0; u < CPT; ++u) {
         if (c0 + u < c_end) {
@@ -1664,12 +1669,14 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_order(OrderJobs<TWO ? 2 : 1> job
 #pragma unroll
   for (int u = 0; u < CPT; ++u) {
     if (c0 + u < c_end) {
-      J.cstart[c0 + u] = start[u];
+      J.cstart[c0 + u] = BATCH ? min(start[u], ob.slot1) : start[u];
       J.count[c0 + u] = 0u;
       // (the lanes past a short block's cells hold numbers of the next run's)
-      if (c0 + u == n_c - 1) J.cstart[n_c] = start[u] + cnt[u];
+      const uint32_t end = start[u] + cnt[u];
+      if (c0 + u == n_c - 1) J.cstart[n_c] = BATCH ? min(end, ob.slot1) : end;
     }
   }
+  auto past_end = [&](uint32_t dst) { return BATCH && dst >= ob.slot1; };
   // work-list entry of the member at slot dst, with hbefore het members in
   // the slots before it: het members in slot order, then the others
   auto put_work = [&](uint32_t dst, uint32_t hbefore, bool het) {
@@ -1709,6 +1716,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_order(OrderJobs<TWO ? 2 : 1> job
         for (uint32_t s2 = b0; s2 < b1; ++s2) rank += (s_id[s2] < id) ? 1u : 0u;
       }
       const uint32_t dst = s_start[l] + rank;
+      if (past_end(dst)) continue;
       const float4 v = s_pos[e];
       J.spos[dst] = v;
       if (J.soi) J.soi[dst] = id;
@@ -1727,6 +1735,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_order(OrderJobs<TWO ? 2 : 1> job
           rank += before ? 1u : 0u;
           hr += (before && (wbits(o) & W_HET)) ? 1u : 0u;
         }
+        if (past_end(start[u] + rank)) continue;
         J.spos[start[u] + rank] = v;
         if (J.soi) J.soi[start[u] + rank] = e;
         if (typed) put_work(start[u] + rank, hoff[u] + hr, (wbits(v) & W_HET) != 0u);
@@ -1739,6 +1748,7 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_order(OrderJobs<TWO ? 2 : 1> job
 #pragma unroll
   for (int u = 0; u < CPT; ++u)
     for (uint32_t k = m[u]; k < cnt[u]; ++k) {
+      if (past_end(start[u] + k)) break;
       J.spos[start[u] + k] = make_float4(1e18f, 1e18f, 1e18f, __uint_as_float(ID_MASK));
       if (J.soi) J.soi[start[u] + k] = ID_MASK;
       if (typed) put_work(start[u] + k, hoff[u] + hc[u], false);

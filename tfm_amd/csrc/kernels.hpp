@@ -140,11 +140,11 @@ struct KPtrs {
 };
 
 // One scan block of a batch: its cells [cell0, cell0 + n_cells), all of one run
-// of systems, that run's first block, and the slots and het members of the
-// systems before the run.
+// of systems, that run's first block and its slots [slot0, slot1), and the het
+// members of the systems before the run.
 struct OrderBlock {
   int cell0, n_cells;
-  uint32_t blk0, slot0, het0;
+  uint32_t blk0, slot0, slot1, het0;
 };
 
 // The scan blocks of a batch's ordering (nblk of them, each of SCAN_BLOCK
