@@ -346,6 +346,25 @@ def test_batch_short_block_before_a_small_last_system(shape, size, phi):
     b.close()
 
 
+@pytest.mark.parametrize("shape", [dict(lanes_per_bead=8, cell_reach=2, cell_size=1.25), {}])
+def test_batch_relaxation_with_overflowing_cells(shape):
+    # three runs of systems whose fullest cells of 1.25 sigma gain beads during
+    # the relaxation, past the cells' storage: the steps that follow within the
+    # round stay inside the runs' slots, and the round is redone
+    step(f"batch with overflowing cells {shape}")
+    systems = [dict(n_beads=n, volume_fraction=v, eps_het=0.6, eps_lam=1.0, het_fraction=0.3, lad_fraction=0.1, seed=s)
+               for n, v, s in [(12, 0.2, 9145), (24, 0.3, 9127), (12, 0.2, 9106), (40, 0.005, 9101), (16, 0.2, 9141),
+                               (24, 0.3, 9109), (12, 0.2, 9135), (40, 0.005, 9105), (40, 0.3, 9134),
+                               (12, 0.2, 9150)]]
+    got = []
+    for capacity in (3, 32):
+        b = tfm_amd.Batch(systems, dict(timestep=0.001, cell_capacity=capacity, **shape))
+        b.generate_initial_conditions()
+        got.append(b.state())
+        b.close()
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+
+
 @pytest.mark.parametrize("shape", [dict(lanes_per_bead=8, cell_reach=2, cell_size=1.25),
                                    dict(lanes_per_bead=5, cell_reach=2, cell_size=1.25)])
 def test_batch_steps_past_an_overflowing_cell(shape):

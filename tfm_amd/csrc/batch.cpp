@@ -412,6 +412,10 @@ struct ccp_batch {
         noise_step = step;
         if (!take_overflow()) break;
         hip_check(hipMemcpyAsync(r.p, rsave.p, (size_t)N * sizeof(float4), hipMemcpyDeviceToDevice, stream));
+        // (with the members an overflow leaves out, the slots of a run's later
+        // systems move down, into the grids of those before: no bead of theirs
+        // left the grid)
+        hip_check(hipMemsetAsync(flags.p, 0, FLAG_COUNT * sizeof(uint32_t), stream));
         step -= spf;
         dstep_dirty = true;
         grow();
