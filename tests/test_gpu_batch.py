@@ -382,10 +382,11 @@ def test_batch_steps_past_an_overflowing_cell(shape):
         z, y, x = i // (m * m), i // m % m, i % m
         y = np.where(z % 2, m - 1 - y, y)  # (a snake: neighbours along the chain are neighbours in space)
         x = np.where((i // m) % 2, m - 1 - x, x)
-        xyz.append((np.stack([x, y, z], 1) - m // 2 + 0.5) * 1.25)
+        far = 5 if n >= 40 else 0  # (the larger systems' chains lie outside the smaller ones' grids)
+        xyz.append((np.stack([x + far, y, z], 1) - m // 2 + 0.5) * 1.25)
         flags.append((i % 3 == 0).astype(np.uint8))
     b.set_state(np.concatenate(xyz).astype(np.float32), np.concatenate(flags))
-    with pytest.raises(tfm_amd.CcpError):
+    with pytest.raises(tfm_amd.CcpError, match="cell_capacity"):
         b.run_steps(400)
         b.synchronize()
     b.close()

@@ -202,8 +202,13 @@ struct ccp_batch {
     if (f[FLAG_NONFINITE] || f[FLAG_OUTSIDE] || f[FLAG_OVERFLOW]) {
       hip_check(hipMemset(flags.p, 0, sizeof(f)));
       if (f[FLAG_NONFINITE]) throw Error(CCP_ERR_STATE, "non-finite bead position");
-      if (f[FLAG_OUTSIDE]) throw Error(CCP_ERR_STATE, "bead left the cell grid");
-      throw Error(CCP_ERR_STATE, "cell_capacity exceeded; raise cell_capacity");
+      // (a full cell shifts the later systems' beads of its run into the grids
+      // of those before, where they count as outside)
+      if (f[FLAG_OVERFLOW])
+        throw Error(CCP_ERR_STATE, f[FLAG_OUTSIDE]
+                                       ? "cell_capacity exceeded; raise cell_capacity (or a bead left the cell grid)"
+                                       : "cell_capacity exceeded; raise cell_capacity");
+      throw Error(CCP_ERR_STATE, "bead left the cell grid");
     }
   }
   bool take_overflow() {
