@@ -1480,7 +1480,7 @@ __global__ __launch_bounds__(BEAD_BLOCK) void k_bin_batch(const SysParams *sys, 
 // After an overflowing cell (reported, but steps already queued go on) the
 // work list can name a run's beads more often than it has them, so starts and
 // slots stop at the run's end: nothing is written past it, and no start lies
-// beyond the arrays.
+// beyond the arrays (0.3 us of those 27).
 constexpr int ORDER_LDS = 1024;
 
 //
